@@ -178,6 +178,25 @@ struct CoarseMat {
   }
 };
 
+// ------------------------------------------------------ level schedules
+// One step of the workgroup that walks a run of narrow levels (ms_levels.hip):
+// rows [t0, t0 + n) of the level order, entry k of its lane t at
+// base + k * roundup(n, 64) + t, w entries at most; near: all
+// neighbours of its rows are in the workgroup's ring (1), or not (0)
+struct SweepStep {
+  int t0, n, w, near;
+  long long base;
+};
+struct SweepPlan {
+  int nsteps = 0;
+  int width = 0;       // entries per row of every step (more: rows beyond the width fetched ahead exist)
+  bool more = false;
+  long long nent = 0;
+  DBuf<SweepStep> steps;
+  DBuf<int> col;   // neighbour positions, -1 padding
+  size_t bytes() const { return steps.bytes() + col.bytes(); }
+};
+
 // ------------------------------------------------- SELL-64 sparse pattern
 // Row r lives in slice s = r/64, lane l = r%64; its k-th entry (columns in
 // ascending order, as csr_t) sits at off[s] + k*64 + l.  Padding entries use
@@ -203,13 +222,18 @@ struct SellPattern {
   std::vector<int> lev_ptr_f, lev_ptr_b;   // rows grouped per level
   DBuf<int> d_lev_rows_f, d_lev_rows_b, d_lev_ptr_f, d_lev_ptr_b;
   // launch plan of a sweep: runs of consecutive narrow levels (at most
-  // kNarrowRows rows each) go to one workgroup that steps through them with
-  // a barrier between levels; every wider level is a launch of its own
+  // kNarrowRows rows each) go to one workgroup that steps through them
+  // (steps [s0, s1), positions from t0 on, `block` threads); every wider
+  // level is a launch of its own
   struct LevSeg {
     int l0, l1;
     bool narrow;
+    int s0 = 0, s1 = 0, t0 = 0, block = kSegThreads;
   };
   std::vector<LevSeg> seg_f, seg_b;
+  SweepPlan sweep_f, sweep_b;
+  bool sweep_ordered = false;   // one run each way, vectors in level order (d_lev_fb: forward position of a backward one)
+  DBuf<int> d_lev_fb;
   // colour classes: rows of colour c are [col_ptr[c], col_ptr[c+1])
   std::vector<int> color_ptr;
   bool has_levels = false;

@@ -1,0 +1,567 @@
+// ms_levels.hip -- level-scheduled natural-order factorizations and
+// triangular sweeps (ILU(0) / IC(0), mod_uns_linsolver.f90:79-142, :328-399).
+//
+// A level holds the rows whose lower (forward) or upper (backward)
+// neighbours all lie in earlier levels.  Levels wider than kNarrowRows take
+// one launch each, a thread per row.  A run of narrower levels takes one
+// workgroup that steps through it: on lexicographic meshes such a run is the
+// whole sweep, a serial chain of hundreds of levels of a few hundred rows,
+// so its time is the latency of one level times their number.
+#include <type_traits>
+
+#include "ms_linalg.hpp"
+#include "ms_reduce.hpp"
+
+namespace ms {
+namespace {
+
+constexpr double kTiny = 2.2250738585072014e-308;   // tiny(1.0_dp)
+
+struct LMat {
+  const long long *off;
+  const int *rowlen, *col, *diagk;
+};
+LMat lmat(const SellPattern &p) { return LMat{p.d_off.p, p.d_rowlen.p, p.d_col.p, p.d_diagk.p}; }
+
+// natural IC(0) of row i, its lower neighbours final (mod_uns_linsolver.f90:328-365)
+template <class T>
+__device__ void ic0_factor_row(int i, const LMat &A, T *F, int *flag) {
+  const long long bi = A.off[i >> 6] + (i & 63);
+  const int dpi = A.diagk[i];
+  for (int kp = 0; kp < dpi; kp++) {
+    const long long qkp = bi + (long long)kp * kSlice;
+    const int k = A.col[qkp];
+    const long long bk = A.off[k >> 6] + (k & 63);
+    const int dpk = A.diagk[k];
+    int p = 0, q = 0;
+    T dsum = T(0);
+    while (p <= kp - 1 && q <= dpk - 1) {
+      const int cp = A.col[bi + (long long)p * kSlice], cq = A.col[bk + (long long)q * kSlice];
+      if (cp < cq) p++;
+      else if (cp > cq) q++;
+      else {
+        dsum = dsum + F[bi + (long long)p * kSlice] * F[bk + (long long)q * kSlice];
+        p++;
+        q++;
+      }
+    }
+    const T s = F[qkp] - dsum;
+    F[qkp] = s / F[bk + (long long)dpk * kSlice];
+  }
+  const long long qd = bi + (long long)dpi * kSlice;
+  T s = F[qd];
+  for (int kp = 0; kp < dpi; kp++) {
+    const T v = F[bi + (long long)kp * kSlice];
+    s = s - v * v;
+  }
+  if (s <= T(0)) {
+    *flag = 2;
+    return;
+  }
+  F[qd] = tsqrt(s);
+}
+
+// natural ILU(0) of row i, IKJ variant (mod_uns_linsolver.f90:79-115)
+template <class T>
+__device__ void ilu0_factor_row(int i, const LMat &A, T *F, int *flag) {
+  const long long bi = A.off[i >> 6] + (i & 63);
+  const int dpi = A.diagk[i], leni = A.rowlen[i];
+  for (int kk = 0; kk < dpi; kk++) {
+    const long long q = bi + (long long)kk * kSlice;
+    const int k = A.col[q];
+    const long long bk = A.off[k >> 6] + (k & 63);
+    const int dpk = A.diagk[k], lenk = A.rowlen[k];
+    const T piv = F[bk + (long long)dpk * kSlice];
+    if (tabs(piv) < (T)kTiny) {
+      *flag = 2;
+      return;
+    }
+    const T aik = F[q] / piv;
+    F[q] = aik;
+    for (int jj = dpk; jj < lenk; jj++) {
+      const int j = A.col[bk + (long long)jj * kSlice];
+      if (j <= k) continue;
+      for (int m = 0; m < leni; m++) {
+        const long long qm = bi + (long long)m * kSlice;
+        const int cm = A.col[qm];
+        if (cm == j) {
+          F[qm] = F[qm] - aik * F[bk + (long long)jj * kSlice];
+          break;
+        }
+        if (cm > j) break;
+      }
+    }
+  }
+}
+
+// forward substitution of row i (unit lower for ILU(0), L of IC(0))
+template <class T>
+__device__ void lower_row(int i, const LMat &A, const T *F, const T *r, T *z, int ic0) {
+  const long long bi = A.off[i >> 6] + (i & 63);
+  const int dpi = A.diagk[i];
+  T s = r[i];
+  for (int k = 0; k < dpi; k++) {
+    const long long q = bi + (long long)k * kSlice;
+    s = s - F[q] * z[A.col[q]];
+  }
+  z[i] = ic0 ? s / F[bi + (long long)dpi * kSlice] : s;
+}
+
+// backward substitution of row i (U of ILU(0), L^T of IC(0) via tpos)
+template <class T>
+__device__ void upper_row(int i, const LMat &A, const long long *tpos, const T *F, T *z, int ic0) {
+  const long long bi = A.off[i >> 6] + (i & 63);
+  const int dpi = A.diagk[i], len = A.rowlen[i];
+  T s = z[i];
+  if (ic0) {
+    for (int k = len - 1; k > dpi; k--) {
+      const long long q = bi + (long long)k * kSlice;
+      s = s - F[tpos[q]] * z[A.col[q]];
+    }
+  } else {
+    for (int k = dpi + 1; k < len; k++) {
+      const long long q = bi + (long long)k * kSlice;
+      s = s - F[q] * z[A.col[q]];
+    }
+  }
+  z[i] = s / F[bi + (long long)dpi * kSlice];
+}
+
+// one wide level: a thread per row
+template <class T>
+__global__ void k_factor_level(const int *rows, int nr, LMat A, T *F, int ic0, int *flag) {
+  int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t >= nr) return;
+  if (ic0) ic0_factor_row(rows[t], A, F, flag);
+  else ilu0_factor_row(rows[t], A, F, flag);
+}
+
+template <class T>
+__global__ void k_lower_level(const int *rows, int nr, LMat A, const T *F, const T *r, T *z, int ic0, const int *done) {
+  if (*done) return;
+  int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < nr) lower_row(rows[t], A, F, r, z, ic0);
+}
+
+template <class T>
+__global__ void k_upper_level(const int *rows, int nr, LMat A, const long long *tpos, const T *F, T *z, int ic0,
+                              const int *done) {
+  if (*done) return;
+  int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < nr) upper_row(rows[t], A, tpos, F, z, ic0);
+}
+
+// a run of narrow levels [l0, l1) in one workgroup: rows of a level are
+// spread over the threads, a barrier orders the levels (the workgroup shares
+// one L1, so rows of the next level see the values just stored).  Every
+// thread reaches every barrier: the level loop is uniform, only the row loop
+// inside a level depends on the thread.
+template <class T>
+__global__ __launch_bounds__(kSegThreads) void k_factor_seg(const int *lev_ptr, int l0, int l1, const int *rows,
+                                                             LMat A, T *F, int ic0, int *flag) {
+  for (int l = l0; l < l1; l++) {
+    const int a = lev_ptr[l], b = lev_ptr[l + 1];
+    for (int t = a + (int)threadIdx.x; t < b; t += kSegThreads) {
+      if (ic0) ic0_factor_row(rows[t], A, F, flag);
+      else ilu0_factor_row(rows[t], A, F, flag);
+    }
+    __syncthreads();
+  }
+}
+
+// ------------------------------------------------------------ packed sweeps
+// One workgroup steps through a run of narrow levels.  A step is a level, or
+// a part of at most kSegThreads rows of a wider one; a row's place in the
+// level order is its position.
+//
+// What bounds it is the latency of one step times the number of steps, so
+// everything that does not depend on the step before is taken off that
+// chain: the factor's off-diagonal entries of each row are packed in step
+// order (pcol: the neighbour's position, pval: the value; entry k of lane t
+// at base + k * stride + t), so they load coalesced and without the SELL
+// offsets, and they, the row ids and the right-hand side are fetched three
+// steps ahead into registers.  The solution of the last kRing positions
+// stays in LDS, so a step costs an LDS read per entry, the row's arithmetic,
+// an LDS write and one barrier that waits for LDS only (the loads in flight
+// and the stores to `out` go on across it).  A step that reads a position
+// older than the ring takes it from `out` behind a full barrier, which
+// orders this workgroup's stores.
+// One FP64 sweep of a 40^3 hex grid (118 levels of up to 1200 rows) went
+// from 541 us (lower) and 698 us (upper) to 84 us each, and of a 128^2
+// cavity (255 levels of up to 128 rows) from 170 and 189 us to 62 and 64 us:
+// 0.25 us a level where the level is its latency, about 45 GB/s where it is
+// wide, which is what one compute unit draws.
+constexpr int kRing = 16384;   // positions kept in LDS (128 KB in FP64)
+constexpr int kPre = 4;        // most entries per row that are fetched ahead (hexahedra 3, prisms 2-3)
+constexpr int kOrderedBlock = 512;   // widest level (in whole wavefronts) from which vectors go in level order
+constexpr int kAheadRows = 3, kAheadOrdered = 4;   // steps fetched ahead (vectors in row order / level order)
+
+constexpr int kTailSteps = 6;  // empty steps after the last, so that fetching ahead needs no bound
+
+// LDS only: a release of the ring's writes, no wait for loads or stores in flight
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <class T, int W>
+struct Ahead {
+  T rhs, dg, v[W];
+  int c[W];
+};
+
+// W: entries per row fetched ahead; MORE: rows may have more than W
+// ORDERED: in and out are in level order (rows is not read), else in row order
+// DIV: divide by the factor's diagonal (U of ILU(0), L and L^T of IC(0))
+// DESC: the entries in descending column order (L^T of IC(0)), as the
+// reference's loops run
+template <class T, int W, bool MORE, bool ORDERED, bool DIV, bool DESC>
+__global__ __launch_bounds__(kSegThreads) void k_sweep_seg(const SweepStep *__restrict__ steps, int nsteps, int seg0,
+                                                           const int *__restrict__ rows,
+                                                           const int *__restrict__ pcol,
+                                                           const T *__restrict__ pval, const T *__restrict__ pdiag,
+                                                           const T *in, T *out, const int *done) {
+  if (*done) return;
+  __shared__ T ring[kRing + 1];
+  const int t = threadIdx.x;
+  if (t == 0) ring[kRing] = T(0);
+  __syncthreads();
+  // constant address space: the steps come through scalar loads, which do
+  // not queue behind the fetches
+  typedef const __attribute__((address_space(4))) SweepStep *StepPtr;
+  const StepPtr sp = (StepPtr)(unsigned long long)steps;
+  auto desc = [&](int s) { return SweepStep{sp[s].t0, sp[s].n, sp[s].w, sp[s].near, sp[s].base}; };
+  // the loads of lanes beyond a step's rows go to its last row: no branch
+  // around them, so nothing waits for them before their step
+  auto lane = [&](const SweepStep &d) { return (unsigned)min(t, max(d.n, 1) - 1); };
+  // uniform pointers plus a 32-bit lane index: one vector instruction per
+  // load, which matters as much as the latency does (16 wavefronts share
+  // four SIMDs)
+  auto fetch = [&](Ahead<T, W> &a, const SweepStep &d, int row) {
+    const unsigned l = lane(d);
+    const int stride = (d.n + 63) & ~63;
+    const int *pc = pcol + d.base;
+    const T *pv = pval + d.base;
+    if (ORDERED) a.rhs = (in + d.t0)[l];
+    else a.rhs = in[row];
+    if (DIV) a.dg = (pdiag + d.t0)[l];
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+      a.c[k] = pc[l];
+      a.v[k] = pv[l];
+      pc += stride;
+      pv += stride;
+    }
+  };
+  // U steps per turn of the loop, so that every register set has a fixed
+  // name; in row order the row ids come two steps before what they address
+  constexpr int NS = ORDERED ? kAheadOrdered : kAheadRows, U = ORDERED ? NS : 2 * NS, DN = ORDERED ? NS : NS + 2;
+  SweepStep d[U];
+  int row[U];
+  Ahead<T, W> a[NS];
+#pragma unroll
+  for (int j = 0; j < DN; j++) d[j] = desc(j);
+#pragma unroll
+  for (int j = 0; j < DN; j++) row[j] = ORDERED ? 0 : (rows + d[j].t0)[lane(d[j])];
+#pragma unroll
+  for (int j = 0; j < NS; j++) fetch(a[j], d[j], row[j]);
+  auto step = [&](auto jc, int s) {
+    constexpr int j = decltype(jc)::value;
+    Ahead<T, W> &p = a[j % NS];
+    const SweepStep e = d[j], next = desc(s + DN);
+    const int r = row[j];
+    // A step whose neighbours are all in the ring has their ring slots in
+    // pcol (the zero slot kRing for padding).  Any other step has positions
+    // (-1: padding): those in [lo, e.t0) are in the ring, older ones in `out`
+    // behind a barrier that orders this workgroup's stores, those before seg0
+    // from earlier launches.
+    const bool near = e.near != 0;
+    const int lo = max(seg0, e.t0 + e.n - kRing);
+    if (!near && lo > seg0) __syncthreads();
+    auto solve = [&](auto get) {
+      T sum = p.rhs;
+      const int stride = (e.n + 63) & ~63;
+      if (MORE && DESC)
+        for (int k = e.w - 1; k >= W; k--) {
+          const long long q = e.base + (long long)k * stride + t;
+          sum = sum - pval[q] * get(pcol[q]);
+        }
+      T z[W];
+#pragma unroll
+      for (int k = 0; k < W; k++) z[k] = get(p.c[k]);
+#pragma unroll
+      for (int i = 0; i < W; i++) {
+        const int k = DESC ? W - 1 - i : i;
+        sum = sum - p.v[k] * z[k];   // padding: 0 * 0, which leaves the sum as it is
+      }
+      if (MORE && !DESC)
+        for (int k = W; k < e.w; k++) {
+          const long long q = e.base + (long long)k * stride + t;
+          sum = sum - pval[q] * get(pcol[q]);
+        }
+      if (DIV) sum = sum / p.dg;
+      ring[(e.t0 + t) & (kRing - 1)] = sum;
+      if (ORDERED) (out + e.t0)[(unsigned)t] = sum;
+      else out[r] = sum;
+    };
+    // two bodies: one select between an LDS and a memory address would make
+    // every read a flat load, which waits for the fetches in flight
+    if (near) {
+      if (t < e.n) solve([&](int c) { return ring[c]; });
+    } else if (t < e.n) {
+      solve([&](int c) {
+        T v = c >= lo ? ring[c & (kRing - 1)] : (c < 0 ? T(0) : out[ORDERED ? c : rows[c]]);
+        asm volatile("" : "+v"(v));   // waited for here, not where the two bodies' common code begins
+        return v;
+      });
+    }
+    lds_barrier();
+    d[(j + DN) % U] = next;
+    fetch(p, d[(j + NS) % U], row[(j + NS) % U]);
+    if (!ORDERED) row[(j + DN) % U] = (rows + next.t0)[lane(next)];
+  };
+  auto turn = [&](auto self, auto jc, int s) {
+    constexpr int j = decltype(jc)::value;
+    if constexpr (j < U) {
+      if (s + j < nsteps) {
+        step(jc, s + j);
+        self(self, std::integral_constant<int, j + 1>{}, s);
+      }
+    }
+  };
+  for (int s = 0; s < nsteps; s += U) turn(turn, std::integral_constant<int, 0>{}, s);
+}
+
+// pcol of every step's rows (one workgroup per step of a run whose first
+// position is seg0): ring slots where all neighbours will be in the ring,
+// else positions; upper: the entries above the diagonal
+__global__ void k_pack_cols(SweepStep *steps, int seg0, const int *rows, const int *pos, LMat A, int upper,
+                            int *pcol) {
+  const SweepStep d = steps[blockIdx.x];
+  const int stride = (d.n + 63) & ~63;
+  __shared__ int far;
+  if (threadIdx.x == 0) far = 0;
+  __syncthreads();
+  for (int pass = 0; pass < 2; pass++) {
+    const bool near = pass == 1 && !far;
+    for (int t = threadIdx.x; t < d.n; t += kBlock) {
+      const int r = rows[d.t0 + t], dk = A.diagk[r];
+      const long long br = A.off[r >> 6] + (r & 63);
+      const int k0 = upper ? dk + 1 : 0, m = upper ? A.rowlen[r] - dk - 1 : dk;
+      for (int k = 0; k < d.w; k++) {
+        const int c = k < m ? pos[A.col[br + (long long)(k0 + k) * kSlice]] : -1;
+        if (pass == 0) {
+          if (k < m && c < max(seg0, d.t0 + d.n - kRing)) far = 1;
+        } else {
+          pcol[d.base + (long long)k * stride + t] = !near ? c : (c < 0 ? kRing : c & (kRing - 1));
+        }
+      }
+    }
+    __syncthreads();
+    if (near && threadIdx.x == 0) steps[blockIdx.x].near = 1;
+  }
+}
+
+// the factor's entries and diagonal in step order (tpos: L^T of IC(0))
+template <class T>
+__global__ void k_pack_vals(const SweepStep *steps, const int *rows, LMat A, int upper, const long long *tpos,
+                            const T *F, T *pval, T *pdiag) {
+  const SweepStep d = steps[blockIdx.x];
+  const int stride = (d.n + 63) & ~63;
+  for (int t = threadIdx.x; t < d.n; t += kBlock) {
+    const int r = rows[d.t0 + t], dk = A.diagk[r];
+    const long long br = A.off[r >> 6] + (r & 63);
+    const int k0 = upper ? dk + 1 : 0, m = upper ? A.rowlen[r] - dk - 1 : dk;
+    for (int k = 0; k < m; k++) {
+      const long long q = br + (long long)(k0 + k) * kSlice;
+      pval[d.base + (long long)k * stride + t] = F[tpos ? tpos[q] : q];
+    }
+    for (int k = m; k < d.w; k++) pval[d.base + (long long)k * stride + t] = T(0);
+    pdiag[d.t0 + t] = F[br + (long long)dk * kSlice];
+  }
+}
+
+template <class T>
+__global__ void k_gather(int n, const int *idx, const T *in, T *out, const int *done) {
+  if (*done) return;
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < n) out[t] = in[idx[t]];
+}
+template <class T>
+__global__ void k_scatter(int n, const int *idx, const T *in, T *out, const int *done) {
+  if (*done) return;
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < n) out[idx[t]] = in[t];
+}
+
+}  // namespace
+
+// The steps of every run of narrow levels, and their packed columns.
+void plan_sweeps(SellPattern &P, const std::vector<int> &rows_f, const std::vector<int> &rows_b) {
+  std::vector<int> pos_f(P.n);
+  for (int t = 0; t < P.n; t++) pos_f[rows_f[t]] = t;
+  auto plan = [&](bool upper, const std::vector<int> &lev, const std::vector<int> &rows,
+                  std::vector<SellPattern::LevSeg> &segs, SweepPlan &S, const DBuf<int> &d_rows) {
+    std::vector<SweepStep> st;
+    long long base = 0;
+    int widest_row = 1;
+    for (auto &g : segs)
+      if (g.narrow)
+        for (int t = lev[g.l0]; t < lev[g.l1]; t++) {
+          const int r = rows[t];
+          widest_row = std::max(widest_row, upper ? P.rowlen[r] - P.diagk[r] - 1 : P.diagk[r]);
+        }
+    S.width = std::min(widest_row, kPre);
+    S.more = widest_row > kPre;
+    for (auto &g : segs) {
+      if (!g.narrow) continue;
+      g.s0 = (int)st.size();
+      g.t0 = lev[g.l0];
+      int widest = 1;
+      for (int l = g.l0; l < g.l1; l++) widest = std::max(widest, lev[l + 1] - lev[l]);
+      g.block = std::min(kSegThreads, (widest + kSlice - 1) / kSlice * kSlice);
+      for (int l = g.l0; l < g.l1; l++)
+        for (int t = lev[l]; t < lev[l + 1]; t += g.block) {
+          SweepStep d{t, std::min(g.block, lev[l + 1] - t), S.width, 0, base};
+          for (int i = 0; S.more && i < d.n; i++) {
+            const int r = rows[t + i];
+            d.w = std::max(d.w, upper ? P.rowlen[r] - P.diagk[r] - 1 : P.diagk[r]);
+          }
+          base += (long long)d.w * ((d.n + 63) & ~63);
+          st.push_back(d);
+        }
+      g.s1 = (int)st.size();
+      for (int i = 0; i < kTailSteps; i++) st.push_back(SweepStep{0, 0, 0, 0, 0});
+    }
+    S.nent = base;
+    S.nsteps = (int)st.size();
+    if (!S.nsteps) return;
+    std::vector<int> pos(P.n);
+    for (int t = 0; t < P.n; t++) pos[rows[t]] = t;
+    DBuf<int> d_pos;
+    d_pos.upload(pos);
+    S.steps.upload(st);
+    S.col.alloc(std::max<long long>(base, 1));
+    for (const auto &g : segs)
+      if (g.narrow)
+        hipLaunchKernelGGL(k_pack_cols, dim3(g.s1 - g.s0), dim3(kBlock), 0, stream(), S.steps.p + g.s0, g.t0,
+                           d_rows.p, d_pos.p, lmat(P), (int)upper, S.col.p);
+    MS_CHECK_LAUNCH();
+    MS_HIP(hipStreamSynchronize(stream()));   // the host arrays above and d_pos go out of scope
+  };
+  plan(false, P.lev_ptr_f, rows_f, P.seg_f, P.sweep_f, P.d_lev_rows_f);
+  plan(true, P.lev_ptr_b, rows_b, P.seg_b, P.sweep_b, P.d_lev_rows_b);
+  // Vectors in level order: the rows of a level are far apart in row order
+  // (a diagonal plane of a grid), so reading and writing them there costs
+  // the one workgroup a cache line per row, 150 us per sweep against 84
+  // on a 40^3 grid; three launches of 4 us that permute for the whole chip cost
+  // less once levels are this wide.  On a 128^2 grid (levels of at most 128
+  // rows) a step is its latency either way and the launches would be lost.
+  P.sweep_ordered = P.seg_f.size() == 1 && P.seg_b.size() == 1 && P.seg_f[0].narrow && P.seg_b[0].narrow &&
+                    P.seg_f[0].block >= kOrderedBlock;
+  if (P.sweep_ordered) {
+    std::vector<int> fb(P.n);
+    for (int t = 0; t < P.n; t++) fb[t] = pos_f[rows_b[t]];
+    P.d_lev_fb.upload(fb);
+    MS_HIP(hipStreamSynchronize(stream()));
+  }
+}
+
+// the factor F (SELL layout) in the order of the packed sweeps
+template <class T>
+void LevelFactor<T>::pack(const SellPattern &P, const T *F, bool ic0) {
+  auto one = [&](const SweepPlan &S, const DBuf<int> &rows, DBuf<T> &v, DBuf<T> &d, bool upper) {
+    if (!S.nsteps) return;
+    if (v.n < (size_t)S.nent) v.alloc(S.nent);
+    if (d.n < (size_t)P.n) d.alloc(P.n);
+    hipLaunchKernelGGL(k_pack_vals<T>, dim3(S.nsteps), dim3(kBlock), 0, stream(), S.steps.p, rows.p, lmat(P),
+                       (int)upper, ic0 && upper ? P.d_tpos.p : nullptr, F, v.p, d.p);
+  };
+  one(P.sweep_f, P.d_lev_rows_f, vf, df, false);
+  one(P.sweep_b, P.d_lev_rows_b, vb, db, true);
+  MS_CHECK_LAUNCH();
+}
+
+template <class T, bool DIV, bool DESC>
+static void sweep_run(const SweepPlan &S, const SellPattern::LevSeg &g, const int *rows, const T *v, const T *d,
+                      const T *in, T *out, const int *done) {
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3(1), dim3(g.block), 0, stream(), S.steps.p + g.s0, g.s1 - g.s0, g.t0, rows, S.col.p, v,
+                       d, in, out, done);
+  };
+  auto by_width = [&](auto ordered) {
+    constexpr bool O = decltype(ordered)::value;
+    if (S.more) go(k_sweep_seg<T, kPre, true, O, DIV, DESC>);
+    else if (S.width == 4) go(k_sweep_seg<T, 4, false, O, DIV, DESC>);
+    else if (S.width == 3) go(k_sweep_seg<T, 3, false, O, DIV, DESC>);
+    else if (S.width == 2) go(k_sweep_seg<T, 2, false, O, DIV, DESC>);
+    else go(k_sweep_seg<T, 1, false, O, DIV, DESC>);
+  };
+  if (rows) by_width(std::false_type{});
+  else by_width(std::true_type{});
+}
+
+// out = (L U)^-1 in or (L L^T)^-1 in
+template <class T>
+void LevelFactor<T>::apply(const SellPattern &P, const T *F, bool ic0, const T *in, T *out, const int *done) {
+  hipStream_t S = stream();
+  const LMat A = lmat(P);
+  const dim3 G(nblocks(P.n)), B(kBlock);
+  auto fwd = [&](const SellPattern::LevSeg &g, const int *rows, const T *x, T *y) {
+    if (ic0) sweep_run<T, true, false>(P.sweep_f, g, rows, vf.p, df.p, x, y, done);
+    else sweep_run<T, false, false>(P.sweep_f, g, rows, vf.p, df.p, x, y, done);
+  };
+  auto bwd = [&](const SellPattern::LevSeg &g, const int *rows, const T *x, T *y) {
+    if (ic0) sweep_run<T, true, true>(P.sweep_b, g, rows, vb.p, db.p, x, y, done);
+    else sweep_run<T, true, false>(P.sweep_b, g, rows, vb.p, db.p, x, y, done);
+  };
+  if (P.sweep_ordered) {
+    if (xf.n < (size_t)P.n) xf.alloc(P.n);
+    if (xb.n < (size_t)P.n) xb.alloc(P.n);
+    hipLaunchKernelGGL(k_gather<T>, G, B, 0, S, P.n, P.d_lev_rows_f.p, in, xf.p, done);
+    fwd(P.seg_f[0], nullptr, xf.p, xf.p);
+    hipLaunchKernelGGL(k_gather<T>, G, B, 0, S, P.n, P.d_lev_fb.p, xf.p, xb.p, done);
+    bwd(P.seg_b[0], nullptr, xb.p, xb.p);
+    hipLaunchKernelGGL(k_scatter<T>, G, B, 0, S, P.n, P.d_lev_rows_b.p, xb.p, out, done);
+    MS_CHECK_LAUNCH();
+    return;
+  }
+  for (const auto &g : P.seg_f) {
+    if (g.narrow) {
+      fwd(g, P.d_lev_rows_f.p, in, out);
+      continue;
+    }
+    const int a = P.lev_ptr_f[g.l0], b = P.lev_ptr_f[g.l1];
+    hipLaunchKernelGGL(k_lower_level<T>, dim3(nblocks(b - a)), B, 0, S, P.d_lev_rows_f.p + a, b - a, A, F, in, out,
+                       (int)ic0, done);
+  }
+  for (const auto &g : P.seg_b) {
+    if (g.narrow) {
+      bwd(g, P.d_lev_rows_b.p, out, out);
+      continue;
+    }
+    const int a = P.lev_ptr_b[g.l0], b = P.lev_ptr_b[g.l1];
+    hipLaunchKernelGGL(k_upper_level<T>, dim3(nblocks(b - a)), B, 0, S, P.d_lev_rows_b.p + a, b - a, A, P.d_tpos.p, F,
+                       out, (int)ic0, done);
+  }
+  MS_CHECK_LAUNCH();
+}
+
+// F (holding the matrix) becomes its ILU(0) / IC(0) factor; *flag = 2 on a
+// breakdown
+void factor_levels(const SellPattern &P, double *F, bool ic0, int *flag) {
+  const LMat A = lmat(P);
+  for (const auto &g : P.seg_f) {
+    if (g.narrow) {
+      hipLaunchKernelGGL(k_factor_seg<double>, dim3(1), dim3(kSegThreads), 0, stream(), P.d_lev_ptr_f.p, g.l0, g.l1,
+                         P.d_lev_rows_f.p, A, F, (int)ic0, flag);
+      continue;
+    }
+    const int a = P.lev_ptr_f[g.l0], b = P.lev_ptr_f[g.l1];
+    hipLaunchKernelGGL(k_factor_level<double>, dim3(nblocks(b - a)), dim3(kBlock), 0, stream(), P.d_lev_rows_f.p + a,
+                       b - a, A, F, (int)ic0, flag);
+  }
+  MS_CHECK_LAUNCH();
+}
+
+template struct LevelFactor<double>;
+template struct LevelFactor<float>;
+
+}  // namespace ms

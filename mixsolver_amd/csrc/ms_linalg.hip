@@ -569,175 +569,6 @@ __global__ void k_jacobi(int n, const T *in, const T *dg, T *out, const int *don
   if (i < n) out[i] = in[i] / dg[i];
 }
 
-// natural IC(0) of row i, its lower neighbours final (mod_uns_linsolver.f90:328-365)
-template <class T>
-__device__ void ic0_factor_row(int i, const Mat &A, T *F, int *flag) {
-  const long long bi = A.off[i >> 6] + (i & 63);
-  const int dpi = A.diagk[i];
-  for (int kp = 0; kp < dpi; kp++) {
-    const long long qkp = bi + (long long)kp * kSlice;
-    const int k = A.col[qkp];
-    const long long bk = A.off[k >> 6] + (k & 63);
-    const int dpk = A.diagk[k];
-    int p = 0, q = 0;
-    T dsum = T(0);
-    while (p <= kp - 1 && q <= dpk - 1) {
-      const int cp = A.col[bi + (long long)p * kSlice], cq = A.col[bk + (long long)q * kSlice];
-      if (cp < cq) p++;
-      else if (cp > cq) q++;
-      else {
-        dsum = dsum + F[bi + (long long)p * kSlice] * F[bk + (long long)q * kSlice];
-        p++;
-        q++;
-      }
-    }
-    const T s = F[qkp] - dsum;
-    F[qkp] = s / F[bk + (long long)dpk * kSlice];
-  }
-  const long long qd = bi + (long long)dpi * kSlice;
-  T s = F[qd];
-  for (int kp = 0; kp < dpi; kp++) {
-    const T v = F[bi + (long long)kp * kSlice];
-    s = s - v * v;
-  }
-  if (s <= T(0)) {
-    *flag = 2;
-    return;
-  }
-  F[qd] = tsqrt(s);
-}
-
-// natural ILU(0) of row i, IKJ variant (mod_uns_linsolver.f90:79-115)
-template <class T>
-__device__ void ilu0_factor_row(int i, const Mat &A, T *F, int *flag) {
-  const long long bi = A.off[i >> 6] + (i & 63);
-  const int dpi = A.diagk[i], leni = A.rowlen[i];
-  for (int kk = 0; kk < dpi; kk++) {
-    const long long q = bi + (long long)kk * kSlice;
-    const int k = A.col[q];
-    const long long bk = A.off[k >> 6] + (k & 63);
-    const int dpk = A.diagk[k], lenk = A.rowlen[k];
-    const T piv = F[bk + (long long)dpk * kSlice];
-    if (tabs(piv) < (T)kTiny) {
-      *flag = 2;
-      return;
-    }
-    const T aik = F[q] / piv;
-    F[q] = aik;
-    for (int jj = dpk; jj < lenk; jj++) {
-      const int j = A.col[bk + (long long)jj * kSlice];
-      if (j <= k) continue;
-      for (int m = 0; m < leni; m++) {
-        const long long qm = bi + (long long)m * kSlice;
-        const int cm = A.col[qm];
-        if (cm == j) {
-          F[qm] = F[qm] - aik * F[bk + (long long)jj * kSlice];
-          break;
-        }
-        if (cm > j) break;
-      }
-    }
-  }
-}
-
-// forward substitution of row i (unit lower for ILU(0), L of IC(0))
-template <class T>
-__device__ void lower_row(int i, const Mat &A, const T *F, const T *r, T *z, int ic0) {
-  const long long bi = A.off[i >> 6] + (i & 63);
-  const int dpi = A.diagk[i];
-  T s = r[i];
-  for (int k = 0; k < dpi; k++) {
-    const long long q = bi + (long long)k * kSlice;
-    s = s - F[q] * z[A.col[q]];
-  }
-  z[i] = ic0 ? s / F[bi + (long long)dpi * kSlice] : s;
-}
-
-// backward substitution of row i (U of ILU(0), L^T of IC(0) via tpos)
-template <class T>
-__device__ void upper_row(int i, const Mat &A, const long long *tpos, const T *F, T *z, int ic0) {
-  const long long bi = A.off[i >> 6] + (i & 63);
-  const int dpi = A.diagk[i], len = A.rowlen[i];
-  T s = z[i];
-  if (ic0) {
-    for (int k = len - 1; k > dpi; k--) {
-      const long long q = bi + (long long)k * kSlice;
-      s = s - F[tpos[q]] * z[A.col[q]];
-    }
-  } else {
-    for (int k = dpi + 1; k < len; k++) {
-      const long long q = bi + (long long)k * kSlice;
-      s = s - F[q] * z[A.col[q]];
-    }
-  }
-  z[i] = s / F[bi + (long long)dpi * kSlice];
-}
-
-// one wide level: a thread per row
-template <class T>
-__global__ void k_factor_level(const int *rows, int nr, Mat A, T *F, int ic0, int *flag) {
-  int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= nr) return;
-  if (ic0) ic0_factor_row(rows[t], A, F, flag);
-  else ilu0_factor_row(rows[t], A, F, flag);
-}
-
-template <class T>
-__global__ void k_lower_level(const int *rows, int nr, Mat A, const T *F, const T *r, T *z, int ic0, const int *done) {
-  if (*done) return;
-  int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t < nr) lower_row(rows[t], A, F, r, z, ic0);
-}
-
-template <class T>
-__global__ void k_upper_level(const int *rows, int nr, Mat A, const long long *tpos, const T *F, T *z, int ic0,
-                              const int *done) {
-  if (*done) return;
-  int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t < nr) upper_row(rows[t], A, tpos, F, z, ic0);
-}
-
-// a run of narrow levels [l0, l1) in one workgroup: rows of a level are
-// spread over the threads, a barrier orders the levels (the workgroup shares
-// one L1, so rows of the next level see the values just stored).  Every
-// thread reaches every barrier: the level loop is uniform, only the row loop
-// inside a level depends on the thread.
-template <class T>
-__global__ __launch_bounds__(kSegThreads) void k_factor_seg(const int *lev_ptr, int l0, int l1, const int *rows,
-                                                             Mat A, T *F, int ic0, int *flag) {
-  for (int l = l0; l < l1; l++) {
-    const int a = lev_ptr[l], b = lev_ptr[l + 1];
-    for (int t = a + (int)threadIdx.x; t < b; t += kSegThreads) {
-      if (ic0) ic0_factor_row(rows[t], A, F, flag);
-      else ilu0_factor_row(rows[t], A, F, flag);
-    }
-    __syncthreads();
-  }
-}
-
-template <class T>
-__global__ __launch_bounds__(kSegThreads) void k_lower_seg(const int *lev_ptr, int l0, int l1, const int *rows, Mat A,
-                                                            const T *F, const T *r, T *z, int ic0, const int *done) {
-  if (*done) return;
-  for (int l = l0; l < l1; l++) {
-    const int a = lev_ptr[l], b = lev_ptr[l + 1];
-    for (int t = a + (int)threadIdx.x; t < b; t += kSegThreads) lower_row(rows[t], A, F, r, z, ic0);
-    __syncthreads();
-  }
-}
-
-template <class T>
-__global__ __launch_bounds__(kSegThreads) void k_upper_seg(const int *lev_ptr, int l0, int l1, const int *rows, Mat A,
-                                                            const long long *tpos, const T *F, T *z, int ic0,
-                                                            const int *done) {
-  if (*done) return;
-  for (int l = l0; l < l1; l++) {
-    const int a = lev_ptr[l], b = lev_ptr[l + 1];
-    for (int t = a + (int)threadIdx.x; t < b; t += kSegThreads) upper_row(rows[t], A, tpos, F, z, ic0);
-    __syncthreads();
-  }
-}
-
 template <class T>
 __global__ void k_dilu_first(int r0, int r1, const T *dg, const T *r, T *z, const int *done) {
   if (*done) return;
@@ -1089,18 +920,9 @@ int Krylov::setup_pc64(PcKind pc, const double *val) {
   if (fac_.n < (size_t)pat->nstore) fac_.alloc(pat->nstore);
   MS_HIP(hipMemcpyAsync(fac_.p, val, pat->nstore * sizeof(double), hipMemcpyDeviceToDevice, stream()));
   MS_HIP(hipMemsetAsync(flag_.p, 0, sizeof(int), stream()));
-  const int ic0 = pc == PC_NATURAL_IC0;
-  for (const auto &g : pat->seg_f) {
-    if (g.narrow) {
-      hipLaunchKernelGGL(k_factor_seg<double>, dim3(1), dim3(kSegThreads), 0, stream(), pat->d_lev_ptr_f.p, g.l0,
-                         g.l1, pat->d_lev_rows_f.p, A, fac_.p, ic0, flag_.p);
-      continue;
-    }
-    const int a = pat->lev_ptr_f[g.l0], b = pat->lev_ptr_f[g.l1];
-    hipLaunchKernelGGL(k_factor_level<double>, dim3(nblocks(b - a)), dim3(kBlock), 0, stream(),
-                       pat->d_lev_rows_f.p + a, b - a, A, fac_.p, ic0, flag_.p);
-  }
-  MS_CHECK_LAUNCH();
+  const bool ic0 = pc == PC_NATURAL_IC0;
+  factor_levels(*pat, fac_.p, ic0, flag_.p);
+  lev_.pack(*pat, fac_.p, ic0);
   int h = 0;
   MS_HIP(hipMemcpyAsync(hpin_, flag_.p, sizeof(int), hipMemcpyDeviceToHost, stream()));
   MS_HIP(hipStreamSynchronize(stream()));
@@ -1121,6 +943,7 @@ void Krylov::setup_pc32(PcKind pc, const double *val) {
     if (fac32_.n < (size_t)pat->nstore) fac32_.alloc(pat->nstore);
     hipLaunchKernelGGL(k_to_float, dim3(nblocks(pat->nstore)), dim3(kBlock), 0, stream(), pat->nstore, fac_.p,
                        fac32_.p);
+    lev32_.pack(*pat, fac32_.p, pc == PC_NATURAL_IC0);
   }
   MS_CHECK_LAUNCH();
 }
@@ -1162,27 +985,8 @@ void Krylov::apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const 
           hipLaunchKernelGGL((k_dilu_bwd<T, 0>), dim3(nblocks(cp[c + 1] - cp[c])), dim3(kBlock), 0, stream(), cp[c],
                              cp[c + 1], A, val, dg, in, out, done, (T *)nullptr);
   } else {
-    const int ic0 = pc == PC_NATURAL_IC0;
-    for (const auto &g : pat->seg_f) {
-      if (g.narrow) {
-        hipLaunchKernelGGL(k_lower_seg<T>, dim3(1), dim3(kSegThreads), 0, stream(), pat->d_lev_ptr_f.p, g.l0, g.l1,
-                           pat->d_lev_rows_f.p, A, fac, in, out, ic0, done);
-        continue;
-      }
-      const int a = pat->lev_ptr_f[g.l0], b = pat->lev_ptr_f[g.l1];
-      hipLaunchKernelGGL(k_lower_level<T>, dim3(nblocks(b - a)), dim3(kBlock), 0, stream(), pat->d_lev_rows_f.p + a,
-                         b - a, A, fac, in, out, ic0, done);
-    }
-    for (const auto &g : pat->seg_b) {
-      if (g.narrow) {
-        hipLaunchKernelGGL(k_upper_seg<T>, dim3(1), dim3(kSegThreads), 0, stream(), pat->d_lev_ptr_b.p, g.l0, g.l1,
-                           pat->d_lev_rows_b.p, A, pat->d_tpos.p, fac, out, ic0, done);
-        continue;
-      }
-      const int a = pat->lev_ptr_b[g.l0], b = pat->lev_ptr_b[g.l1];
-      hipLaunchKernelGGL(k_upper_level<T>, dim3(nblocks(b - a)), dim3(kBlock), 0, stream(), pat->d_lev_rows_b.p + a,
-                         b - a, A, pat->d_tpos.p, fac, out, ic0, done);
-    }
+    if constexpr (sizeof(T) == 8) lev_.apply(*pat, fac, pc == PC_NATURAL_IC0, in, out, done);
+    else lev32_.apply(*pat, fac, pc == PC_NATURAL_IC0, in, out, done);
   }
   MS_CHECK_LAUNCH();
 }

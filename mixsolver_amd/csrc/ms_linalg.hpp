@@ -77,6 +77,17 @@ void set_schur_matfree(bool on);
 // Preconditioner kinds used internally.
 enum PcKind { PC_JACOBI = 0, PC_NATURAL_IC0 = 1, PC_NATURAL_ILU0 = 2, PC_DILU = 3 };
 
+// ms_levels.hip: the natural-order factor packed in the order of the
+// level-scheduled sweeps, and their application
+template <class T>
+struct LevelFactor {
+  DBuf<T> vf, vb, df, db;   // forward / backward entries and diagonals, step order
+  void pack(const SellPattern &P, const T *F, bool ic0);
+  DBuf<T> xf, xb;           // vectors in level order (SellPattern::sweep_ordered)
+  void apply(const SellPattern &P, const T *F, bool ic0, const T *in, T *out, const int *done);
+};
+void factor_levels(const SellPattern &P, double *F, bool ic0, int *flag);
+
 class Krylov {
  public:
   explicit Krylov(const SellPattern *pat);
@@ -131,6 +142,8 @@ class Krylov {
   DBuf<double> cnu_split_;   // c.nu parts of k_finish_split
   DBuf<float> pq32_;         // the SpMV's p.q partials on the split path
   DBuf<int> flag_;
+  LevelFactor<double> lev_;
+  LevelFactor<float> lev32_;
   CoarseMat cm_;             // E, E^-1 and nu of the coarse space for the current matrix
   DBuf<double> co_part_;     // chunk sums of a BiCGSTAB coarse correction
   const MatFree *mf_ = nullptr;

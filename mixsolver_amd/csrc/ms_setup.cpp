@@ -237,6 +237,8 @@ void csr_to_sell(SellPattern &P, int n, const std::vector<int> &rp, const std::v
   }
 }
 
+void plan_sweeps(SellPattern &P, const std::vector<int> &rows_f, const std::vector<int> &rows_b);   // ms_levels.hip
+
 void SellPattern::build_levels() {
   // forward: level(i) = 1 + max level of lower neighbours; backward on upper
   std::vector<int> lf(n, 0), lb(n, 0);
@@ -269,13 +271,13 @@ void SellPattern::build_levels() {
     const int nl = (int)ptr.size() - 1;
     for (int l = 0; l < nl;) {
       if (ptr[l + 1] - ptr[l] > kNarrowRows) {
-        seg.push_back({l, l + 1, false});
+        seg.push_back({l, l + 1, false, 0, 0, 0, 0});
         l++;
         continue;
       }
       int e = l;
       while (e < nl && ptr[e + 1] - ptr[e] <= kNarrowRows) e++;
-      seg.push_back({l, e, true});
+      seg.push_back({l, e, true, 0, 0, 0, kSegThreads});
       l = e;
     }
   };
@@ -285,6 +287,7 @@ void SellPattern::build_levels() {
   d_lev_rows_b.upload(rb);
   d_lev_ptr_f.upload(lev_ptr_f);
   d_lev_ptr_b.upload(lev_ptr_b);
+  plan_sweeps(*this, rf, rb);
   has_levels = true;
 }
 
@@ -303,7 +306,7 @@ void SellPattern::upload() {
 size_t SellPattern::device_bytes() const {
   return d_off.bytes() + d_rowlen.bytes() + d_col.bytes() + d_diagk.bytes() + d_tpos.bytes() +
          d_lev_rows_f.bytes() + d_lev_rows_b.bytes() + d_lev_ptr_f.bytes() + d_lev_ptr_b.bytes() +
-         coarse.device_bytes() + d_col16.bytes() + d_cbase.bytes();
+         sweep_f.bytes() + sweep_b.bytes() + d_lev_fb.bytes() + coarse.device_bytes() + d_col16.bytes() + d_cbase.bytes();
 }
 
 // ------------------------------------------------------------ orderings
