@@ -332,6 +332,8 @@ struct FinRU {         // after x += sigma*y and r = b - A x in FP64
     }
     st->scale = st->sigma / rt;            // p and r.z move to the new scale
     st->rz = st->rz * st->scale * st->scale;
+    for (double &v : st->rz2) v = v * st->scale * st->scale;
+    st->trig = 1;
     st->sigma = rt;
     st->rmax = 1.0;
     st->ru = 2;                            // k_ru_rescale pending

@@ -369,6 +369,307 @@ __global__ void k_pcg_p_split(Rows R, const T *r, const T *dg, T *p, const doubl
   }
 }
 
+// ------------------------------------------------------- two-launch PCG
+// PCG without a coarse space.  An iteration is the launch-bound end of a
+// solve: at 16,000 rows its five kernels (product, alpha, update, beta, p)
+// took 15.5 us for 3 us of memory traffic.  Here the scalar recurrences have no
+// kernels of their own: every workgroup reduces the partials of the launch
+// before it, in the same fixed order, so all hold the same alpha or beta,
+// and workgroup 0 keeps the solver state; and the p update rides along the
+// product, which forms each neighbour's p = z + beta p_old from the two
+// vectors (p is double-buffered, so nobody reads what this launch writes).
+//   k_cg_ps: [r.r, r.z -> stop?, beta]  p = z + beta p_old, q = A p; p.q
+//   k_cg_xr: [p.q -> alpha]             x += alpha p, r -= alpha q; r.r
+//            and with Jacobi z = r/d; r.z
+// Preconditioners with sweeps run between the two and leave their own r.z
+// partials.  The grid is capped so that the partials every workgroup reads
+// stay few; a workgroup takes a contiguous range of row blocks.
+// Kernel time per iteration, five launches before, two now: 13.4 -> 7.4 us at
+// 1,728 rows in FP64, 15.5 -> 7.3 at 16,384, 21 -> 13.2 at 216,000; 20.5 ->
+// 16.3 at 432,000 rows in FP32.
+// The parity of the iteration comes from the device's own count: st->it
+// changes in k_cg_xr only, st->par in k_cg_ps only.
+constexpr int kCgGrid = 2048;
+constexpr int kCgPre = 8;   // entries of the first row loaded before the partials arrive
+
+struct RowRange {
+  int b0, b1;
+};
+__device__ __forceinline__ RowRange cg_range(int n) {
+  const int nb = (n + kBlock - 1) / kBlock, G = gridDim.x, b = xcd_block(blockIdx.x, G);
+  return RowRange{(int)((long long)b * nb / G), (int)((long long)(b + 1) * nb / G)};
+}
+
+// sum of up to two partial arrays by a whole workgroup, in a fixed order
+template <class T>
+__device__ __forceinline__ void cg_sums(int n1, const T *p1, int n2, const T *p2, T (&a)[2]) {
+  __shared__ T lds[2 * (kBlock / 64)];
+  a[0] = a[1] = T(0);
+  int b = threadIdx.x;
+  const int nmax = max(n1, n2);
+  for (; b < nmax; b += 4 * kBlock) {
+    T u[4], v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int i = b + j * kBlock;
+      u[j] = i < n1 ? p1[i] : T(0);
+      v[j] = i < n2 ? p2[i] : T(0);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      a[0] = a[0] + u[j];
+      a[1] = a[1] + v[j];
+    }
+  }
+  block_reduce<OpSum, 2, T, kBlock>(a, lds);
+}
+
+struct CgParts {   // r.r and r.z partials of the last update / preconditioner
+  int nrr, nrz;
+};
+
+// The residual test and beta of the next iteration from the partials (all
+// threads call it; the result is thread 0's).  Returns 0 go on, 1 converged,
+// 2 breakdown.  writer: keep the solver state.
+// mixed: the FP32 iteration on r / sigma, as FinUpdateRU.
+template <class T, bool MIXED>
+__device__ __forceinline__ int cg_test(KS *st, int first, T rr, T rz, int par, bool writer, double &beta) {
+  const double rzn = (double)rz, old = st->rz2[par ^ 1];
+  beta = 0.0;
+  if (!first) {
+    if constexpr (MIXED) {
+      const double rn = sqrt((double)rr), res = rn * st->sigma / st->bnrm;
+      const bool test = !st->trig;
+      if (writer) {
+        st->res = res;
+        if (test && (res <= st->tol || rn < st->delta * st->rmax)) st->ru = 1;
+        if (!test) st->ru = 0;
+      }
+      if (test && res <= st->tol) {
+        if (writer) st->done = 2;
+        return 1;
+      }
+      if (writer && rn > st->rmax) st->rmax = rn;
+    } else {
+      const double res = sqrt((double)rr) / st->bnrm;
+      if (writer) {
+        st->rr = rr;
+        st->res = res;
+      }
+      if (res <= st->tol) {
+        if (writer) st->done = 1;
+        return 1;
+      }
+    }
+    if (fabs(old) < kTiny) {
+      if (writer) {
+        st->ierr = 2;
+        st->done = 1;
+      }
+      return 2;
+    }
+    beta = rzn / old;
+  }
+  return 0;
+}
+
+template <class T, bool MIXED, int C16>
+__global__ __launch_bounds__(kBlock) void k_cg_ps(int n, Mat A, const T *val, const T *z, T *p0, T *p1, T *q, KS *st,
+                                                  CgParts np, const T *rrp, const T *rzp, T *pqp) {
+  if (st->done) return;
+  const int first = st->it == 0, par = st->it & 1;
+  const T *po = par ? p0 : p1;
+  T *pn = par ? p1 : p0;
+  const RowRange R = cg_range(n);
+  __shared__ double beta_s;
+  __shared__ int stop_s;
+  // the first row's matrix entries and vector values are loaded before the
+  // partials are waited for
+  int i = R.b0 * kBlock + threadIdx.x, w = 0;
+  long long base = 0;
+  int c[kCgPre];
+  T a[kCgPre], zc[kCgPre], pc[kCgPre], zi = T(0), pi = T(0);
+  auto load = [&]() {
+    const int s = i >> 6;
+    const long long o0 = A.off[s];
+    w = (int)((A.off[s + 1] - o0) >> 6);
+    base = o0 + (i & 63);
+    zi = z[i];
+    pi = first ? T(0) : po[i];
+#pragma unroll
+    for (int k = 0; k < kCgPre; k++) c[k] = k < w ? col_at<C16>(A, base + (long long)k * kSlice, i, s) : i;
+#pragma unroll
+    for (int k = 0; k < kCgPre; k++) a[k] = k < w ? val[base + (long long)k * kSlice] : T(0);
+#pragma unroll
+    for (int k = 0; k < kCgPre; k++) zc[k] = k < w ? z[c[k]] : T(0);
+#pragma unroll
+    for (int k = 0; k < kCgPre; k++) pc[k] = (k < w && !first) ? po[c[k]] : T(0);
+  };
+  if (R.b0 < R.b1 && i < n) load();
+  T sums[2];
+  cg_sums<T>(np.nrr, rrp, np.nrz, rzp, sums);
+  if (threadIdx.x == 0) {
+    double beta;
+    stop_s = cg_test<T, MIXED>(st, first, sums[0], sums[1], par, blockIdx.x == 0, beta);
+    beta_s = beta;
+    if (blockIdx.x == 0 && !stop_s) {
+      st->beta = beta;
+      st->rz2[par] = (double)sums[1];
+      st->par = par;
+    }
+  }
+  __syncthreads();
+  if (stop_s) return;
+  const T beta = (T)beta_s;
+  T v[1] = {T(0)};
+  for (int b = R.b0; b < R.b1; b++) {
+    i = b * kBlock + threadIdx.x;
+    if (i < n) {
+      if (b > R.b0) load();
+      const T xi = zi + beta * pi;
+      T acc = T(0);
+#pragma unroll
+      for (int k = 0; k < kCgPre; k++)
+        if (k < w) {
+          const T xk = zc[k] + beta * pc[k];
+          if constexpr (sizeof(T) == 4) acc = acc + a[k] * (c[k] == i ? xi : xk - xi);
+          else acc = acc + a[k] * xk;
+        }
+      for (int k = kCgPre; k < w; k++) {
+        const long long e = base + (long long)k * kSlice;
+        const int ck = col_at<C16>(A, e, i, i >> 6);
+        const T xk = z[ck] + beta * (first ? T(0) : po[ck]);
+        if constexpr (sizeof(T) == 4) acc = acc + val[e] * (ck == i ? xi : xk - xi);
+        else acc = acc + val[e] * xk;
+      }
+      pn[i] = xi;
+      q[i] = acc;
+      v[0] = v[0] + xi * acc;
+    }
+  }
+  block_partials<OpSum, 1>(v, pqp);
+}
+
+// mode 1 Jacobi (z = r/d, r.z), 2 DILU (z = r/d on the first colour block),
+// 0 neither
+template <class T, class X>
+__global__ __launch_bounds__(kBlock) void k_cg_xr(int n, const T *p0, const T *p1, const T *q, X *x, T *r, T *z,
+                                                  const T *dg, int mode, int c0end, KS *st, int npq, const T *pqp,
+                                                  T *rrp, T *rzp) {
+  if (st->done) return;
+  const int par = st->par;
+  const T *p = par ? p1 : p0;
+  const RowRange R = cg_range(n);
+  __shared__ double alpha_s;
+  __shared__ int bad_s;
+  int i = R.b0 * kBlock + threadIdx.x;
+  T pi = T(0), qi = T(0), ri = T(0), di = T(1);
+  X xi = X(0);
+  auto load = [&]() {
+    pi = p[i];
+    qi = q[i];
+    ri = r[i];
+    xi = x[i];
+    if (mode == 1 || (mode == 2 && i < c0end)) di = dg[i];
+  };
+  if (R.b0 < R.b1 && i < n) load();
+  T sums[2];
+  cg_sums<T>(npq, pqp, 0, pqp, sums);
+  if (threadIdx.x == 0) {
+    const double pap = (double)sums[0];
+    const int bad = fabs(pap) < kTiny;
+    bad_s = bad;
+    alpha_s = bad ? 0.0 : st->rz2[par] / pap;
+    if (blockIdx.x == 0) {
+      st->it = st->it + 1;
+      st->pap = pap;
+      st->trig = 0;
+      if (bad) {
+        st->ierr = 2;
+        st->done = 1;
+      } else {
+        st->alpha = alpha_s;
+      }
+    }
+  }
+  __syncthreads();
+  if (bad_s) return;
+  const T alpha = (T)alpha_s;
+  T v[2] = {T(0), T(0)};
+  for (int b = R.b0; b < R.b1; b++) {
+    i = b * kBlock + threadIdx.x;
+    if (i < n) {
+      if (b > R.b0) load();
+      x[i] = xi + (X)(alpha * pi);
+      const T rn = ri - alpha * qi;
+      r[i] = rn;
+      v[0] = v[0] + rn * rn;
+      if (mode == 1 || (mode == 2 && i < c0end)) {
+        const T zn = rn / di;
+        z[i] = zn;
+        if (mode == 1) v[1] = v[1] + rn * zn;
+      }
+    }
+  }
+  __shared__ T lds[2 * (kBlock / 64)];
+  block_reduce<OpSum, 2, T>(v, lds);
+  if (threadIdx.x == 0) {
+    rrp[blockIdx.x] = v[0];
+    if (mode == 1) rzp[blockIdx.x] = v[1];
+  }
+}
+
+// the residual test after the last update of a chunk, for the host to read
+// (the next k_cg_ps comes to the same answer)
+template <class T, bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_cg_peek(KS *st, int nrr, const T *rrp) {
+  if (st->done || st->it == 0) return;
+  T sums[2];
+  cg_sums<T>(nrr, rrp, 0, rrp, sums);
+  if (threadIdx.x != 0) return;
+  const double rn = sqrt((double)sums[0]);
+  if constexpr (MIXED) {
+    st->res = rn * st->sigma / st->bnrm;
+    if (!st->trig && (st->res <= st->tol || rn < st->delta * st->rmax)) st->ru = 1;
+    if (!st->trig && st->res <= st->tol) st->done = 2;
+  } else {
+    st->rr = (double)sums[0];
+    st->res = rn / st->bnrm;
+    if (st->res <= st->tol) st->done = 1;
+  }
+}
+
+// after a reliable update: r32 = r64 / sigma, the p the next k_cg_ps reads as
+// the old one moved to the new scale, r.r and z, r.z as k_cg_xr
+__global__ __launch_bounds__(kBlock) void k_cg_rescale(int n, const double *r64, float *r32, float *p0, float *p1,
+                                                       float *z, const float *dg, int mode, int c0end, const KS *st,
+                                                       float *rrp, float *rzp) {
+  if (st->done || st->ru != 2) return;
+  const RowRange R = cg_range(n);
+  float *p = (st->it & 1) ? p0 : p1;
+  float v[2] = {0.0f, 0.0f};
+  for (int b = R.b0; b < R.b1; b++) {
+    const int i = b * kBlock + threadIdx.x;
+    if (i < n) {
+      const float ri = (float)(r64[i] / st->sigma);
+      r32[i] = ri;
+      p[i] = p[i] * (float)st->scale;
+      v[0] = v[0] + ri * ri;
+      if (mode == 1 || (mode == 2 && i < c0end)) {
+        const float zi = ri / dg[i];
+        z[i] = zi;
+        if (mode == 1) v[1] = v[1] + ri * zi;
+      }
+    }
+  }
+  __shared__ float lds[2 * (kBlock / 64)];
+  block_reduce<OpSum, 2, float>(v, lds);
+  if (threadIdx.x == 0) {
+    rrp[blockIdx.x] = v[0];
+    if (mode == 1) rzp[blockIdx.x] = v[1];
+  }
+}
+
 __global__ void k_clear_pup(KS *st) {
   if (threadIdx.x == 0) st->pup = 0;
 }
@@ -381,17 +682,23 @@ __global__ void k_dot(int n, const T *a, const T *b, const KS *st, T *part) {
   block_partials<OpSum, 1>(v, part);
 }
 
+// z of the initial residual: r/d and r.z (mode 1), r/d on the first colour
+// block (mode 2)
 template <class T>
-__global__ void k_jac_rz(int n, const T *r, const T *dg, T *z, const KS *st, T *part) {
+__global__ __launch_bounds__(kBlock) void k_cg_z(int n, const T *r, const T *dg, T *z, int mode, int c0end,
+                                                 const KS *st, T *rzp) {
   if (st->done) return;
-  int i = blockIdx.x * kBlock + threadIdx.x;
+  const RowRange R = cg_range(n);
   T v[1] = {T(0)};
-  if (i < n) {
-    T zi = r[i] / dg[i];
-    z[i] = zi;
-    v[0] = r[i] * zi;
+  for (int b = R.b0; b < R.b1; b++) {
+    const int i = b * kBlock + threadIdx.x;
+    if (i < (mode == 2 ? c0end : n)) {
+      const T ri = r[i], zi = ri / dg[i];
+      z[i] = zi;
+      v[0] = v[0] + ri * zi;
+    }
   }
-  block_partials<OpSum, 1>(v, part);
+  if (mode == 1) block_partials<OpSum, 1>(v, rzp);
 }
 
 // ------------------------------------------------------- reliable updates
@@ -1108,6 +1415,81 @@ void Krylov::coarse_apply(const T *in, T *out, const int *done, KS *st) {
   hipLaunchKernelGGL((k_co_prolong<T>), dim3(C.nchunks), dim3(kBlock), 0, stream(), RW, cm_.nu.p, out, done);
 }
 
+// buffers of the two-launch PCG: the vectors of the precision, p double
+// buffered in the BiCGSTAB's ph, three partial arrays
+template <class T>
+Krylov::Cg2<T> Krylov::cg2(PcKind pc) {
+  Cg2<T> c;
+  c.pc = pc;
+  c.mode = pc == PC_JACOBI ? 1 : (pc == PC_DILU ? 2 : 0);
+  c.G = std::min(nblk_, kCgGrid);
+  const size_t stride = (size_t)nblk_ + 64;
+  T *part;
+  if constexpr (sizeof(T) == 8) {
+    c.r = r_.p, c.z = z_.p, c.p0 = p_.p, c.p1 = ph_.p, c.q = q_.p, c.dg = dg_.p;
+    part = part_.p;
+    c.swp = prz_.p;
+  } else {
+    c.r = r32_.p, c.z = z32_.p, c.p0 = p32_.p, c.p1 = ph32_.p, c.q = q32_.p, c.dg = dg32_.p;
+    part = part32_.p;
+    c.swp = prz32_.p;
+  }
+  c.rr = part;
+  c.rz = part + stride;
+  c.pq = part + 2 * stride;
+  c.nrz = c.G;
+  if (c.mode == 2) {   // the sweeps' partials: rows of colours 1.. forward, all but the last backward
+    const auto &cp = pat->color_ptr;
+    const int nc = (int)cp.size() - 1;
+    c.nrz = 0;
+    for (int k = 1; k < nc; k++) c.nrz += nblocks(cp[k + 1] - cp[k]);
+    for (int k = nc - 2; k >= 0; k--) c.nrz += nblocks(cp[k + 1] - cp[k]);
+    c.rz = c.swp;
+  } else if (c.mode == 0) {
+    c.nrz = nblk_;
+    c.rz = c.swp;
+  }
+  return c;
+}
+
+// z and the r.z partials of the current r
+template <class T>
+void Krylov::cg2_precond(const Cg2<T> &c, const T *val, const T *fac) {
+  if (c.mode == 2) {
+    dilu_sweeps<T>(pat, matof(pat), val, c.dg, c.r, c.z, &st_.p->done, c.swp);
+  } else if (c.mode == 0) {
+    apply_pc<T>(c.pc, val, fac, c.dg, c.r, c.z, &st_.p->done);
+    hipLaunchKernelGGL(k_dot<T>, dim3(nblk_), dim3(kBlock), 0, stream(), n, c.r, c.z, st_.p, c.swp);
+  }
+}
+
+template <class T>
+void Krylov::cg2_start(const Cg2<T> &c, const T *val, const T *fac) {
+  if (c.mode)
+    hipLaunchKernelGGL(k_cg_z<T>, dim3(c.G), dim3(kBlock), 0, stream(), n, c.r, c.dg, c.z, c.mode, pat->color_ptr[1],
+                       st_.p, c.rz);
+  cg2_precond<T>(c, val, fac);
+  MS_CHECK_LAUNCH();
+}
+
+template <class T, bool MIXED, class X>
+void Krylov::cg2_iteration(const Cg2<T> &c, const T *val, const T *fac, X *x, hipEvent_t e0, hipEvent_t e1) {
+  const Mat A = matof(pat);
+  const dim3 G(c.G), B(kBlock);
+  hipStream_t S = stream();
+  auto ps = [&](auto k) {
+    if (e0) hipExtLaunchKernelGGL(k, G, B, 0, S, e0, e1, 0, n, A, val, c.z, c.p0, c.p1, c.q, st_.p, CgParts{c.G, c.nrz},
+                                  c.rr, c.rz, c.pq);
+    else hipLaunchKernelGGL(k, G, B, 0, S, n, A, val, c.z, c.p0, c.p1, c.q, st_.p, CgParts{c.G, c.nrz}, c.rr, c.rz,
+                            c.pq);
+  };
+  if (sizeof(T) == 4 && pat->has16) ps(k_cg_ps<T, MIXED, 1>);
+  else ps(k_cg_ps<T, MIXED, 0>);
+  hipLaunchKernelGGL((k_cg_xr<T, X>), G, B, 0, S, n, c.p0, c.p1, c.q, x, c.r, c.z, c.dg, c.mode, pat->color_ptr[1],
+                     st_.p, c.G, c.pq, c.rr, c.rz);
+  cg2_precond<T>(c, val, fac);
+}
+
 SolveResult Krylov::pcg(const double *val, const double *b, double *x, double tol, int maxit, PcKind pc,
                         bool coarse, bool reuse) {
   SolveResult R;
@@ -1151,6 +1533,28 @@ SolveResult Krylov::pcg(const double *val, const double *b, double *x, double to
   if (hs.done) return R;
   const int jac = pc == PC_JACOBI;
   const int *done = &st->done;
+  if (!coarse) {
+    const Cg2<double> cg = cg2<double>(pc);
+    cg2_start<double>(cg, val, fac_.p);
+    for (int enq = 0, chunk = 8;;) {
+      const int m = std::min(chunk, maxit - enq);
+      for (int it = 0; it < m; it++) cg2_iteration<double, false>(cg, val, fac_.p, x, nullptr, nullptr);
+      hipLaunchKernelGGL((k_cg_peek<double, false>), dim3(1), B, 0, S, st, cg.G, cg.rr);
+      MS_CHECK_LAUNCH();
+      enq += m;
+      hs = read_state<double>(st);
+      if (hs.done || enq >= maxit) break;
+      chunk = std::min(chunk * 2, 128);
+    }
+    R.it = hs.it;
+    R.res = hs.res;
+    R.ierr = hs.ierr;
+    if (!hs.done) {        // DO-loop exhaustion: it = maxit + 1, ierr = 1
+      R.it = maxit + 1;
+      R.ierr = 1;
+    }
+    return R;
+  }
   const Rows RW = rows_of(pat, coarse);
   const dim3 GR(coarse ? pat->coarse.nchunks : nblk_);
   const CoDev co = codev_of(pat, cm_, coarse, st);
@@ -1562,7 +1966,13 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
   MS_HIP(hipMemsetAsync(y, 0, n * sizeof(float), S));
   hipLaunchKernelGGL(k_set_sigma, dim3(1), dim3(64), 0, S, st);
   hipLaunchKernelGGL(k_scale_down, G, B, 0, S, n, r_.p, r, st);
-  if (fused) {
+  // without a coarse space the two-launch iteration (the matrix-free product
+  // has launches of its own)
+  const bool two = !coarse && !matfree_on();
+  const Cg2<float> cg = two ? cg2<float>(pc) : Cg2<float>{};
+  if (two) {
+    cg2_start<float>(cg, v32, fac);
+  } else if (fused) {
     hipLaunchKernelGGL(k_rsum<float>, GR, B, 0, S, RW, r, st, part32);
     const auto &cp = pat->color_ptr;
     hipLaunchKernelGGL(k_dilu_first<float>, dim3(nblocks(cp[1] - cp[0])), B, 0, S, cp[0], cp[1], dg, r, z, done);
@@ -1617,6 +2027,16 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
     hipLaunchKernelGGL(k_pcg_p<float>, GR, B, 0, S, RW, r, z, dg, jac, p, nu, st);
   };
   auto reliable_update = [&](bool paused) {
+    if (two) {   // the p update of the last iteration is always pending here
+      hipLaunchKernelGGL(k_fold, G, B, 0, S, n, y, x, st);
+      hipLaunchKernelGGL(k_true_res, G, B, 0, S, n, A, val, b, x, r_.p, st, part);
+      finish<OpSum, 1>(nblk_, part, FinRU{st});
+      hipLaunchKernelGGL(k_cg_rescale, dim3(cg.G), B, 0, S, n, r_.p, r, cg.p0, cg.p1, z, dg, mode, c0end, st, cg.rr,
+                         cg.rz);
+      cg2_precond<float>(cg, v32, fac);
+      MS_CHECK_LAUNCH();
+      return;
+    }
     if (pfused) {   // apply a pending p update before r, p and z are rescaled
       hipLaunchKernelGGL(k_pcg_p_split<float>, GR, B, 0, S, RW, r, dg, p, nu, st, cnu_split_.p, nsplit, 1);
       hipLaunchKernelGGL(k_clear_pup, dim3(1), dim3(64), 0, S, st);
@@ -1637,6 +2057,19 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
   if (split && pq32_.n < (size_t)nblk_) pq32_.alloc(nblk_);
   float *spart = split ? pq32_.p : part32;
   auto chunk = [&](int m, bool probe_last) {
+    if (two) {
+      for (int it = 0; it < m; it++) {
+        hipEvent_t e0 = nullptr, e1 = nullptr;
+        if (probe_last && it == m - 1) {
+          probe_pair = g_probe.next;
+          g_probe.next = (g_probe.next + 1) % kProbePairs;
+          e0 = g_probe.ev[2 * probe_pair], e1 = g_probe.ev[2 * probe_pair + 1];
+        }
+        cg2_iteration<float, true>(cg, v32, fac, y, e0, e1);
+      }
+      hipLaunchKernelGGL((k_cg_peek<float, true>), dim3(1), B, 0, S, st, cg.G, cg.rr);
+      return;
+    }
     for (int it = 0; it < m; it++) {
       if (probe_last && it == m - 1) {
         probe_pair = g_probe.next;

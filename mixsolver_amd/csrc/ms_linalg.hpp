@@ -17,6 +17,11 @@ struct KS {              // device-resident solver scalars (one per solve)
   int ru;                // reliable update requested for this iteration
   int nru;               // reliable updates performed
   int pup;               // a p update is pending for the next product (fused p update)
+  // two-launch PCG (k_cg_ps / k_cg_xr): r.z of the last two iterations, the
+  // parity of the iteration under way, and whether r comes from a reliable
+  // update (its residual is not tested again)
+  double rz2[2];
+  int par, trig;
 };
 
 struct SolveResult {
@@ -131,6 +136,18 @@ class Krylov {
   template <class T> void apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const T *in, T *out,
                                    const int *done);
   template <class T> KS read_state(KS *d);
+  // two-launch PCG (no coarse space): its vectors and partial arrays
+  template <class T> struct Cg2 {
+    PcKind pc = PC_JACOBI;
+    int mode = 0, G = 0, nrz = 0;   // grid; r.z partials in rz
+    T *r = nullptr, *z = nullptr, *p0 = nullptr, *p1 = nullptr, *q = nullptr, *dg = nullptr;
+    T *rr = nullptr, *rz = nullptr, *pq = nullptr, *swp = nullptr;
+  };
+  template <class T> Cg2<T> cg2(PcKind pc);
+  template <class T> void cg2_precond(const Cg2<T> &c, const T *val, const T *fac);
+  template <class T> void cg2_start(const Cg2<T> &c, const T *val, const T *fac);
+  template <class T, bool MIXED, class X>
+  void cg2_iteration(const Cg2<T> &c, const T *val, const T *fac, X *x, hipEvent_t e0, hipEvent_t e1);
   SolveResult bicg32(PcKind pc, int maxit, int window, bool coarse);
   template <class T> void coarse_apply(const T *in, T *out, const int *done, KS *st);
   void ensure32();

@@ -1,0 +1,55 @@
+"""The two-launch PCG (no coarse space) at the sizes where its launches
+change form: one row, a partial and a full workgroup, rows with more entries
+than are loaded ahead of the partials, and more row blocks than the capped
+grid has workgroups.
+
+FP64 against the oracle after k iterations: only the order of the dot
+products' sums differs, so the histories agree to the bar of the
+reference's solver histories (1e-10).  Mixed precision against the FP64
+residual it is asked for."""
+import numpy as np
+import pytest
+
+from mixsolver_amd import linsolver
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(n, lags, seed=3):
+    rng = np.random.default_rng(seed)
+    rows, cols, vals = [np.arange(n)], [np.arange(n)], [np.zeros(n)]
+    for lag in lags:
+        if lag >= n:
+            continue
+        i = np.arange(lag, n)
+        w = rng.uniform(0.5, 1.5, n - lag)
+        rows += [i, i - lag]
+        cols += [i - lag, i]
+        vals += [-w, -w]
+    rows, cols, vals = (np.concatenate(v) for v in (rows, cols, vals))
+    vals[:n] = np.bincount(rows, np.abs(vals), n) * 1.05 + 0.1
+    o = np.lexsort((cols, rows))
+    rp = (np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]) + 1).astype(np.int32)
+    return rp, (cols[o] + 1).astype(np.int32), vals[o], rng.normal(size=n)
+
+
+@pytest.mark.parametrize("n,lags", [(1, ()), (2, (1,)), (255, (1, 7)), (256, (1, 7)), (257, (1, 7, 100)),
+                                    (5000, (1, 2, 3, 5, 8, 13, 21)), (2048 * 256 + 3, (1, 300))])
+def test_two_launch_pcg_against_oracle(n, lags):
+    from oracle import pyoracle
+    rp, ci, val, b = _system(n, lags)
+    for k in (1, 2, 7):
+        x, it, res, ierr = linsolver.cg_jacobi(rp, ci, val, b, np.zeros(n), 1e-30, k)
+        xr, itr, resr, ierrr = pyoracle.solve("cg_jacobi", rp, ci, val, b, np.zeros(n), 1e-30, k, mpi=True)
+        assert (it, ierr) == (itr, ierrr), k
+        assert np.linalg.norm(x - xr) <= 1e-10 * np.linalg.norm(xr), k
+        if n > 2:   # a one- or two-row system is solved to rounding by then
+            assert abs(res - resr) <= 1e-10 * resr, (k, res, resr)
+    # FP32 Krylov directions run out on a system of a few rows before the
+    # reliable updates reach 1e-10, so mixed precision starts at a workgroup
+    for prec in ("fp64", "mixed") if n >= 255 else ("fp64",):
+        x, it, res, ierr = linsolver.solve(rp, ci, val, b, np.zeros(n), 1e-10, 500, precision=prec, inner_tol=0.1)
+        row = np.repeat(np.arange(n), np.diff(rp))
+        r = b - np.bincount(row, val * x[ci - 1], n)
+        assert ierr == 0 and res <= 1e-10
+        assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(b), (prec, np.linalg.norm(r) / np.linalg.norm(b))
