@@ -560,30 +560,16 @@ static void solve_csr(int n, const int *row_ptr, const int *col_idx, const doubl
                       double *res, int *ierr) {
   if (n <= 0 || !row_ptr || !col_idx || !val || !b || !x) fail(MS_EINVAL, "bad solver arguments");
   ensure_runtime(-1);
-  std::vector<int> rp(n + 1), ci(row_ptr[n] - 1);
-  for (int i = 0; i <= n; i++) rp[i] = row_ptr[i] - 1;
-  for (size_t k = 0; k < ci.size(); k++) {
-    ci[k] = col_idx[k] - 1;
-    if (ci[k] < 0 || ci[k] >= n) fail(MS_EINVAL, "column index out of range");
-  }
-  for (int i = 0; i < n; i++)
-    for (int k = rp[i] + 1; k < rp[i + 1]; k++)
-      if (ci[k] <= ci[k - 1]) fail(MS_EINVAL, "CSR columns must be strictly ascending per row");
-  SellPattern pat;
-  csr_to_sell(pat, n, rp, ci);
   if (precond == MS_PC_DILU) {
     // colour classes in natural order (rows renumbering is the caller's choice)
     fail(MS_EINVAL, "DILU needs a colour-blocked ordering; use a system with gpu_ppe_precond = dilu");
   }
-  pat.upload();
-  if (precond == MS_PC_NATURAL) pat.build_levels();
-  std::vector<double> vs(pat.nstore, 0.0);
-  for (int r = 0; r < n; r++)
-    for (int k = 0; k < pat.rowlen[r]; k++) vs[pat.slot(r, k)] = val[rp[r] + k];
+  SellPattern pat;
   DBuf<double> dv, db, dx;
-  dv.upload(vs);
+  csr_to_device(pat, n, row_ptr, col_idx, val, precond == MS_PC_NATURAL, dv);
   db.upload(b, n);
   dx.upload(x, n);
+  if (precond == MS_PC_NATURAL) pat.build_levels(row_ptr, col_idx);
   Krylov K(&pat);
   PcKind pc = precond == MS_PC_JACOBI ? PC_JACOBI : (solver == 0 ? PC_NATURAL_IC0 : PC_NATURAL_ILU0);
   SolveResult R;

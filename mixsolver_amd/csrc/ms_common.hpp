@@ -241,11 +241,16 @@ struct SellPattern {
   Coarse coarse;                     // coarse space of the pressure-correction solves
   long long slot(int r, int k) const { return off[r / kSlice] + (long long)k * kSlice + (r % kSlice); }
   void build_from_csr(int n, const std::vector<int> &rp0, const std::vector<int> &ci0); // 0-based CSR
-  void build_levels();
+  void build_levels();                                          // from the host arrays above
+  void build_levels(const int *row_ptr, const int *col_idx);    // from the caller's 1-based CSR
+  template <class Col> void build_levels_from(Col col_of);
   void upload();
   size_t device_bytes() const;
 };
 
-
+// a caller's CSR to the device arrays of P and its values in their layout
+// (ms_convert.hip); transpose: with the transpose slots and P.symmetric
+void csr_to_device(SellPattern &P, int n, const int *row_ptr, const int *col_idx, const double *v, bool transpose,
+                   DBuf<double> &val);
 
 }  // namespace ms

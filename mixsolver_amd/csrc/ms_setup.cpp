@@ -239,19 +239,20 @@ void csr_to_sell(SellPattern &P, int n, const std::vector<int> &rp, const std::v
 
 void plan_sweeps(SellPattern &P, const std::vector<int> &rows_f, const std::vector<int> &rows_b);   // ms_levels.hip
 
-void SellPattern::build_levels() {
+template <class Col>
+void SellPattern::build_levels_from(Col col_of) {
   // forward: level(i) = 1 + max level of lower neighbours; backward on upper
   std::vector<int> lf(n, 0), lb(n, 0);
   int nlf = 0, nlb = 0;
   for (int r = 0; r < n; r++) {
     int l = 0;
-    for (int k = 0; k < diagk[r]; k++) l = std::max(l, lf[col[slot(r, k)]] + 1);
+    for (int k = 0; k < diagk[r]; k++) l = std::max(l, lf[col_of(r, k)] + 1);
     lf[r] = l;
     nlf = std::max(nlf, l + 1);
   }
   for (int r = n - 1; r >= 0; r--) {
     int l = 0;
-    for (int k = diagk[r] + 1; k < rowlen[r]; k++) l = std::max(l, lb[col[slot(r, k)]] + 1);
+    for (int k = diagk[r] + 1; k < rowlen[r]; k++) l = std::max(l, lb[col_of(r, k)] + 1);
     lb[r] = l;
     nlb = std::max(nlb, l + 1);
   }
@@ -289,6 +290,21 @@ void SellPattern::build_levels() {
   d_lev_ptr_b.upload(lev_ptr_b);
   plan_sweeps(*this, rf, rb);
   has_levels = true;
+}
+
+void SellPattern::build_levels() {
+  build_levels_from([&](int r, int k) { return col[slot(r, k)]; });
+}
+
+void SellPattern::build_levels(const int *row_ptr, const int *col_idx) {
+  rowlen.resize(n);
+  diagk.resize(n);
+  for (int r = 0; r < n; r++) {
+    const int *c = col_idx + row_ptr[r] - 1;
+    rowlen[r] = row_ptr[r + 1] - row_ptr[r];
+    diagk[r] = (int)(std::lower_bound(c, c + rowlen[r], r + 1) - c);
+  }
+  build_levels_from([&](int r, int k) { return col_idx[row_ptr[r] - 1 + k] - 1; });
 }
 
 void SellPattern::upload() {
