@@ -94,20 +94,6 @@ FieldRef lookup(System &s, const char *name) {
   fail(MS_EINVAL, "unknown field name: " + n);
 }
 
-void to_device_order(const System &s, const double *h, int w, std::vector<double> &out) {
-  out.resize((size_t)s.nc * w);
-  for (int i = 0; i < s.nc; i++)
-    for (int j = 0; j < w; j++) out[(size_t)s.o2n[i] * w + j] = h[(size_t)i * w + j];
-}
-void from_device_order(const System &s, const std::vector<double> &d, int w, double *h) {
-  for (int i = 0; i < s.nc; i++)
-    for (int j = 0; j < w; j++) h[(size_t)i * w + j] = d[(size_t)s.o2n[i] * w + j];
-}
-void download(const DBuf<double> &b, std::vector<double> &h, size_t n) {
-  h.resize(n);
-  b.download(h.data(), n);
-  MS_HIP(hipStreamSynchronize(stream()));
-}
 System &sys(ms_system *s) {
   if (!s || !s->s) fail(MS_EINVAL, "null system handle");
   return *s->s;
@@ -256,12 +242,10 @@ int ms_set_field(ms_system *h, const char *name, const double *host, long long n
       fail(MS_EINVAL, std::string(name) + ": zone properties cannot change while sweep cases share this system");
     if (f.kind == FACE) {
       if (n != s.nf) fail(MS_EINVAL, "face field size mismatch");
-      s.face_upload(*f.buf, std::vector<double>(host, host + n));
+      faces_in(s, host, *f.buf);
     } else {
       if (n != (long long)s.nc * f.width) fail(MS_EINVAL, "cell field size mismatch");
-      std::vector<double> d;
-      to_device_order(s, host, f.width, d);
-      if (f.buf) f.buf->upload(d);
+      if (f.buf) cells_in(s, host, f.width, *f.buf);
       if (f.kind == PROP) {
         f.host->assign(host, host + n);
         s.props_dirty = true;
@@ -295,21 +279,15 @@ int ms_get_field(ms_system *h, const char *name, double *host, long long n) {
     if (nm == "vol") return copy(s.vol_nat);
     if (nm == "xc") return copy(s.xc_nat);
     FieldRef f = lookup(s, name);
-    std::vector<double> d;
     if (f.kind == PROP) {
       if (n != (long long)s.nc * f.width) fail(MS_EINVAL, "cell field size mismatch");
       std::memcpy(host, f.host->data(), (size_t)n * sizeof(double));
     } else if (f.kind == FACE) {
       if (n != s.nf) fail(MS_EINVAL, "face field size mismatch");
-      download(*f.buf, d, s.nf);
-      for (int g = 0; g < s.nf; g++) host[g] = d[s.fo2d[g]];   // device face order -> face order
-      // a periodic shadow face carries its joined face's flux, oriented out of its own cell
-      for (int g = 0; g < s.nf; g++)
-        if (s.shadow[g] >= 0) host[g] = -host[s.shadow[g]];
+      faces_out(s, *f.buf, host);
     } else {
       if (n != (long long)s.nc * f.width) fail(MS_EINVAL, "cell field size mismatch");
-      download(*f.buf, d, (size_t)s.nc * f.width);
-      from_device_order(s, d, f.width, host);
+      cells_out(s, *f.buf, f.width, host);
     }
   });
 }
@@ -380,15 +358,11 @@ int ms_nan_scan(ms_system *h, int *field, int *cell, double *val, int *kind, int
   return guarded([&] {
     if (!field || !cell || !val || !kind || !ifin) fail(MS_EINVAL, "null output");
     System &s = sys(h);
-    std::vector<double> d, u(3 * (size_t)s.nc), p(s.nc), T(s.nc), Ts(s.nc);
-    download(s.u, d, 3 * (size_t)s.nc);
-    from_device_order(s, d, 3, u.data());
-    download(s.p, d, s.nc);
-    from_device_order(s, d, 1, p.data());
-    download(s.T, d, s.nc);
-    from_device_order(s, d, 1, T.data());
-    download(s.T_s, d, s.nc);
-    from_device_order(s, d, 1, Ts.data());
+    std::vector<double> u(3 * (size_t)s.nc), p(s.nc), T(s.nc), Ts(s.nc);
+    cells_out(s, s.u, 3, u.data());
+    cells_out(s, s.p, 1, p.data());
+    cells_out(s, s.T, 1, T.data());
+    cells_out(s, s.T_s, 1, Ts.data());
     *field = -1, *cell = 0, *val = 0.0, *kind = 0, *ifin = 0;
     for (int c = 0; c < s.nc && !*ifin; c++) {
       const double v[6] = {u[3 * (size_t)c], u[3 * (size_t)c + 1], u[3 * (size_t)c + 2], p[c], T[c], Ts[c]};
@@ -497,19 +471,9 @@ int ms_spmv_probe(int on, long long *launches, double *total_ms, long long *rows
 
 // ---- per-call level --------------------------------------------------------
 static void matrix_out(System &s, double *val, double *rhs, double *ap) {
-  std::vector<double> d;
-  if (val) {
-    download(s.val, d, s.pat.nstore);
-    for (size_t k = 0; k < s.ref2dev.size(); k++) val[k] = d[s.ref2dev[k]];
-  }
-  if (rhs) {
-    download(s.rhs, d, s.nc);
-    from_device_order(s, d, 1, rhs);
-  }
-  if (ap) {
-    download(s.ap, d, s.nc);
-    from_device_order(s, d, 1, ap);
-  }
+  if (val) matrix_values_out(s, val);
+  if (rhs) cells_out(s, s.rhs, 1, rhs);
+  if (ap) cells_out(s, s.ap, 1, ap);
 }
 
 int ms_compute_gradients(ms_system *h) { return guarded([&] { call_gradients(sys(h)); }); }
@@ -543,14 +507,9 @@ int ms_ppe_assembly(ms_system *h, double *val, double *rhs) {
 int ms_correct_fields(ms_system *h, const double *pp, double *dpp) {
   return guarded([&] {
     System &s = sys(h);
-    std::vector<double> d;
-    to_device_order(s, pp, 1, d);
-    s.pp.upload(d);
+    cells_in(s, pp, 1, s.pp);
     call_correct(s, s.pp.p);
-    if (dpp) {
-      download(s.dpp, d, 3 * (size_t)s.nc);
-      from_device_order(s, d, 3, dpp);
-    }
+    if (dpp) cells_out(s, s.dpp, 3, dpp);
   });
 }
 

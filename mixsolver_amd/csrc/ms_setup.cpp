@@ -1048,6 +1048,7 @@ System *create_system(int nnodes, const double *x, int nfaces, const long long *
     for (size_t k = 0; k < ent.size(); k++) ent[k] = 2 * s.fo2d[s.cf_ent[k] >> 1] + (s.cf_ent[k] & 1);
     s.d_cf_ent.upload(ent);
   }
+  if (s.renumbered) s.d_o2n.upload(s.o2n);
   s.d_cf_slot.upload(s.cf_slot);
   s.d_diag_slot.upload(s.diag_slot);
   s.face_upload(s.d_xf, s.xf, 3);
@@ -1582,6 +1583,7 @@ size_t System::device_bytes() const {
        d_iface_slip_C.bytes() + d_iface_peer_vel.bytes() + d_tval_s.bytes();
   b += d_c0.bytes() + d_c1.bytes() + d_fgrp.bytes() + d_pidx.bytes() + d_cf_ptr.bytes() + d_cf_ent.bytes() + d_cf_slot.bytes() +
        d_diag_slot.bytes();
+  b += d_o2n.bytes() + d_fo2d.bytes() + d_face_get.bytes() + d_ref2dev.bytes();
   b += d_e_oth.bytes() + d_e_lf.bytes() + d_e_sf.bytes() + d_e_Dm.bytes() + d_e_muf.bytes() + d_e_tcor.bytes();
   return b;
 }

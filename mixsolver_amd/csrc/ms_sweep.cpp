@@ -254,15 +254,9 @@ class Sweep {
 
   // final fields in the natural cell order
   void keep_fields(System &f, SweepCase &c) {
-    const int nc = f.nc;
-    std::vector<double> d;
     auto get = [&](const DBuf<double> &b, int w, std::vector<double> &out) {
-      d.resize((size_t)nc * w);
-      b.download(d.data(), d.size());
-      MS_HIP(hipStreamSynchronize(stream()));
-      out.resize(d.size());
-      for (int i = 0; i < nc; i++)
-        for (int j = 0; j < w; j++) out[(size_t)i * w + j] = d[(size_t)base_.o2n[i] * w + j];
+      out.resize((size_t)f.nc * w);
+      cells_out(f, b, w, out.data());
     };
     get(f.u, 3, c.u);
     get(f.p, 1, c.p);

@@ -153,6 +153,10 @@ struct System {
   // device mesh data
   DBuf<int> d_c0, d_c1, d_fgrp, d_cf_ptr, d_cf_ent;
   DBuf<long long> d_cf_slot, d_diag_slot;
+  // numbering maps of the API boundary (ms_io.hip): cells (renumbered systems),
+  // faces and matrix slots (uploaded on first use)
+  DBuf<int> d_o2n, d_fo2d, d_face_get;
+  DBuf<long long> d_ref2dev;
   DBuf<int> d_e_oth;
   DBuf<double> d_e_lf, d_e_sf, d_e_Dm, d_e_muf, d_e_tcor;
   // host face array (face order, width values per face) -> per cell-face entry
@@ -247,6 +251,14 @@ System *fork_system(System &base, const std::vector<ms_bcgroup_t> &groups);
 // errors as create_system.
 void periodic_match(int nnodes, const double *x, int nfaces, const long long *fptr, const int *fnodes,
                     const int *c0, const int *c1, const int *zone, int ncells, const ms_ctrl_t *ctrl, int *partner);
+
+// Arrays across the API boundary, natural order on the host and device order
+// on the device (ms_io.hip); they use af as staging and return synchronised.
+void cells_out(System &s, const DBuf<double> &buf, int w, double *h);
+void cells_in(System &s, const double *h, int w, DBuf<double> &buf);
+void faces_out(System &s, const DBuf<double> &buf, double *h);
+void faces_in(System &s, const double *h, DBuf<double> &buf);
+void matrix_values_out(System &s, double *h);
 
 // Wall-zone post-processing on the device fields (mod_uns_forces.f90):
 // out14 = Fx Fy Fz CD CL u_inf A_ref p_inf, pressure parts, viscous parts;
