@@ -154,7 +154,8 @@ struct Coarse {
   std::vector<int> agg_cptr, agg_cidx; // chunks of each aggregate (CSR)
   std::vector<int> e_ptr, e_key;      // E gather map: entry key a*k+b, slots [e_ptr[i], e_ptr[i+1])
   std::vector<int> e_slot;            // matrix slots, grouped by key, ascending
-  DBuf<int> d_chunk_ptr, d_chunk_agg, d_agg_cptr, d_agg_cidx, d_e_ptr, d_e_key, d_e_slot;
+  std::vector<int> chunk_pos;          // place of each chunk in agg_cidx
+  DBuf<int> d_chunk_pos, d_chunk_ptr, d_chunk_agg, d_agg_cptr, d_agg_cidx, d_e_ptr, d_e_key, d_e_slot;
   // (the matrix-dependent E, its inverse and the coarse solution belong to
   // each solver: CoarseMat)
   void upload();

@@ -177,15 +177,6 @@ struct FinResidual {
 // the coarse space is active (kept separate so the one-level path is
 // unchanged bit for bit).
 __device__ __forceinline__ double rz_total(const KS *st, double a) { return st->coarse ? a + st->cnu : a; }
-// r.z formed by k_pcg_p_split waits in st->rz_next (st->rzp = 1) until the
-// next finisher that reads st->rz takes it over.
-__device__ __forceinline__ void take_rz(KS *st) {
-  if (st->rzp) {
-    st->rz = st->rz_next;
-    st->rzp = 0;
-  }
-}
-
 struct FinNop {
   KS *st;
   __device__ bool skip() const { return st->done == 1; }
@@ -200,7 +191,6 @@ struct FinPap {
   KS *st;
   __device__ bool skip() const { return st->done != 0; }
   template <class T> __device__ void operator()(const T *a) const {
-    take_rz(st);
     st->it = st->it + 1;
     st->pap = a[0];
     if (fabs((double)a[0]) < kTiny) {
@@ -287,41 +277,10 @@ struct FinUpdateRU {
     }
   }
 };
-// FinUpdateRU for k_finish_split (Jacobi): the same residual checks; the
-// Jacobi part of r.z goes to st->rzd, and beta is formed by k_pcg_p_split
-// once the coarse parts c.nu are in.
-struct FinUpdateSplit {
-  KS *st;
-  int trigger;
-  __device__ bool skip() const { return st->done != 0; }
-  template <class T> __device__ void operator()(const T *a) const {
-    take_rz(st);   // the r.z this iteration's alpha used (k_pcg_update_fa)
-    const double rn = sqrt((double)a[0]);
-    st->res = rn * st->sigma / st->bnrm;
-    if (trigger) {
-      if (st->res <= st->tol) {
-        st->ru = 1;
-        st->done = 2;
-        return;
-      }
-      if (rn < st->delta * st->rmax) st->ru = 1;
-    }
-    if (rn > st->rmax) st->rmax = rn;
-    if (!trigger) st->ru = 0;
-    if (fabs(st->rz) < kTiny) {
-      st->ierr = 2;
-      st->done = 1;
-    } else {
-      st->rzd = (double)a[1];
-      st->pup = 1;   // the p update of this iteration is pending (k_pcg_p_split or the fused product)
-    }
-  }
-};
 struct FinRU {         // after x += sigma*y and r = b - A x in FP64
   KS *st;
   __device__ bool skip() const { return st->done == 1 || st->ru != 1; }
   template <class T> __device__ void operator()(const T *a) const {
-    take_rz(st);
     const double rt = sqrt((double)a[0]);
     st->rr = a[0];
     st->res = rt / st->bnrm;
@@ -340,70 +299,6 @@ struct FinRU {         // after x += sigma*y and r = b - A x in FP64
     st->done = 0;                          // resume the iteration
   }
 };
-// DILU iterations finish the update's r.r (first of the three chunk partials)
-// and the sweeps' r.z in one kernel after the sweeps: the convergence and
-// reliable-update checks of r.r move behind the preconditioner, which leaves
-// the iterates unchanged (one unneeded sweep on the last iteration).
-struct FinUpdRz {        // FP64 PCG: FinUpdate then FinRz
-  KS *st;
-  __device__ bool skip() const { return st->done != 0; }
-  template <class T> __device__ void operator()(const T *a1, const T *a2) const {
-    st->rr = a1[0];
-    st->res = sqrt((double)a1[0]) / st->bnrm;
-    if (st->res <= st->tol) {
-      st->done = 1;
-      return;
-    }
-    if (fabs(st->rz) < kTiny) {
-      st->ierr = 2;
-      st->done = 1;
-    } else {
-      const double rzn = rz_total(st, (double)a2[0]);
-      st->beta = rzn / st->rz;
-      st->rz = rzn;
-    }
-  }
-};
-struct FinUpdRzRU {      // mixed PCG: FinUpdateRU then FinRz
-  KS *st;
-  int trigger;
-  __device__ bool skip() const { return st->done != 0; }
-  template <class T> __device__ void operator()(const T *a1, const T *a2) const {
-    const double rn = sqrt((double)a1[0]);
-    st->res = rn * st->sigma / st->bnrm;
-    if (trigger) {
-      if (st->res <= st->tol) {
-        st->ru = 1;
-        st->done = 2;
-        return;
-      }
-      if (rn < st->delta * st->rmax) st->ru = 1;
-    }
-    if (rn > st->rmax) st->rmax = rn;
-    if (st->ru == 2) st->ru = 0;
-    if (fabs(st->rz) < kTiny) {
-      st->ierr = 2;
-      st->done = 1;
-    } else {
-      const double rzn = rz_total(st, (double)a2[0]);
-      st->beta = rzn / st->rz;
-      st->rz = rzn;
-    }
-  }
-};
-
-template <class T, class Fin>
-__global__ __launch_bounds__(kFinThreads) void k_finish2(int n1, const T *p1, int n2, const T *p2, Fin fin) {
-  if (fin.skip()) return;
-  T a1[3], a2[1];
-  fin_gather<OpSum, 3, T>(n1, p1, a1);
-  fin_gather<OpSum, 1, T>(n2, p2, a2);
-  __shared__ T l1[3 * (kFinThreads / 64)], l2[kFinThreads / 64];
-  block_reduce<OpSum, 3, T, kFinThreads>(a1, l1);
-  block_reduce<OpSum, 1, T, kFinThreads>(a2, l2);
-  if (threadIdx.x == 0) fin(a1, a2);
-}
-
 struct FinBiRho {
   KS *st;
   __device__ bool skip() const { return st->done != 0; }
@@ -525,15 +420,15 @@ __global__ void k_dilu_setup(int r0, int r1, Mat A, const long long *tpos, const
 
 // Coarse solve riding along a DILU forward-sweep launch: nwg extra
 // workgroups of kBlock threads, each recomputing c = Z^T r from the chunk
-// partials (third of three values per chunk) and four rows of nu = E^-1 c;
+// sums and four rows of nu = E^-1 c;
 // c.nu partials go to cnu_part[g], summed with the sweep's r.z partials.
 template <class T>
 struct CoWork {
   int k, nwg;
-  const int *agg_cptr, *agg_cidx;
+  const int *agg_cptr;
   const float *Einv;
   double *nu;
-  const T *cpart;
+  const T *csum;   // chunk sums of r, the chunks of an aggregate side by side
   T *cnu_part;
 };
 
@@ -548,11 +443,11 @@ __device__ void coarse_ride(const CoWork<T> &cw, int g) {
     for (; j + 7 < j1; j += 8) {       // eight independent far loads in flight, summed in index order
       T x[8];
 #pragma unroll
-      for (int u = 0; u < 8; u++) x[u] = cw.cpart[cw.agg_cidx[j + u] * 3 + 2];
+      for (int u = 0; u < 8; u++) x[u] = cw.csum[j + u];
 #pragma unroll
       for (int u = 0; u < 8; u++) s = s + (double)x[u];
     }
-    for (; j < j1; j++) s = s + (double)cw.cpart[cw.agg_cidx[j] * 3 + 2];
+    for (; j < j1; j++) s = s + (double)cw.csum[j];
     c[b] = s;
   }
   __syncthreads();
@@ -674,50 +569,7 @@ __global__ __launch_bounds__(kFinThreads) void k_finish_co(int nparts, const T *
   if (threadIdx.x == 0) fin(acc);
 }
 
-// Finisher of the mixed Jacobi PCG with a coarse space, spread over 1 + G
-// workgroups (G = ceil(k / kSplitRows)) so the coarse solve no longer runs
-// in one workgroup: workgroup 0 reduces the update's scalar partials and
-// runs the functor; workgroup g >= 1 recomputes c = Z^T r from the chunk
-// partials, forms rows [kSplitRows (g-1), kSplitRows g) of nu = E^-1 c (one
-// wavefront per row, E^-1 read along its rows) and writes the c.nu sum of
-// its rows to cnu_part[g-1].  k_pcg_p_split adds the parts (fixed order).
-constexpr int kSplitRows = kFinThreads / 64;
-constexpr int kSplitMaxParts = (kMaxAgg + kSplitRows - 1) / kSplitRows;   // coarse workgroups at most (64)
-template <int NV, class T, class Fin>
-__global__ __launch_bounds__(kFinThreads) void k_finish_split(int nparts, const T *partial, Fin fin, CoDev co,
-                                                              double *cnu_part) {
-  if (fin.skip()) return;
-  if (blockIdx.x == 0) {
-    T acc[NV];
-    fin_gather<OpSum, NV, T>(nparts, partial, acc);
-    __shared__ T lds[NV * (kFinThreads / 64)];
-    block_reduce<OpSum, NV, T, kFinThreads>(acc, lds);
-    if (threadIdx.x == 0) fin(acc);
-    return;
-  }
-  __shared__ double c[kMaxAgg], partq[kFinThreads], pr[kSplitRows];
-  coarse_c<NV, T>(partial, co, c, partq);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int a = (blockIdx.x - 1) * kSplitRows + w;
-  double prod = 0.0;
-  if (a < co.k) {
-    double s = 0.0;
-    for (int b = lane; b < co.k; b += 64) s = s + (double)co.Einv[(size_t)a * co.k + b] * c[b];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s = s + __shfl_down(s, o, 64);
-    if (lane == 0) {
-      co.nu[a] = s;
-      prod = s * c[a];
-    }
-  }
-  if (lane == 0) pr[w] = prod;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int j = 0; j < kSplitRows; j++) t = t + pr[j];
-    cnu_part[blockIdx.x - 1] = t;
-  }
-}
+constexpr int kSplitRows = kFinThreads / 64;   // rows of nu = E^-1 c per workgroup of k_cx_coarse
 
 __global__ void k_fill64(long long n, double *v, double x) {
   long long i = (long long)blockIdx.x * kBlock + threadIdx.x;

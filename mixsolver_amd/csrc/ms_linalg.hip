@@ -82,34 +82,11 @@ __global__ void k_pcg_spmv(int n, Mat A, const T *val, const T *p, T *q, const K
 // difference or a row-sum term, as in row_apply's difference form, so a
 // constant vector gives the row sums' product exactly.  The slot loop runs
 // the slice width of A (diagonal and padding slots have col = row).
-// The pending p update of the split PCG (p = r/d + nu[agg] + beta p, as
-// k_pcg_p_split) can ride along the product (PU): both stages compute beta
-// from the coarse finisher's parts in every workgroup, stage 1 forms the
+// The pending p update of the PCG with a coarse space (p = r/d + nu[agg] +
+// beta p, as k_cx_p) can ride along the product (PU): stage 1 forms the
 // updated p of each neighbour it reads, stage 2 that of its own row and
-// stores it (stage 1 has finished reading the old p by then).  The values
-// are those k_pcg_p_split would store, bit for bit.
-__device__ __forceinline__ float pu_beta(KS *st, const double *cnu, int G, bool writer) {
-  __shared__ double parts[kSplitMaxParts + 2];
-  __shared__ float beta_f;
-  const int t = threadIdx.x;
-  if (t < G) parts[t] = cnu[t];
-  else if (t == kSplitMaxParts) parts[t] = st->rzd;
-  else if (t == kSplitMaxParts + 1) parts[t] = st->rz;
-  __syncthreads();
-  if (t == 0) {
-    double rzn = parts[kSplitMaxParts];
-    for (int g = 0; g < G; g++) rzn = rzn + parts[g];
-    const double beta = rzn / parts[kSplitMaxParts + 1];
-    beta_f = (float)beta;
-    if (writer) {
-      st->rz_next = rzn;
-      st->rzp = 1;
-      st->beta = beta;
-    }
-  }
-  __syncthreads();
-  return beta_f;
-}
+// stores it (stage 1 has finished reading the old p by then).  The values are
+// those k_cx_p would store, bit for bit.
 template <bool PU>
 __device__ __forceinline__ float pu_val(int j, const float *p, const PUp &u, float beta, bool up) {
   if constexpr (PU) {
@@ -146,9 +123,9 @@ __global__ void k_mf_stage1(int n0, Mat A, const float *w, const float *x, float
   if (st->done) return;
   float beta = 0.f;
   bool up = false;
-  if constexpr (PU) {
-    up = st->pup != 0;   // the same for every workgroup: pup changes only in k_pcg_update_fa
-    if (up) beta = pu_beta(st, u.cnu, u.G, false);
+  if constexpr (PU) {   // the same for every workgroup: both change between products only
+    up = st->pup != 0;
+    beta = (float)st->beta;
   }
   const int k = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (k >= n0) return;
@@ -200,7 +177,7 @@ __global__ void k_mf_stage2(int n0, int n1, Mat A, const float *w, float *x, con
   bool up = false;
   if constexpr (PU) {
     up = st->pup != 0;
-    if (up) beta = pu_beta(st, u.cnu, u.G, blockIdx.x == 0);
+    beta = (float)st->beta;
   }
   const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   float v[1] = {0.f};
@@ -274,101 +251,6 @@ __global__ void k_pcg_p(Rows R, const T *r, const T *z, const T *dg, int jac, T 
   }
 }
 
-// k_pcg_update (Jacobi) with the alpha finisher folded in, for the mixed
-// Jacobi PCG with a coarse space: every workgroup reduces the SpMV's p.q
-// partials itself, in the same fixed order, so all hold the same pap and
-// alpha (r.z is the value the last p update left pending, when it left one);
-// workgroup 0 keeps the solver state as FinPap does (iteration count, pap,
-// alpha, the breakdown test).  One launch and one kernel boundary less per
-// iteration.
-template <class T>
-__global__ void k_pcg_update_fa(Rows R, int np, const T *ppart, const T *p, const T *q, T *y, T *r, const T *dg,
-                                KS *st, T *part) {
-  if (st->done) return;
-  __shared__ T lds[kBlock / 64];
-  __shared__ double alpha_s;
-  __shared__ int bad_s;
-  T acc[1] = {T(0)};
-  int b = threadIdx.x;
-  for (; b + 3 * kBlock < np; b += 4 * kBlock) {   // four loads in flight, summed in index order
-    const T x0 = ppart[b], x1 = ppart[b + kBlock], x2 = ppart[b + 2 * kBlock], x3 = ppart[b + 3 * kBlock];
-    acc[0] = acc[0] + x0;
-    acc[0] = acc[0] + x1;
-    acc[0] = acc[0] + x2;
-    acc[0] = acc[0] + x3;
-  }
-  for (; b < np; b += kBlock) acc[0] = acc[0] + ppart[b];
-  block_reduce<OpSum, 1, T, kBlock>(acc, lds);
-  if (threadIdx.x == 0) {
-    const double pap = (double)acc[0];
-    const double rz = st->rzp ? st->rz_next : st->rz;
-    const int bad = fabs(pap) < kTiny;
-    bad_s = bad;
-    alpha_s = bad ? 0.0 : rz / pap;
-    if (blockIdx.x == 0) {
-      st->it = st->it + 1;
-      st->pap = pap;
-      st->pup = 0;   // the product before this kernel applied any pending p update
-      if (bad) {
-        st->ierr = 2;
-        st->done = 1;
-      } else {
-        st->alpha = alpha_s;
-      }
-    }
-  }
-  __syncthreads();
-  if (bad_s) return;
-  int i, a;
-  T v[3] = {T(0), T(0), T(0)};
-  if (R.get(i, a)) {
-    const T alpha = (T)alpha_s;
-    const T pi = p[i], qi = q[i], r0 = r[i], yi = y[i], di = dg[i];
-    y[i] = yi + alpha * pi;
-    const T ri = r0 - alpha * qi;
-    r[i] = ri;
-    v[0] = ri * ri;
-    v[1] = ri * (ri / di);
-    v[2] = ri;
-  }
-  block_partials<OpSum, 3>(v, part);
-}
-
-// p = r/d + nu_agg + beta p after k_finish_split: every workgroup forms
-// r.z = rzd + the coarse parts (fixed order) and beta = r.z / rz; workgroup 0
-// leaves r.z in st->rz_next for the next finisher.
-template <class T>
-__global__ void k_pcg_p_split(Rows R, const T *r, const T *dg, T *p, const double *nu, KS *st,
-                              const double *cnu_part, int G, int flush = 0) {
-  if (st->done) return;
-  if (flush && !st->pup) return;   // flush: apply a pending update only
-  // the parts, rzd and rz are loaded by different threads at once (one load
-  // latency), then added by thread 0 in part order
-  __shared__ double parts[kSplitMaxParts + 2], beta_s;
-  const int t = threadIdx.x;
-  if (t < G) parts[t] = cnu_part[t];
-  else if (t == kSplitMaxParts) parts[t] = st->rzd;
-  else if (t == kSplitMaxParts + 1) parts[t] = st->rz;
-  __syncthreads();
-  if (t == 0) {
-    double rzn = parts[kSplitMaxParts];
-    for (int g = 0; g < G; g++) rzn = rzn + parts[g];
-    const double beta = rzn / parts[kSplitMaxParts + 1];
-    beta_s = beta;
-    if (blockIdx.x == 0) {
-      st->rz_next = rzn;
-      st->rzp = 1;
-      st->beta = beta;
-    }
-  }
-  __syncthreads();
-  int i, a;
-  if (R.get(i, a)) {
-    const T zi = r[i] / dg[i] + (T)nu[a];
-    p[i] = zi + (T)beta_s * p[i];
-  }
-}
-
 // ------------------------------------------------------- two-launch PCG
 // PCG without a coarse space.  An iteration is the launch-bound end of a
 // solve: at 16,000 rows its five kernels (product, alpha, update, beta, p)
@@ -433,8 +315,8 @@ struct CgParts {   // r.r and r.z partials of the last update / preconditioner
 // 2 breakdown.  writer: keep the solver state.
 // mixed: the FP32 iteration on r / sigma, as FinUpdateRU.
 template <class T, bool MIXED>
-__device__ __forceinline__ int cg_test(KS *st, int first, T rr, T rz, int par, bool writer, double &beta) {
-  const double rzn = (double)rz, old = st->rz2[par ^ 1];
+__device__ __forceinline__ int cg_test(KS *st, int first, T rr, double rzn, int par, bool writer, double &beta) {
+  const double old = st->rz2[par ^ 1];
   beta = 0.0;
   if (!first) {
     if constexpr (MIXED) {
@@ -510,7 +392,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_ps(int n, Mat A, const T *val, co
   cg_sums<T>(np.nrr, rrp, np.nrz, rzp, sums);
   if (threadIdx.x == 0) {
     double beta;
-    stop_s = cg_test<T, MIXED>(st, first, sums[0], sums[1], par, blockIdx.x == 0, beta);
+    stop_s = cg_test<T, MIXED>(st, first, sums[0], (double)sums[1], par, blockIdx.x == 0, beta);
     beta_s = beta;
     if (blockIdx.x == 0 && !stop_s) {
       st->beta = beta;
@@ -667,6 +549,290 @@ __global__ __launch_bounds__(kBlock) void k_cg_rescale(int n, const double *r64,
   if (threadIdx.x == 0) {
     rrp[blockIdx.x] = v[0];
     if (mode == 1) rzp[blockIdx.x] = v[1];
+  }
+}
+
+// -------------------------------------------------- PCG with a coarse space
+// The same idea where the coarse solve needs Z^T r of the whole update before
+// p can be formed, so p keeps a launch of its own:
+//   product with p.q partials
+//   k_cx_update: [p.q -> alpha]  x, r; r.r, (Jacobi) r.z, chunk sums of r,
+//                (DILU) z on the first colour
+//   Jacobi: k_cx_coarse, nu = E^-1 Z^T r;  DILU: the sweeps, the first of
+//                which carries the coarse solve
+//   k_cx_p:      [r.r, r.z + c.nu -> stop?, beta]  p = z + nu + beta p
+// A wavefront takes a chunk (at most 256 rows of one aggregate, four per
+// lane): its loads are all in flight at once and issued before the partials
+// are waited for, its chunk sum needs shuffles only, and four chunks share
+// the reduction of the partials, which every workgroup repeats.  With one
+// workgroup per chunk (3,907 at 1M rows) those repeats read 61 MB through the
+// L2s, twice the data of the update itself.
+// Per iteration of the reduced p' solve at 2M cells, in us: update 11.9 ->
+// @U@, coarse solve 8.0 -> @C@, p update 6.0 -> @P@.
+constexpr int kCxGrid = 1024;
+constexpr int kCxRows = kBlock / kSlice;   // rows per lane
+
+struct Chunks {
+  const int *ptr, *agg, *pos;
+  int n;
+};
+__device__ __forceinline__ RowRange cx_range(const Chunks &C) {
+  const int G = gridDim.x, b = xcd_block(blockIdx.x, G);
+  return RowRange{(int)((long long)b * C.n / G), (int)((long long)(b + 1) * C.n / G)};
+}
+
+// sum over the wavefront, on every lane, in a fixed order
+template <class T>
+__device__ __forceinline__ T wave_sum(T v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
+  return v;
+}
+
+template <class T, class X>
+__global__ __launch_bounds__(kBlock) void k_cx_update(Chunks C, int npq, const T *pqp, const T *p, const T *q, X *x,
+                                                      T *r, T *z, const T *dg, int mode, int c0end, KS *st, T *rrp,
+                                                      T *rzp, T *csum) {
+  const int done = st->done;
+  const RowRange R = cx_range(C);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int ch = R.b0 + wv, r0 = 0, r1 = 0, pos = 0;
+  T pi[kCxRows], qi[kCxRows], ri[kCxRows], di[kCxRows];
+  X xi[kCxRows];
+  auto load = [&]() {
+    r0 = C.ptr[ch] + lane;
+    r1 = C.ptr[ch + 1];
+    pos = C.pos[ch];
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = min(r0 + u * kSlice, r1 - 1);   // lanes beyond the chunk repeat its last row
+      pi[u] = p[i];
+      qi[u] = q[i];
+      ri[u] = r[i];
+      xi[u] = x[i];
+      di[u] = dg[i];
+    }
+  };
+  if (ch < R.b1) load();
+  if (done) return;
+  __shared__ double alpha_s;
+  __shared__ int bad_s;
+  T sums[2];
+  cg_sums<T>(npq, pqp, 0, pqp, sums);
+  if (threadIdx.x == 0) {
+    const double pap = (double)sums[0];
+    const int bad = fabs(pap) < kTiny;
+    bad_s = bad;
+    alpha_s = bad ? 0.0 : st->rz2[st->par] / pap;
+    if (blockIdx.x == 0) {
+      st->it = st->it + 1;
+      st->pap = pap;
+      st->trig = 0;
+      st->pup = 0;   // the product before this launch applied a pending p update
+      if (bad) {
+        st->ierr = 2;
+        st->done = 1;
+      } else {
+        st->alpha = alpha_s;
+      }
+    }
+  }
+  __syncthreads();
+  if (bad_s) return;
+  const T alpha = (T)alpha_s;
+  T v[2] = {T(0), T(0)};
+  for (; ch < R.b1; ch += kBlock / kSlice) {
+    if (ch >= R.b0 + kBlock / kSlice) load();
+    T cs = T(0);
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = r0 + u * kSlice;
+      if (i < r1) {
+        x[i] = xi[u] + (X)(alpha * pi[u]);
+        const T rn = ri[u] - alpha * qi[u];
+        r[i] = rn;
+        v[0] = v[0] + rn * rn;
+        cs = cs + rn;
+        if (mode == 1) v[1] = v[1] + rn * (rn / di[u]);
+        else if (i < c0end) z[i] = rn / di[u];
+      }
+    }
+    cs = wave_sum(cs);
+    if (lane == 0) csum[pos] = cs;
+  }
+  __shared__ T lds[2 * (kBlock / 64)];
+  block_reduce<OpSum, 2, T>(v, lds);
+  if (threadIdx.x == 0) {
+    rrp[blockIdx.x] = v[0];
+    if (mode == 1) rzp[blockIdx.x] = v[1];
+  }
+}
+
+// The sums of an r that no update made: the initial residual (r64 null), or
+// after a reliable update r = r64 / sigma with p moved to the new scale.
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_cx_start(Chunks C, const double *r64, T *r, T *p, T *z, const T *dg,
+                                                     int mode, int c0end, const KS *st, T *rrp, T *rzp, T *csum) {
+  if (st->done || (r64 && st->ru != 2)) return;
+  const RowRange R = cx_range(C);
+  const int lane = threadIdx.x & 63;
+  T v[2] = {T(0), T(0)};
+  for (int ch = R.b0 + (threadIdx.x >> 6); ch < R.b1; ch += kBlock / kSlice) {
+    const int r1 = C.ptr[ch + 1];
+    T cs = T(0);
+    for (int i = C.ptr[ch] + lane; i < r1; i += kSlice) {
+      T ri;
+      if (r64) {
+        ri = (T)(r64[i] / st->sigma);
+        r[i] = ri;
+        p[i] = p[i] * (T)st->scale;
+      } else {
+        ri = r[i];
+      }
+      v[0] = v[0] + ri * ri;
+      cs = cs + ri;
+      if (mode == 1) v[1] = v[1] + ri * (ri / dg[i]);
+      else if (i < c0end) z[i] = ri / dg[i];
+    }
+    cs = wave_sum(cs);
+    if (lane == 0) csum[C.pos[ch]] = cs;
+  }
+  __shared__ T lds[2 * (kBlock / 64)];
+  block_reduce<OpSum, 2, T>(v, lds);
+  if (threadIdx.x == 0) {
+    rrp[blockIdx.x] = v[0];
+    if (mode == 1) rzp[blockIdx.x] = v[1];
+  }
+}
+
+// nu = E^-1 c, c = Z^T r from the chunk sums: workgroup g recomputes c and
+// forms rows [kSplitRows g, kSplitRows (g + 1)) of nu, a wavefront per row,
+// and the c.nu sum of its rows.  It is a chain of far loads in few
+// workgroups: E^-1, which no load waits for, is fetched first, and an
+// aggregate's chunk sums lie side by side.
+constexpr int kCoPre = 4;   // 64-column pieces of an E^-1 row fetched ahead (k <= 256)
+template <class T>
+__global__ __launch_bounds__(kFinThreads) void k_cx_coarse(int k, const int *cptr, const float *Einv, const T *csum,
+                                                           double *nu, double *cnu_part, const KS *st) {
+  const int done = st->done;
+  __shared__ double c[kMaxAgg], partq[kFinThreads], pr[kSplitRows];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, a = blockIdx.x * kSplitRows + w;
+  float e[kCoPre];
+#pragma unroll
+  for (int j = 0; j < kCoPre; j++) {
+    const int b = lane + 64 * j;
+    e[j] = a < k && b < k ? Einv[(size_t)a * k + b] : 0.0f;
+  }
+  // Q threads per aggregate, each every Q-th of its chunks
+  const int Q = k <= kFinThreads / 4 ? 4 : (k <= kFinThreads / 2 ? 2 : 1), span = kFinThreads / Q;
+  const int g = threadIdx.x % span, qq = threadIdx.x / span;
+  if (g < k) {
+    double s = 0.0;
+    int j = cptr[g] + qq;
+    const int je = cptr[g + 1];
+    for (; j + 3 * Q < je; j += 4 * Q) {
+      const T v0 = csum[j], v1 = csum[j + Q], v2 = csum[j + 2 * Q], v3 = csum[j + 3 * Q];
+      s = s + (double)v0;
+      s = s + (double)v1;
+      s = s + (double)v2;
+      s = s + (double)v3;
+    }
+    for (; j < je; j += Q) s = s + (double)csum[j];
+    partq[qq * span + g] = s;
+  }
+  if (done) return;
+  __syncthreads();
+  if (qq == 0 && g < k) {
+    double s = partq[g];
+    for (int i = 1; i < Q; i++) s = s + partq[i * span + g];
+    c[g] = s;
+  }
+  __syncthreads();
+  double prod = 0.0;
+  if (a < k) {
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < kCoPre; j++) {
+      const int b = lane + 64 * j;
+      if (b < k) s = s + (double)e[j] * c[b];
+    }
+    for (int b = lane + 64 * kCoPre; b < k; b += 64) s = s + (double)Einv[(size_t)a * k + b] * c[b];
+    s = wave_sum(s);
+    if (lane == 0) {
+      nu[a] = s;
+      prod = s * c[a];
+    }
+  }
+  if (lane == 0) pr[w] = prod;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int j = 0; j < kSplitRows; j++) t = t + pr[j];
+    cnu_part[blockIdx.x] = t;
+  }
+}
+
+// p = z + nu + beta p (z = r/d with Jacobi); ncn coarse parts of r.z.
+// what: kCxAll; kCxTest (one workgroup, C.n = 0): the test and beta only, and
+// the update is left pending for the product; kCxPending: a pending update
+// only.
+enum { kCxAll = 0, kCxTest = 1, kCxPending = 2 };
+template <class T, bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_cx_p(Chunks C, const T *r, const T *z, const T *dg, int mode, T *p,
+                                                 const double *nu, KS *st, CgParts np, const T *rrp, const T *rzp,
+                                                 int ncn, const double *cnu_part, int what) {
+  const int done = st->done;
+  if (what == kCxPending && !st->pup) return;
+  const RowRange R = cx_range(C);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int ch = R.b0 + wv, r0 = 0, r1 = 0;
+  T zi[kCxRows], di[kCxRows], pi[kCxRows], nua = T(0);
+  auto load = [&]() {
+    r0 = C.ptr[ch] + lane;
+    r1 = C.ptr[ch + 1];
+    nua = (T)nu[C.agg[ch]];
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = min(r0 + u * kSlice, r1 - 1);
+      zi[u] = mode == 1 ? r[i] : z[i];
+      di[u] = mode == 1 ? dg[i] : T(1);
+      pi[u] = p[i];
+    }
+  };
+  if (ch < R.b1) load();
+  double cn = wv == 0 && lane < ncn ? cnu_part[lane] : 0.0;
+  if (done) return;
+  const int first = st->it == 0, par = st->it & 1;
+  T sums[2];
+  cg_sums<T>(np.nrr, rrp, np.nrz, rzp, sums);
+  cn = wave_sum(cn);
+  __shared__ double beta_s;
+  __shared__ int stop_s;
+  if (threadIdx.x == 0) {
+    const double rzn = (double)sums[1] + cn;
+    double beta = st->beta;
+    stop_s = what == kCxPending ? 0 : cg_test<T, MIXED>(st, first, sums[0], rzn, par, blockIdx.x == 0, beta);
+    beta_s = beta;
+    if (what != kCxPending && blockIdx.x == 0 && !stop_s) {
+      st->beta = beta;
+      st->rz2[par] = rzn;
+      st->par = par;
+      st->pup = what == kCxTest;
+    }
+  }
+  __syncthreads();
+  if (stop_s) return;
+  const T beta = (T)beta_s;
+  for (; ch < R.b1; ch += kBlock / kSlice) {
+    if (ch >= R.b0 + kBlock / kSlice) load();
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = r0 + u * kSlice;
+      if (i < r1) {
+        const T zn = (mode == 1 ? zi[u] / di[u] : zi[u]) + nua;
+        p[i] = first ? zn : zn + beta * pi[u];
+      }
+    }
   }
 }
 
@@ -1353,17 +1519,16 @@ static CoDev codev_of(const SellPattern *pat, const CoarseMat &cm, bool coarse, 
   return CoDev{C.k, C.d_agg_cptr.p, C.d_agg_cidx.p, cm.Einv.p, cm.nu.p, st};
 }
 template <class T>
-static CoWork<T> cowork_of(const SellPattern *pat, const CoarseMat &cm, bool fused, const T *cpart) {
+static CoWork<T> cowork_of(const SellPattern *pat, const CoarseMat &cm, bool fused, const T *csum) {
   CoWork<T> cw{};
   if (!fused) return cw;
   const Coarse &C = pat->coarse;
   cw.k = C.k;
   cw.nwg = (C.k + kBlock / 64 - 1) / (kBlock / 64);
   cw.agg_cptr = C.d_agg_cptr.p;
-  cw.agg_cidx = C.d_agg_cidx.p;
   cw.Einv = cm.Einv.p;
   cw.nu = cm.nu.p;
-  cw.cpart = cpart;
+  cw.csum = csum;
   return cw;
 }
 
@@ -1452,6 +1617,90 @@ Krylov::Cg2<T> Krylov::cg2(PcKind pc) {
   return c;
 }
 
+// buffers of the PCG with a coarse space (Jacobi, or DILU with the coarse
+// solve riding along the sweeps)
+template <class T>
+Krylov::Cx<T> Krylov::cx(PcKind pc) {
+  const Coarse &C = pat->coarse;
+  Cx<T> c;
+  c.mode = pc == PC_JACOBI ? 1 : 2;
+  c.G = std::min((C.nchunks + kBlock / kSlice - 1) / (kBlock / kSlice), kCxGrid);
+  const size_t stride = (size_t)std::max(nblk_, C.nchunks) + 64;
+  T *part, *sweep;
+  if constexpr (sizeof(T) == 8) {
+    c.r = r_.p, c.z = z_.p, c.p = p_.p, c.q = q_.p, c.dg = dg_.p;
+    part = part_.p;
+    sweep = prz_.p;
+  } else {
+    c.r = r32_.p, c.z = z32_.p, c.p = p32_.p, c.q = q32_.p, c.dg = dg32_.p;
+    part = part32_.p;
+    sweep = prz32_.p;
+  }
+  c.rr = part;
+  c.rz = part + stride;
+  c.csum = part + 2 * stride;
+  c.pq = part + 3 * stride;
+  c.nrz = c.G;
+  if (c.mode == 1) {
+    c.ncn = (C.k + kSplitRows - 1) / kSplitRows;
+    if (cnu_split_.n < (size_t)c.ncn) cnu_split_.alloc(c.ncn);
+  } else {
+    c.rz = sweep;
+    c.cw = (C.k + kBlock / 64 - 1) / (kBlock / 64);
+    c.nrz = c.cw;
+    const auto &cp = pat->color_ptr;
+    const int nc = (int)cp.size() - 1;
+    for (int k = 1; k < nc; k++) c.nrz += nblocks(cp[k + 1] - cp[k]);
+    for (int k = nc - 2; k >= 0; k--) c.nrz += nblocks(cp[k + 1] - cp[k]);
+  }
+  return c;
+}
+
+static Chunks chunks_of(const SellPattern *pat) {
+  const Coarse &C = pat->coarse;
+  return Chunks{C.d_chunk_ptr.p, C.d_chunk_agg.p, C.d_chunk_pos.p, C.nchunks};
+}
+
+// the preconditioner of the current r, and p
+template <class T, bool MIXED>
+void Krylov::cx_p(const Cx<T> &c, int what) {
+  Chunks C = chunks_of(pat);
+  if (what == kCxTest) C.n = 0;
+  hipLaunchKernelGGL((k_cx_p<T, MIXED>), dim3(what == kCxTest ? 1 : c.G), dim3(kBlock), 0, stream(), C, c.r, c.z, c.dg,
+                     c.mode, c.p, cm_.nu.p, st_.p, CgParts{c.G, c.nrz}, c.rr, c.rz, c.ncn, cnu_split_.p, what);
+}
+
+template <class T, bool MIXED>
+void Krylov::cx_direction(const Cx<T> &c, const T *val, int what) {
+  const Coarse &C = pat->coarse;
+  hipStream_t S = stream();
+  if (c.mode == 1) {
+    hipLaunchKernelGGL(k_cx_coarse<T>, dim3(c.ncn), dim3(kFinThreads), 0, S, C.k, C.d_agg_cptr.p, cm_.Einv.p, c.csum,
+                       cm_.nu.p, cnu_split_.p, st_.p);
+  } else {
+    dilu_sweeps<T>(pat, matof(pat), val, c.dg, c.r, c.z, &st_.p->done, c.rz, cowork_of<T>(pat, cm_, true, c.csum));
+  }
+  cx_p<T, MIXED>(c, what);
+}
+
+// sums and direction of a new r: the initial one (r64 null), or the one of a
+// reliable update; direction = false: p is already that of the next iteration
+template <class T, bool MIXED>
+void Krylov::cx_restart(const Cx<T> &c, const T *val, const double *r64, bool direction) {
+  hipLaunchKernelGGL(k_cx_start<T>, dim3(c.G), dim3(kBlock), 0, stream(), chunks_of(pat), r64, c.r, c.p, c.z, c.dg,
+                     c.mode, pat->color_ptr[1], st_.p, c.rr, c.rz, c.csum);
+  if (direction) cx_direction<T, MIXED>(c, val, kCxAll);
+  MS_CHECK_LAUNCH();
+}
+
+// the part of an iteration after the product
+template <class T, bool MIXED, class X>
+void Krylov::cx_update(const Cx<T> &c, const T *val, X *x, bool ride) {
+  hipLaunchKernelGGL((k_cx_update<T, X>), dim3(c.G), dim3(kBlock), 0, stream(), chunks_of(pat), nblk_, c.pq, c.p, c.q,
+                     x, c.r, c.z, c.dg, c.mode, pat->color_ptr[1], st_.p, c.rr, c.rz, c.csum);
+  cx_direction<T, MIXED>(c, val, ride ? kCxTest : kCxAll);
+}
+
 // z and the r.z partials of the current r
 template <class T>
 void Krylov::cg2_precond(const Cg2<T> &c, const T *val, const T *fac) {
@@ -1504,7 +1753,7 @@ SolveResult Krylov::pcg(const double *val, const double *b, double *x, double to
   KS h{};
   h.tol = tol;
   h.maxit = maxit;
-  h.coarse = coarse && !fused;
+  h.coarse = coarse && !fused && pc != PC_JACOBI;
   MS_HIP(hipMemcpyAsync(st, &h, sizeof(h), hipMemcpyHostToDevice, S));
   hipLaunchKernelGGL(k_sumsq<double>, G, B, 0, S, n, b, part);
   finish<OpSum, 1>(nblk_, part, FinBnorm{st});
@@ -1555,58 +1804,53 @@ SolveResult Krylov::pcg(const double *val, const double *b, double *x, double to
     }
     return R;
   }
-  const Rows RW = rows_of(pat, coarse);
-  const dim3 GR(coarse ? pat->coarse.nchunks : nblk_);
-  const CoDev co = codev_of(pat, cm_, coarse, st);
-  const double *nu = coarse ? cm_.nu.p : nullptr;
-  const CoWork<double> cw = cowork_of<double>(pat, cm_, fused, part);
-  double *prz = prz_.p;
-  if (fused) {
-    hipLaunchKernelGGL(k_rsum<double>, GR, B, 0, S, RW, r_.p, st, part);
-    const auto &cp = pat->color_ptr;
-    hipLaunchKernelGGL(k_dilu_first<double>, dim3(nblocks(cp[1] - cp[0])), B, 0, S, cp[0], cp[1], dg_.p, r_.p, z_.p,
-                       done);
-    const int np = dilu_sweeps<double>(pat, A, val, dg_.p, r_.p, z_.p, done, prz, cw);
-    finish<OpSum, 1>(np, prz, FinRz0{st});
-    MS_HIP(hipMemsetAsync(p_.p, 0, n * sizeof(double), S));
-    hipLaunchKernelGGL(k_pcg_p<double>, GR, B, 0, S, RW, r_.p, z_.p, dg_.p, 0, p_.p, nu, st);   // beta = 0
-  } else {
-    if (coarse) {
-      hipLaunchKernelGGL(k_rsum<double>, GR, B, 0, S, RW, r_.p, st, part);
-      finish_co<3>((int)GR.x, part, FinNop{st}, co);
+  if (jac || fused) {
+    const Cx<double> c = cx<double>(pc);
+    cx_restart<double, false>(c, val, nullptr, true);
+    for (int enq = 0, chunk = 8;;) {
+      const int m = std::min(chunk, maxit - enq);
+      for (int it = 0; it < m; it++) {
+        hipLaunchKernelGGL((k_pcg_spmv<double, 0>), G, B, 0, S, n, A, val, c.p, c.q, st, c.pq);
+        cx_update<double, false>(c, val, x, false);
+      }
+      MS_CHECK_LAUNCH();
+      enq += m;
+      hs = read_state<double>(st);
+      if (hs.done || enq >= maxit) break;
+      chunk = std::min(chunk * 2, 128);
     }
-    if (!jac) apply_pc<double>(pc, val, fac_.p, dg_.p, r_.p, z_.p, done);
-    hipLaunchKernelGGL(k_pcg_start<double>, GR, B, 0, S, RW, r_.p, z_.p, dg_.p, jac, p_.p, nu, st, part);
-    finish<OpSum, 1>((int)GR.x, part, FinRz0{st});
+    R.it = hs.it;
+    R.res = hs.res;
+    R.ierr = hs.ierr;
+    if (!hs.done) {
+      R.it = maxit + 1;
+      R.ierr = 1;
+    }
+    return R;
   }
-  const int mode = jac ? 1 : (pc == PC_DILU ? 2 : 0);
-  const int c0end = pat->color_ptr[1];
-  const CoDev co_upd = fused ? CoDev{0, nullptr, nullptr, nullptr, nullptr, st} : co;
-  const bool merged = mode == 2 && (!coarse || fused);
+  // a coarse space beside a level-scheduled factorization
+  const Rows RW = rows_of(pat, true);
+  const dim3 GR(pat->coarse.nchunks);
+  const CoDev co = codev_of(pat, cm_, true, st);
+  const double *nu = cm_.nu.p;
+  hipLaunchKernelGGL(k_rsum<double>, GR, B, 0, S, RW, r_.p, st, part);
+  finish_co<3>((int)GR.x, part, FinNop{st}, co);
+  apply_pc<double>(pc, val, fac_.p, dg_.p, r_.p, z_.p, done);
+  hipLaunchKernelGGL(k_pcg_start<double>, GR, B, 0, S, RW, r_.p, z_.p, dg_.p, 0, p_.p, nu, st, part);
+  finish<OpSum, 1>((int)GR.x, part, FinRz0{st});
   int enq = 0, chunk = 8;
   while (true) {
     int m = std::min(chunk, maxit - enq);
     for (int it = 0; it < m; it++) {
       hipLaunchKernelGGL(k_pcg_spmv<double>, G, B, 0, S, n, A, val, p_.p, q_.p, st, part);
       finish<OpSum, 1>(nblk_, part, FinPap{st});
-      hipLaunchKernelGGL((k_pcg_update<double, double>), GR, B, 0, S, RW, p_.p, q_.p, x, r_.p, z_.p, dg_.p, mode,
-                         c0end, st, part);
-      if (merged) {      // convergence check and r.z in one finisher after the sweeps
-        const int np = dilu_sweeps<double>(pat, A, val, dg_.p, r_.p, z_.p, done, prz, cw);
-        hipLaunchKernelGGL((k_finish2<double, FinUpdRz>), dim3(1), dim3(kFinThreads), 0, S, (int)GR.x, part, np, prz,
-                           FinUpdRz{st});
-      } else {
-        finish_co<3>((int)GR.x, part, FinUpdate{st, jac}, co_upd);
-      }
-      if (mode == 2 && !merged) {
-        int np = dilu_sweeps<double>(pat, A, val, dg_.p, r_.p, z_.p, done, prz, cw);
-        finish<OpSum, 1>(np, prz, FinRz{st});
-      } else if (mode == 0) {
-        apply_pc<double>(pc, val, fac_.p, dg_.p, r_.p, z_.p, done);
-        hipLaunchKernelGGL(k_dot<double>, G, B, 0, S, n, r_.p, z_.p, st, part);
-        finish<OpSum, 1>(nblk_, part, FinRz{st});
-      }
-      hipLaunchKernelGGL(k_pcg_p<double>, GR, B, 0, S, RW, r_.p, z_.p, dg_.p, jac, p_.p, nu, st);
+      hipLaunchKernelGGL((k_pcg_update<double, double>), GR, B, 0, S, RW, p_.p, q_.p, x, r_.p, z_.p, dg_.p, 0, 0, st,
+                         part);
+      finish_co<3>((int)GR.x, part, FinUpdate{st, 0}, co);
+      apply_pc<double>(pc, val, fac_.p, dg_.p, r_.p, z_.p, done);
+      hipLaunchKernelGGL(k_dot<double>, G, B, 0, S, n, r_.p, z_.p, st, part);
+      finish<OpSum, 1>(nblk_, part, FinRz{st});
+      hipLaunchKernelGGL(k_pcg_p<double>, GR, B, 0, S, RW, r_.p, z_.p, dg_.p, 0, p_.p, nu, st);
     }
     MS_CHECK_LAUNCH();
     enq += m;
@@ -1961,7 +2205,6 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
   const dim3 GR(coarse ? pat->coarse.nchunks : nblk_);
   const CoDev co = codev_of(pat, cm_, coarse && !fused, st);
   const double *nu = coarse ? cm_.nu.p : nullptr;
-  const CoWork<float> cw = cowork_of<float>(pat, cm_, fused, part32);
   float *prz = prz32_.p;
   MS_HIP(hipMemsetAsync(y, 0, n * sizeof(float), S));
   hipLaunchKernelGGL(k_set_sigma, dim3(1), dim3(64), 0, S, st);
@@ -1970,16 +2213,16 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
   // has launches of its own)
   const bool two = !coarse && !matfree_on();
   const Cg2<float> cg = two ? cg2<float>(pc) : Cg2<float>{};
+  // Jacobi or DILU with a coarse space; on request the p update rides along
+  // the next matrix-free product
+  const bool with_co = coarse && (fused || mode == 1);
+  const bool pfused = with_co && mode == 1 && matfree_on() && mf_->agg1 && p_fused_enabled();
+  const PUp pu{r, dg, mf_ ? mf_->agg1 : nullptr, nu};
+  const Cx<float> cxf = with_co ? cx<float>(pc) : Cx<float>{};
   if (two) {
     cg2_start<float>(cg, v32, fac);
-  } else if (fused) {
-    hipLaunchKernelGGL(k_rsum<float>, GR, B, 0, S, RW, r, st, part32);
-    const auto &cp = pat->color_ptr;
-    hipLaunchKernelGGL(k_dilu_first<float>, dim3(nblocks(cp[1] - cp[0])), B, 0, S, cp[0], cp[1], dg, r, z, done);
-    const int np = dilu_sweeps<float>(pat, A, v32, dg, r, z, done, prz, cw);
-    finish<OpSum, 1>(np, prz, FinRz0{st});
-    MS_HIP(hipMemsetAsync(p, 0, n * sizeof(float), S));
-    hipLaunchKernelGGL(k_pcg_p<float>, GR, B, 0, S, RW, r, z, dg, 0, p, nu, st);   // beta = 0
+  } else if (with_co) {
+    cx_restart<float, true>(cxf, v32, nullptr, true);
   } else {
     if (coarse) {
       hipLaunchKernelGGL(k_rsum<float>, GR, B, 0, S, RW, r, st, part32);
@@ -1990,39 +2233,16 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
     finish<OpSum, 1>((int)GR.x, part32, FinRz0{st});
   }
   // the part of an iteration after the update kernel: residual check,
-  // preconditioner, r.z and p update.  DILU finishes r.r and r.z in one
-  // kernel after the sweeps (trigger: reliable-update checks active).
-  const bool merged = mode == 2 && (!coarse || fused);
-  // Jacobi with a coarse space: the coarse solve is spread over the split
-  // finisher's workgroups and beta is formed in the p update
-  const bool split = coarse && !fused && mode == 1;
-  const int nsplit = split ? (pat->coarse.k + kSplitRows - 1) / kSplitRows : 0;
-  if (split && cnu_split_.n < (size_t)nsplit) cnu_split_.alloc(nsplit);
-  // the split path's p update rides along the next matrix-free product
-  const bool pfused = split && matfree_on() && mf_->agg1 && p_fused_enabled();
-  const PUp pu{r, dg, mf_ ? mf_->agg1 : nullptr, nu, cnu_split_.p, nsplit};
+  // preconditioner, r.z and p update (trigger: reliable-update checks active)
   auto tail = [&](int trigger) {
-    if (split) {
-      hipLaunchKernelGGL((k_finish_split<3, float, FinUpdateSplit>), dim3(1 + nsplit), dim3(kFinThreads), 0, S,
-                         (int)GR.x, part32, FinUpdateSplit{st, trigger}, co, cnu_split_.p);
-      if (!pfused)
-        hipLaunchKernelGGL(k_pcg_p_split<float>, GR, B, 0, S, RW, r, dg, p, nu, st, cnu_split_.p, nsplit, 0);
-      return;
-    }
-    if (merged) {
-      const int np = dilu_sweeps<float>(pat, A, v32, dg, r, z, done, prz, cw);
-      hipLaunchKernelGGL((k_finish2<float, FinUpdRzRU>), dim3(1), dim3(kFinThreads), 0, S, (int)GR.x, part32, np,
-                         prz, FinUpdRzRU{st, trigger});
-    } else {
-      finish_co<3>((int)GR.x, part32, FinUpdateRU{st, jac, trigger}, co);
-      if (mode == 2) {
-        int np = dilu_sweeps<float>(pat, A, v32, dg, r, z, done, prz, cw);
-        finish<OpSum, 1>(np, prz, FinRz{st});
-      } else if (mode == 0) {
-        apply_pc<float>(pc, v32, fac, dg, r, z, done);
-        hipLaunchKernelGGL(k_dot<float>, G, B, 0, S, n, r, z, st, part32);
-        finish<OpSum, 1>(nblk_, part32, FinRz{st});
-      }
+    finish_co<3>((int)GR.x, part32, FinUpdateRU{st, jac, trigger}, co);
+    if (mode == 2) {
+      int np = dilu_sweeps<float>(pat, A, v32, dg, r, z, done, prz);
+      finish<OpSum, 1>(np, prz, FinRz{st});
+    } else if (mode == 0) {
+      apply_pc<float>(pc, v32, fac, dg, r, z, done);
+      hipLaunchKernelGGL(k_dot<float>, G, B, 0, S, n, r, z, st, part32);
+      finish<OpSum, 1>(nblk_, part32, FinRz{st});
     }
     hipLaunchKernelGGL(k_pcg_p<float>, GR, B, 0, S, RW, r, z, dg, jac, p, nu, st);
   };
@@ -2037,9 +2257,16 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
       MS_CHECK_LAUNCH();
       return;
     }
-    if (pfused) {   // apply a pending p update before r, p and z are rescaled
-      hipLaunchKernelGGL(k_pcg_p_split<float>, GR, B, 0, S, RW, r, dg, p, nu, st, cnu_split_.p, nsplit, 1);
-      hipLaunchKernelGGL(k_clear_pup, dim3(1), dim3(64), 0, S, st);
+    if (with_co) {
+      if (pfused) {   // apply a pending p update before r and p are rescaled
+        cx_p<float, true>(cxf, kCxPending);
+        hipLaunchKernelGGL(k_clear_pup, dim3(1), dim3(64), 0, S, st);
+      }
+      hipLaunchKernelGGL(k_fold, G, B, 0, S, n, y, x, st);
+      hipLaunchKernelGGL(k_true_res, G, B, 0, S, n, A, val, b, x, r_.p, st, part);
+      finish<OpSum, 1>(nblk_, part, FinRU{st});
+      cx_restart<float, true>(cxf, v32, r_.p, paused);   // paused: complete the interrupted iteration on the new r
+      return;
     }
     hipLaunchKernelGGL(k_fold, G, B, 0, S, n, y, x, st);
     hipLaunchKernelGGL(k_true_res, G, B, 0, S, n, A, val, b, x, r_.p, st, part);
@@ -2052,10 +2279,7 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
   const bool probe = g_probe.on;
   if (probe) g_probe.rows = n;
   int probe_pair = -1;   // the probe pair of the chunk last queued
-  // split path: the SpMV's p.q partials stay apart from the update's, which
-  // the update writes while other workgroups still read the SpMV's
-  if (split && pq32_.n < (size_t)nblk_) pq32_.alloc(nblk_);
-  float *spart = split ? pq32_.p : part32;
+  float *spart = with_co ? cxf.pq : part32;
   auto chunk = [&](int m, bool probe_last) {
     if (two) {
       for (int it = 0; it < m; it++) {
@@ -2079,13 +2303,12 @@ SolveResult Krylov::mixed(const double *val, const double *b, double *x, double 
       } else {
         spmv32(val, v32, p, q, st, spart, nullptr, nullptr, pfused ? &pu : nullptr);
       }
-      if (split) {   // alpha reduced inside the update (the SpMV's partials go to a buffer of their own)
-        hipLaunchKernelGGL(k_pcg_update_fa<float>, GR, B, 0, S, RW, nblk_, pq32_.p, p, q, y, r, dg, st, part32);
-      } else {
-        finish<OpSum, 1>(nblk_, part32, FinPap{st});
-        hipLaunchKernelGGL((k_pcg_update<float, float>), GR, B, 0, S, RW, p, q, y, r, z, dg, mode, c0end, st,
-                           part32);
+      if (with_co) {
+        cx_update<float, true>(cxf, v32, y, pfused);
+        continue;
       }
+      finish<OpSum, 1>(nblk_, part32, FinPap{st});
+      hipLaunchKernelGGL((k_pcg_update<float, float>), GR, B, 0, S, RW, p, q, y, r, z, dg, mode, c0end, st, part32);
       tail(1);
     }
   };

@@ -10,8 +10,6 @@ struct KS {              // device-resident solver scalars (one per solve)
   double sigma, scale;   // FP32 iteration runs on r/sigma; scale = sigma_old/sigma_new at an update
   double cnu;            // coarse part of r.z: (Z^T r) . E^-1 (Z^T r)
   double tol;
-  double rzd, rz_next;   // split coarse finisher: Jacobi part of r.z, r.z waiting to become rz
-  int rzp;               // rz_next pending
   int it, ierr, done, maxit;  // done: 0 running, 1 finished, 2 paused for a reliable update
   int coarse;            // coarse correction active
   int ru;                // reliable update requested for this iteration
@@ -67,12 +65,11 @@ struct MatFree {
 // 2M cells)
 bool p_fused_enabled();
 void set_p_fused(bool on);
-// arguments of the fused p update (beta from the coarse finisher's parts)
+// arguments of the fused p update (beta from the solver state)
 struct PUp {
   const float *r, *dg;
   const int *agg1;
-  const double *nu, *cnu;
-  int G;
+  const double *nu;
 };
 // the reduced solve's FP32 iterations apply S matrix-free (default on;
 // MIXSOLVER_SCHUR_MF=0 or ms_set_schur_matfree(0) forms S for them too)
@@ -148,6 +145,17 @@ class Krylov {
   template <class T> void cg2_start(const Cg2<T> &c, const T *val, const T *fac);
   template <class T, bool MIXED, class X>
   void cg2_iteration(const Cg2<T> &c, const T *val, const T *fac, X *x, hipEvent_t e0, hipEvent_t e1);
+  // PCG with a coarse space: vectors, partial arrays, chunk sums
+  template <class T> struct Cx {
+    int mode = 0, G = 0, nrz = 0, ncn = 0, cw = 0;   // grid; r.z partials; coarse parts of r.z; coarse workgroups
+    T *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *dg = nullptr;
+    T *rr = nullptr, *rz = nullptr, *csum = nullptr, *pq = nullptr;
+  };
+  template <class T> Cx<T> cx(PcKind pc);
+  template <class T, bool MIXED> void cx_p(const Cx<T> &c, int what);
+  template <class T, bool MIXED> void cx_direction(const Cx<T> &c, const T *val, int what);
+  template <class T, bool MIXED> void cx_restart(const Cx<T> &c, const T *val, const double *r64, bool direction);
+  template <class T, bool MIXED, class X> void cx_update(const Cx<T> &c, const T *val, X *x, bool ride);
   SolveResult bicg32(PcKind pc, int maxit, int window, bool coarse);
   template <class T> void coarse_apply(const T *in, T *out, const int *done, KS *st);
   void ensure32();
@@ -156,8 +164,7 @@ class Krylov {
   DBuf<double> r_, r0_, p_, q_, z_, s_, t_, ph_, sh_, fac_, dg_, part_, prz_;   // prz_: DILU sweep partials
   DBuf<float> val32_, r32_, r032_, p32_, q32_, z32_, s32_, t32_, ph32_, sh32_, x32_, fac32_, dg32_, part32_, prz32_;
   DBuf<KS> st_, st32_;
-  DBuf<double> cnu_split_;   // c.nu parts of k_finish_split
-  DBuf<float> pq32_;         // the SpMV's p.q partials on the split path
+  DBuf<double> cnu_split_;   // c.nu parts of k_cx_coarse
   DBuf<int> flag_;
   LevelFactor<double> lev_;
   LevelFactor<float> lev32_;

@@ -489,7 +489,11 @@ void build_coarse(SellPattern &P, const std::vector<int> &agg_dev, int k) {
   C.agg_cidx.assign(C.nchunks, 0);
   {
     std::vector<int> fill(C.agg_cptr.begin(), C.agg_cptr.end() - 1);
-    for (int c = 0; c < C.nchunks; c++) C.agg_cidx[fill[C.chunk_agg[c]]++] = c;
+    C.chunk_pos.assign(C.nchunks, 0);
+    for (int c = 0; c < C.nchunks; c++) {
+      C.chunk_pos[c] = fill[C.chunk_agg[c]]++;
+      C.agg_cidx[C.chunk_pos[c]] = c;
+    }
   }
   // counting sort of the stored entries by key agg(row)*k + agg(col)
   if (P.nstore > 0x7fffffffLL) fail(MS_EINVAL, "coarse space: matrix too large for 32-bit slots");
@@ -522,13 +526,14 @@ void Coarse::upload() {
   d_chunk_agg.upload(chunk_agg);
   d_agg_cptr.upload(agg_cptr);
   d_agg_cidx.upload(agg_cidx);
+  d_chunk_pos.upload(chunk_pos);
   d_e_ptr.upload(e_ptr);
   d_e_key.upload(e_key);
   d_e_slot.upload(e_slot);
 }
 
 size_t Coarse::device_bytes() const {
-  return d_chunk_ptr.bytes() + d_chunk_agg.bytes() + d_agg_cptr.bytes() + d_agg_cidx.bytes() + d_e_ptr.bytes() +
+  return d_chunk_pos.bytes() + d_chunk_ptr.bytes() + d_chunk_agg.bytes() + d_agg_cptr.bytes() + d_agg_cidx.bytes() + d_e_ptr.bytes() +
          d_e_key.bytes() + d_e_slot.bytes();
 }
 
