@@ -163,18 +163,17 @@ struct Coarse {
 };
 
 // Values of the coarse space for one matrix: dense E (k x k), FP64
-// Gauss-Jordan work matrix and pivot snapshots, E^-1 in FP32, and the
+// Gauss-Jordan work matrix, E^-1 in FP32, and the
 // coarse solution nu (k).  Owned by the solver, so systems that share a
 // pattern (forked sweep cases) keep their own.
 struct CoarseMat {
-  DBuf<double> E, nu, W, rc, Eparts;
+  DBuf<double> E, nu, W, Eparts;
   DBuf<float> Einv;
   void ensure(int k) {
     const size_t kk = (size_t)k * k;
     if (E.n < kk) E.alloc(kk);
     if (Einv.n < kk) Einv.alloc(kk);
     if (W.n < kk) W.alloc(kk);
-    if (rc.n < 4 * (size_t)k) rc.alloc(4 * (size_t)k);
     if (nu.n < (size_t)k) nu.alloc(k);
   }
 };
@@ -230,6 +229,7 @@ struct SellPattern {
     int l0, l1;
     bool narrow;
     int s0 = 0, s1 = 0, t0 = 0, block = kSegThreads;
+    SweepStep step{};   // a wide level's
   };
   std::vector<LevSeg> seg_f, seg_b;
   SweepPlan sweep_f, sweep_b;

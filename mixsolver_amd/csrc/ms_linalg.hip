@@ -923,21 +923,8 @@ __global__ void k_set_sigma(KS *st) {
 // -------------------------------------------------------------- BiCGSTAB
 // Additive coarse correction of a BiCGSTAB preconditioner application,
 // out += Z E^-1 Z^T in (the p' matrix and so E are symmetric): chunk sums of
-// in (FP64, one workgroup per aggregate chunk), nu = E^-1 c by one finisher
-// workgroup, then nu of each row's aggregate added to out.  All three skip a
-// finished solve, as the other BiCGSTAB kernels do.
-template <class T>
-__global__ void k_co_restrict(Rows RW, const T *in, double *cpart, const int *done) {
-  if (*done) return;
-  int i, a;
-  double v[1] = {0.0};
-  if (RW.get(i, a)) v[0] = (double)in[i];
-  block_partials<OpSum, 1, double>(v, cpart);
-}
-__global__ __launch_bounds__(kFinThreads) void k_co_solve(const double *cpart, CoDev co, const int *done) {
-  if (*done) return;
-  coarse_solve<1, double>(cpart, co);
-}
+// in come from the launch that formed it (FP64), nu = E^-1 c from k_cx_coarse,
+// then nu of each row's aggregate is added to out.
 template <class T>
 __global__ void k_co_prolong(Rows RW, const double *nu, T *out, const int *done) {
   if (*done) return;
@@ -945,32 +932,143 @@ __global__ void k_co_prolong(Rows RW, const double *nu, T *out, const int *done)
   if (RW.get(i, a)) out[i] = out[i] + (T)nu[a];
 }
 
-template <class T>
-__global__ void k_bi_init(int n, const T *r, T *r0, T *p, T *v, KS *st) {
-  int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) {
-    r0[i] = r[i];
-    p[i] = T(0);
-    v[i] = T(0);
+// An iteration, with the scalar recurrences in the prologues of the launches
+// that need them, as the PCG above (it took fourteen launches beside the
+// preconditioner's, most of them a few microseconds of latency each):
+//   k_bi_p:  [r.r -> stop?, rho = r.r0 -> beta]  p = r + beta (p - omega v)
+//            and the preconditioner's first stage; chunk sums of p
+//   (preconditioner)   ph = M^-1 p
+//   k_bi_spmv_dot:     v = A ph; v.r0
+//   k_bi_s:  [v.r0 -> alpha]  s = r - alpha v, first stage; s.s
+//   k_finish (FinBiS): |s| small enough?  (x + alpha ph then ends the solve)
+//   (preconditioner)   sh = M^-1 s
+//   k_bi_spmv_omega:   t = A sh; t.t, t.s
+//   k_bi_xr: [t.t, t.s -> omega]  x += alpha ph + omega sh, r = s - omega t;
+//            r.r, r.r0
+// First stage: Jacobi's ph = p/d (mode 1), DILU's p/d on the first colour
+// (mode 2).  Rows go by chunks of at most 256, a wavefront each: aggregate
+// chunks with a coarse space, else plain blocks (C.ptr null).
+__device__ __forceinline__ void chunk_rows(const Chunks &C, int n, int ch, int &r0, int &r1) {
+  if (C.ptr) {
+    r0 = C.ptr[ch];
+    r1 = C.ptr[ch + 1];
+  } else {
+    r0 = ch * kBlock;
+    r1 = min(n, r0 + kBlock);
   }
-  if (i == 0) {
-    st->rho_old = 1.0;
-    st->alpha = 1.0;
-    st->omega = 1.0;
+}
+
+// r0 = r and the r.r, r.r0 partials of the initial residual
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_bi_init(int n, const T *r, T *r0, T *rrp, T *rhop) {
+  T v[1] = {T(0)};
+  const RowRange R = cg_range(n);
+  for (int b = R.b0; b < R.b1; b++) {
+    const int i = b * kBlock + threadIdx.x;
+    if (i < n) {
+      const T ri = r[i];
+      r0[i] = ri;
+      v[0] = v[0] + ri * ri;
+    }
+  }
+  __shared__ T lds[kBlock / 64];
+  block_reduce<OpSum, 1, T>(v, lds);
+  if (threadIdx.x == 0) {
+    rrp[blockIdx.x] = v[0];
+    rhop[blockIdx.x] = v[0];
   }
 }
 
 template <class T>
-__global__ void k_bi_p(int n, const T *r, const T *v, T *p, const KS *st) {
-  if (st->done) return;
-  int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) p[i] = r[i] + (T)st->beta * (p[i] - (T)st->omega * v[i]);
+__global__ __launch_bounds__(kBlock) void k_bi_p(Chunks C, int n, const T *r, const T *v, T *p, T *ph, const T *dg,
+                                                 int mode, int c0end, KS *st, int np, const T *rrp, const T *rhop,
+                                                 double *csum) {
+  const int done = st->done;
+  const RowRange R = cx_range(C);
+  const int lane = threadIdx.x & 63;
+  int ch = R.b0 + (int)(threadIdx.x >> 6), r0 = 0, r1 = 0;
+  T ri[kCxRows], pi[kCxRows], vi[kCxRows];
+  auto load = [&]() {
+    chunk_rows(C, n, ch, r0, r1);
+    r0 += lane;
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = min(r0 + u * kSlice, r1 - 1);
+      ri[u] = r[i];
+      pi[u] = p[i];
+      vi[u] = v[i];
+    }
+  };
+  if (ch < R.b1) load();
+  if (done) return;
+  const int first = st->it == 0, par = st->it & 1;
+  T sums[2];
+  cg_sums<T>(np, rrp, np, rhop, sums);
+  __shared__ double beta_s;
+  __shared__ int stop_s;
+  if (threadIdx.x == 0) {
+    const bool w = blockIdx.x == 0;
+    const double res = sqrt((double)sums[0]) / st->bnrm, rho = (double)sums[1];
+    double beta = 0.0;
+    int stop = 0;
+    if (!first && res <= st->tol) {
+      stop = 1;
+      if (w) {
+        st->rr = (double)sums[0];
+        st->res = res;
+        st->done = 1;
+      }
+    } else if (fabs(rho) < kTiny) {
+      stop = 1;
+      if (w) {
+        st->it = st->it + 1;
+        st->rho = rho;
+        st->ierr = 2;
+        st->done = 1;
+      }
+    } else {
+      beta = first ? rho : (rho / st->rz2[par ^ 1]) * (st->alpha / st->omega);
+      if (w) {
+        if (!first) {
+          st->rr = (double)sums[0];
+          st->res = res;
+        }
+        st->rho = rho;
+        st->beta = beta;
+        st->rz2[par] = rho;
+        st->par = par;
+      }
+    }
+    beta_s = beta;
+    stop_s = stop;
+  }
+  __syncthreads();
+  if (stop_s) return;
+  const T beta = (T)beta_s, omega = first ? T(1) : (T)st->omega;
+  for (; ch < R.b1; ch += kBlock / kSlice) {
+    if (ch >= R.b0 + kBlock / kSlice) load();
+    double cs = 0.0;
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = r0 + u * kSlice;
+      if (i < r1) {
+        const T pn = first ? ri[u] : ri[u] + beta * (pi[u] - omega * vi[u]);
+        p[i] = pn;
+        cs = cs + (double)pn;
+        if (mode == 1 || (mode == 2 && i < c0end)) ph[i] = pn / dg[i];
+      }
+    }
+    if (csum) {
+      cs = wave_sum(cs);
+      if (lane == 0) csum[C.pos[ch]] = cs;
+    }
+  }
 }
 
 template <class T, int C16 = -1>
 __global__ void k_bi_spmv_dot(int n, Mat A, const T *val, const T *ph, const T *r0, T *v, const KS *st, T *part) {
   if (st->done) return;
-  int i = blockIdx.x * kBlock + threadIdx.x;
+  int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   T w[1] = {T(0)};
   if (i < n) {
     const T r0i = r0[i];
@@ -982,18 +1080,59 @@ __global__ void k_bi_spmv_dot(int n, Mat A, const T *val, const T *ph, const T *
 }
 
 template <class T>
-__global__ void k_bi_s(int n, const T *r, const T *v, T *s, const KS *st, T *part) {
-  if (st->done) return;
-  int i = blockIdx.x * kBlock + threadIdx.x;
-  T w[1] = {T(0)};
-  if (i < n) {
-    T si = r[i] - (T)st->alpha * v[i];
-    s[i] = si;
-    w[0] = si * si;
+__global__ __launch_bounds__(kBlock) void k_bi_s(Chunks C, int n, const T *r, const T *v, T *s, T *sh, const T *dg,
+                                                 int mode, int c0end, KS *st, int nvp, const T *vp, T *ssp,
+                                                 double *csum) {
+  const int done = st->done;
+  const RowRange R = cx_range(C);
+  const int lane = threadIdx.x & 63;
+  int ch = R.b0 + (int)(threadIdx.x >> 6), r0 = 0, r1 = 0;
+  T ri[kCxRows], vi[kCxRows];
+  auto load = [&]() {
+    chunk_rows(C, n, ch, r0, r1);
+    r0 += lane;
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = min(r0 + u * kSlice, r1 - 1);
+      ri[u] = r[i];
+      vi[u] = v[i];
+    }
+  };
+  if (ch < R.b1) load();
+  if (done) return;
+  T sums[2];
+  cg_sums<T>(nvp, vp, 0, vp, sums);
+  __shared__ double alpha_s;
+  if (threadIdx.x == 0) {
+    alpha_s = st->rz2[st->par] / (double)sums[0];
+    if (blockIdx.x == 0) st->alpha = alpha_s;
   }
-  block_partials<OpSum, 1>(w, part);
+  __syncthreads();
+  const T alpha = (T)alpha_s;
+  T w[1] = {T(0)};
+  for (; ch < R.b1; ch += kBlock / kSlice) {
+    if (ch >= R.b0 + kBlock / kSlice) load();
+    double cs = 0.0;
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = r0 + u * kSlice;
+      if (i < r1) {
+        const T si = ri[u] - alpha * vi[u];
+        s[i] = si;
+        w[0] = w[0] + si * si;
+        cs = cs + (double)si;
+        if (mode == 1 || (mode == 2 && i < c0end)) sh[i] = si / dg[i];
+      }
+    }
+    if (csum) {
+      cs = wave_sum(cs);
+      if (lane == 0) csum[C.pos[ch]] = cs;
+    }
+  }
+  block_partials<OpSum, 1>(w, ssp);
 }
 
+// x + alpha ph of a solve that ended on |s| (done = 2)
 template <class T>
 __global__ void k_bi_early(int n, const T *ph, T *x, const KS *st) {
   if (st->done != 2) return;
@@ -1001,14 +1140,11 @@ __global__ void k_bi_early(int n, const T *ph, T *x, const KS *st) {
   if (i < n) x[i] = x[i] + (T)st->alpha * ph[i];
 }
 
-__global__ void k_done2_to_1(KS *st) {
-  if (threadIdx.x == 0 && st->done == 2) st->done = 1;
-}
-
 template <class T, int C16 = -1>
-__global__ void k_bi_spmv_omega(int n, Mat A, const T *val, const T *sh, const T *s, T *t, const KS *st, T *part) {
+__global__ void k_bi_spmv_omega(int n, Mat A, const T *val, const T *sh, const T *s, T *t, const KS *st, T *ttp,
+                                T *tsp) {
   if (st->done) return;
-  int i = blockIdx.x * kBlock + threadIdx.x;
+  int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   T w[2] = {T(0), T(0)};
   if (i < n) {
     const T si = s[i];
@@ -1017,21 +1153,80 @@ __global__ void k_bi_spmv_omega(int n, Mat A, const T *val, const T *sh, const T
     w[0] = ti * ti;
     w[1] = ti * si;
   }
-  block_partials<OpSum, 2>(w, part);
+  __shared__ T lds[2 * (kBlock / 64)];
+  block_reduce<OpSum, 2, T>(w, lds);
+  if (threadIdx.x == 0) {
+    ttp[blockIdx.x] = w[0];
+    tsp[blockIdx.x] = w[1];
+  }
 }
 
 template <class T>
-__global__ void k_bi_xr(int n, const T *ph, const T *sh, const T *s, const T *t, T *x, T *r, const KS *st, T *part) {
-  if (st->done) return;
-  int i = blockIdx.x * kBlock + threadIdx.x;
-  T w[1] = {T(0)};
-  if (i < n) {
-    x[i] = x[i] + (T)st->alpha * ph[i] + (T)st->omega * sh[i];
-    T ri = s[i] - (T)st->omega * t[i];
-    r[i] = ri;
-    w[0] = ri * ri;
+__global__ __launch_bounds__(kBlock) void k_bi_xr(Chunks C, int n, const T *ph, const T *sh, const T *s, const T *t,
+                                                  const T *r0v, T *x, T *r, KS *st, int np, const T *ttp,
+                                                  const T *tsp, T *rrp, T *rhop) {
+  const int done = st->done;
+  const RowRange R = cx_range(C);
+  const int lane = threadIdx.x & 63;
+  int ch = R.b0 + (int)(threadIdx.x >> 6), r0 = 0, r1 = 0;
+  T pi[kCxRows], hi[kCxRows], si[kCxRows], ti[kCxRows], xi[kCxRows], oi[kCxRows];
+  auto load = [&]() {
+    chunk_rows(C, n, ch, r0, r1);
+    r0 += lane;
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = min(r0 + u * kSlice, r1 - 1);
+      pi[u] = ph[i];
+      hi[u] = sh[i];
+      si[u] = s[i];
+      ti[u] = t[i];
+      xi[u] = x[i];
+      oi[u] = r0v[i];
+    }
+  };
+  if (ch < R.b1) load();
+  if (done) return;
+  T sums[2];
+  cg_sums<T>(np, ttp, np, tsp, sums);
+  __shared__ double omega_s;
+  __shared__ int stop_s;
+  if (threadIdx.x == 0) {
+    const double tt = (double)sums[0], omega = (double)sums[1] / tt;
+    stop_s = tt < kTiny || fabs(omega) < kTiny;
+    omega_s = omega;
+    if (blockIdx.x == 0) {
+      st->tt = tt;
+      if (!(tt < kTiny)) st->omega = omega;
+      if (stop_s) {
+        st->ierr = 2;
+        st->done = 1;
+      }
+    }
   }
-  block_partials<OpSum, 1>(w, part);
+  __syncthreads();
+  if (stop_s) return;
+  const T alpha = (T)st->alpha, omega = (T)omega_s;
+  T w[2] = {T(0), T(0)};
+  for (; ch < R.b1; ch += kBlock / kSlice) {
+    if (ch >= R.b0 + kBlock / kSlice) load();
+#pragma unroll
+    for (int u = 0; u < kCxRows; u++) {
+      const int i = r0 + u * kSlice;
+      if (i < r1) {
+        x[i] = xi[u] + alpha * pi[u] + omega * hi[u];
+        const T rn = si[u] - omega * ti[u];
+        r[i] = rn;
+        w[0] = w[0] + rn * rn;
+        w[1] = w[1] + rn * oi[u];
+      }
+    }
+  }
+  __shared__ T lds[2 * (kBlock / 64)];
+  block_reduce<OpSum, 2, T>(w, lds);
+  if (threadIdx.x == 0) {
+    rrp[blockIdx.x] = w[0];
+    rhop[blockIdx.x] = w[1];
+  }
 }
 
 // ------------------------------------------------ preconditioner kernels
@@ -1429,14 +1624,15 @@ static int c16_of(const SellPattern *pat) {
 }
 
 template <class T>
-void Krylov::apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const T *in, T *out, const int *done) {
+void Krylov::apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const T *in, T *out, const int *done,
+                      bool staged) {
   Mat A = matof(pat);
   if (pc == PC_JACOBI) {
-    hipLaunchKernelGGL(k_jacobi<T>, dim3(nblk_), dim3(kBlock), 0, stream(), n, in, dg, out, done);
+    if (!staged) hipLaunchKernelGGL(k_jacobi<T>, dim3(nblk_), dim3(kBlock), 0, stream(), n, in, dg, out, done);
   } else if (pc == PC_DILU) {
     const auto &cp = pat->color_ptr;
     const int nc = (int)cp.size() - 1;
-    if (cp[1] > cp[0])
+    if (cp[1] > cp[0] && !staged)
       hipLaunchKernelGGL(k_dilu_first<T>, dim3(nblocks(cp[1] - cp[0])), dim3(kBlock), 0, stream(), cp[0], cp[1], dg,
                          in, out, done);
     for (int c = 1; c < nc; c++)
@@ -1458,8 +1654,8 @@ void Krylov::apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const 
           hipLaunchKernelGGL((k_dilu_bwd<T, 0>), dim3(nblocks(cp[c + 1] - cp[c])), dim3(kBlock), 0, stream(), cp[c],
                              cp[c + 1], A, val, dg, in, out, done, (T *)nullptr);
   } else {
-    if constexpr (sizeof(T) == 8) lev_.apply(*pat, fac, pc == PC_NATURAL_IC0, in, out, done);
-    else lev32_.apply(*pat, fac, pc == PC_NATURAL_IC0, in, out, done);
+    if constexpr (sizeof(T) == 8) lev_.apply(*pat, pc == PC_NATURAL_IC0, in, out, done);
+    else lev32_.apply(*pat, pc == PC_NATURAL_IC0, in, out, done);
   }
   MS_CHECK_LAUNCH();
 }
@@ -1556,28 +1752,24 @@ void Krylov::coarse_setup(const double *val) {
     MS_CHECK_LAUNCH();
     return;
   }
-  // FP64 Gauss-Jordan over the grid, one launch per pivot (k <= 1024)
-  double *rc[2][2] = {{M.rc.p, M.rc.p + C.k}, {M.rc.p + 2 * C.k, M.rc.p + 3 * C.k}};
-  const dim3 g(nblocks(kk));
-  hipLaunchKernelGGL(k_gj_init, g, dim3(kBlock), 0, stream(), C.k, M.E.p, M.W.p, rc[0][0], rc[0][1]);
-  for (int j = 0; j < C.k; j++) {
-    const int cur = j & 1, nxt = cur ^ 1;
-    hipLaunchKernelGGL(k_gj_step, g, dim3(kBlock), 0, stream(), C.k, j, M.W.p, rc[cur][0], rc[cur][1], rc[nxt][0],
-                       rc[nxt][1]);
-  }
-  hipLaunchKernelGGL(k_gj_out, g, dim3(kBlock), 0, stream(), kk, M.W.p, M.Einv.p);
+  const int kb = (C.k + kGjBlock - 1) / kGjBlock;
+  double *in = M.E.p, *out = M.W.p;
+  for (int j = 0; j < kb; j++, std::swap(in, out))
+    hipLaunchKernelGGL(k_gj_block, dim3(kb, kb), dim3(kBlock), 0, stream(), C.k, j, in, out,
+                       j + 1 == kb ? M.Einv.p : nullptr);
   MS_CHECK_LAUNCH();
 }
 
+// out += Z E^-1 c, c the chunk sums a BiCGSTAB launch left in co_part_
 template <class T>
-void Krylov::coarse_apply(const T *in, T *out, const int *done, KS *st) {
+void Krylov::coarse_apply(T *out, KS *st) {
   const Coarse &C = pat->coarse;
-  if (co_part_.n < (size_t)C.nchunks) co_part_.alloc(C.nchunks);
-  const Rows RW = rows_of(pat, true);
-  hipLaunchKernelGGL((k_co_restrict<T>), dim3(C.nchunks), dim3(kBlock), 0, stream(), RW, in, co_part_.p, done);
-  hipLaunchKernelGGL(k_co_solve, dim3(1), dim3(kFinThreads), 0, stream(), co_part_.p, codev_of(pat, cm_, true, st),
-                     done);
-  hipLaunchKernelGGL((k_co_prolong<T>), dim3(C.nchunks), dim3(kBlock), 0, stream(), RW, cm_.nu.p, out, done);
+  const int ncn = (C.k + kSplitRows - 1) / kSplitRows;
+  if (cnu_split_.n < (size_t)ncn) cnu_split_.alloc(ncn);
+  hipLaunchKernelGGL(k_cx_coarse<double>, dim3(ncn), dim3(kFinThreads), 0, stream(), C.k, C.d_agg_cptr.p, cm_.Einv.p,
+                     co_part_.p, cm_.nu.p, cnu_split_.p, st);
+  hipLaunchKernelGGL((k_co_prolong<T>), dim3(C.nchunks), dim3(kBlock), 0, stream(), rows_of(pat, true), cm_.nu.p, out,
+                     &st->done);
 }
 
 // buffers of the two-launch PCG: the vectors of the precision, p double
@@ -1869,6 +2061,72 @@ SolveResult Krylov::pcg(const double *val, const double *b, double *x, double to
 }
 
 // ---- BiCGSTAB -----------------------------------------------------------------
+// partial arrays of a solve in its buffer: r.r, r.r0 | v.r0, s.s | t.t, t.s
+template <class T>
+static void bi_parts(const SellPattern *pat, T *part, T *(&a)[6]) {
+  const size_t stride = (size_t)std::max(nblocks(pat->n), pat->coarse.nchunks) + 64;
+  for (int i = 0; i < 6; i++) a[i] = part + i * stride;
+}
+
+template <class T>
+void Krylov::bi_start(const Bi<T> &w) {
+  T *pt[6];
+  bi_parts(pat, w.part, pt);
+  const int G = std::min((nblk_ + kBlock / kSlice - 1) / (kBlock / kSlice), kCxGrid);
+  hipLaunchKernelGGL(k_bi_init<T>, dim3(G), dim3(kBlock), 0, stream(), n, w.r, w.r0, pt[0], pt[1]);
+  MS_CHECK_LAUNCH();
+}
+
+template <class T>
+void Krylov::bi_iteration(const Bi<T> &w, PcKind pc, const T *val, bool coarse) {
+  T *pt[6];
+  bi_parts(pat, w.part, pt);
+  const Mat A = matof(pat);
+  hipStream_t S = stream();
+  const dim3 B(kBlock), GS(nblk_);
+  const int *done = &w.st->done;
+  const int mode = pc == PC_JACOBI ? 1 : (pc == PC_DILU ? 2 : 0), c0end = pat->color_ptr[1];
+  const Chunks C = coarse ? chunks_of(pat) : Chunks{nullptr, nullptr, nullptr, nblk_};
+  if (coarse && co_part_.n < (size_t)C.n) co_part_.alloc(C.n);
+  double *csum = coarse ? co_part_.p : nullptr;
+  // the grid of the vector launches; the first iteration's partials are k_bi_init's
+  const int G0 = std::min((nblk_ + kBlock / kSlice - 1) / (kBlock / kSlice), kCxGrid);
+  const dim3 G(G0);
+  hipLaunchKernelGGL(k_bi_p<T>, G, B, 0, S, C, n, w.r, w.v, w.p, w.ph, w.dg, mode, c0end, w.st, G0, pt[0], pt[1],
+                     csum);
+  apply_pc<T>(pc, val, w.fac, w.dg, w.p, w.ph, done, true);
+  if (coarse) coarse_apply<T>(w.ph, w.st);
+  const bool c16 = c16_of<T>(pat);
+  if (c16) hipLaunchKernelGGL((k_bi_spmv_dot<T, 1>), GS, B, 0, S, n, A, val, w.ph, w.r0, w.v, w.st, pt[2]);
+  else hipLaunchKernelGGL((k_bi_spmv_dot<T, 0>), GS, B, 0, S, n, A, val, w.ph, w.r0, w.v, w.st, pt[2]);
+  hipLaunchKernelGGL(k_bi_s<T>, G, B, 0, S, C, n, w.r, w.v, w.s, w.sh, w.dg, mode, c0end, w.st, nblk_, pt[2], pt[3],
+                     csum);
+  finish<OpSum, 1>(G0, pt[3], FinBiS{w.st});
+  apply_pc<T>(pc, val, w.fac, w.dg, w.s, w.sh, done, true);
+  if (coarse) coarse_apply<T>(w.sh, w.st);
+  if (c16) hipLaunchKernelGGL((k_bi_spmv_omega<T, 1>), GS, B, 0, S, n, A, val, w.sh, w.s, w.t, w.st, pt[4], pt[5]);
+  else hipLaunchKernelGGL((k_bi_spmv_omega<T, 0>), GS, B, 0, S, n, A, val, w.sh, w.s, w.t, w.st, pt[4], pt[5]);
+  hipLaunchKernelGGL(k_bi_xr<T>, G, B, 0, S, C, n, w.ph, w.sh, w.s, w.t, w.r0, w.x, w.r, w.st, nblk_, pt[4], pt[5],
+                     pt[0], pt[1]);
+}
+
+// the state after a chunk: the residual test of its last iteration, and x of a
+// solve that ended on |s|
+template <class T>
+KS Krylov::bi_state(const Bi<T> &w) {
+  T *pt[6];
+  bi_parts(pat, w.part, pt);
+  const int G0 = std::min((nblk_ + kBlock / kSlice - 1) / (kBlock / kSlice), kCxGrid);
+  hipLaunchKernelGGL((k_cg_peek<T, false>), dim3(1), dim3(kBlock), 0, stream(), w.st, G0, pt[0]);
+  MS_CHECK_LAUNCH();
+  const KS hs = read_state<T>(w.st);
+  if (hs.done == 2) {
+    hipLaunchKernelGGL(k_bi_early<T>, dim3(nblk_), dim3(kBlock), 0, stream(), n, w.ph, w.x, w.st);
+    MS_CHECK_LAUNCH();
+  }
+  return hs;
+}
+
 SolveResult Krylov::bicgstab(const double *val, const double *b, double *x, double tol, int maxit, PcKind pc,
                              bool coarse) {
   SolveResult R;
@@ -1899,38 +2157,18 @@ SolveResult Krylov::bicgstab(const double *val, const double *b, double *x, doub
   if (coarse) coarse_setup(val);
   hipLaunchKernelGGL(k_residual<double>, G, B, 0, S, n, A, val, b, x, r_.p, part);
   finish<OpSum, 1>(nblk_, part, FinResidual{st});
-  hipLaunchKernelGGL(k_bi_init<double>, G, B, 0, S, n, r_.p, r0_.p, p_.p, q_.p, st);
   MS_CHECK_LAUNCH();
   hs = read_state<double>(st);
   R.res = hs.res;
   if (hs.done) return R;
-  double *v = q_.p;
-  const int *done = &st->done;
+  const Bi<double> w{r_.p, r0_.p, p_.p, q_.p, s_.p, t_.p, ph_.p, sh_.p, x, dg_.p, fac_.p, part, st};
+  bi_start<double>(w);
   int enq = 0, chunk = 2;
   while (true) {
     int m = std::min(chunk, maxit - enq);
-    for (int k = 0; k < m; k++) {
-      hipLaunchKernelGGL(k_dot<double>, G, B, 0, S, n, r_.p, r0_.p, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiRho{st});
-      hipLaunchKernelGGL(k_bi_p<double>, G, B, 0, S, n, r_.p, v, p_.p, st);
-      apply_pc<double>(pc, val, fac_.p, dg_.p, p_.p, ph_.p, done);
-      if (coarse) coarse_apply<double>(p_.p, ph_.p, done, st);
-      hipLaunchKernelGGL(k_bi_spmv_dot<double>, G, B, 0, S, n, A, val, ph_.p, r0_.p, v, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiAlpha{st});
-      hipLaunchKernelGGL(k_bi_s<double>, G, B, 0, S, n, r_.p, v, s_.p, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiS{st});
-      hipLaunchKernelGGL(k_bi_early<double>, G, B, 0, S, n, ph_.p, x, st);
-      hipLaunchKernelGGL(k_done2_to_1, dim3(1), dim3(64), 0, S, st);
-      apply_pc<double>(pc, val, fac_.p, dg_.p, s_.p, sh_.p, done);
-      if (coarse) coarse_apply<double>(s_.p, sh_.p, done, st);
-      hipLaunchKernelGGL(k_bi_spmv_omega<double>, G, B, 0, S, n, A, val, sh_.p, s_.p, t_.p, st, part);
-      finish<OpSum, 2>(nblk_, part, FinBiOmega{st});
-      hipLaunchKernelGGL(k_bi_xr<double>, G, B, 0, S, n, ph_.p, sh_.p, s_.p, t_.p, x, r_.p, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiXR{st});
-    }
-    MS_CHECK_LAUNCH();
+    for (int k = 0; k < m; k++) bi_iteration<double>(w, pc, val, coarse);
     enq += m;
-    hs = read_state<double>(st);
+    hs = bi_state<double>(w);
     if (hs.done || enq >= maxit) break;
     chunk = std::min(chunk * 2, 32);
   }
@@ -1949,50 +2187,18 @@ SolveResult Krylov::bicgstab(const double *val, const double *b, double *x, doub
 // refinement restarts it from the FP64 residual).
 SolveResult Krylov::bicg32(PcKind pc, int maxit, int window, bool coarse) {
   SolveResult R;
-  Mat A = matof(pat);
-  const dim3 G(nblk_), B(kBlock);
-  hipStream_t S = stream();
-  KS *st = st32_.p;
-  float *part = part32_.p;
-  float *v = q32_.p;
-  const int *done = &st->done;
-  hipLaunchKernelGGL(k_bi_init<float>, G, B, 0, S, n, r32_.p, r032_.p, p32_.p, v, st);
+  const Bi<float> w{r32_.p,  r032_.p, p32_.p, q32_.p,  s32_.p,  t32_.p, ph32_.p,
+                    sh32_.p, x32_.p,  dg32_.p, fac32_.p, part32_.p, st32_.p};
+  bi_start<float>(w);
   int enq = 0, chunk = 4;
   KS hs{};
   double best = HUGE_VAL;
   int it_best = 0;
   while (true) {
     int m = std::min(chunk, maxit - enq);
-    for (int k = 0; k < m; k++) {
-      hipLaunchKernelGGL(k_dot<float>, G, B, 0, S, n, r32_.p, r032_.p, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiRho{st});
-      hipLaunchKernelGGL(k_bi_p<float>, G, B, 0, S, n, r32_.p, v, p32_.p, st);
-      apply_pc<float>(pc, val32_.p, fac32_.p, dg32_.p, p32_.p, ph32_.p, done);
-      if (coarse) coarse_apply<float>(p32_.p, ph32_.p, done, st);
-      if (pat->has16)
-        hipLaunchKernelGGL((k_bi_spmv_dot<float, 1>), G, B, 0, S, n, A, val32_.p, ph32_.p, r032_.p, v, st, part);
-      else
-        hipLaunchKernelGGL((k_bi_spmv_dot<float, 0>), G, B, 0, S, n, A, val32_.p, ph32_.p, r032_.p, v, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiAlpha{st});
-      hipLaunchKernelGGL(k_bi_s<float>, G, B, 0, S, n, r32_.p, v, s32_.p, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiS{st});
-      hipLaunchKernelGGL(k_bi_early<float>, G, B, 0, S, n, ph32_.p, x32_.p, st);
-      hipLaunchKernelGGL(k_done2_to_1, dim3(1), dim3(64), 0, S, st);
-      apply_pc<float>(pc, val32_.p, fac32_.p, dg32_.p, s32_.p, sh32_.p, done);
-      if (coarse) coarse_apply<float>(s32_.p, sh32_.p, done, st);
-      if (pat->has16)
-        hipLaunchKernelGGL((k_bi_spmv_omega<float, 1>), G, B, 0, S, n, A, val32_.p, sh32_.p, s32_.p, t32_.p, st,
-                           part);
-      else
-        hipLaunchKernelGGL((k_bi_spmv_omega<float, 0>), G, B, 0, S, n, A, val32_.p, sh32_.p, s32_.p, t32_.p, st,
-                           part);
-      finish<OpSum, 2>(nblk_, part, FinBiOmega{st});
-      hipLaunchKernelGGL(k_bi_xr<float>, G, B, 0, S, n, ph32_.p, sh32_.p, s32_.p, t32_.p, x32_.p, r32_.p, st, part);
-      finish<OpSum, 1>(nblk_, part, FinBiXR{st});
-    }
-    MS_CHECK_LAUNCH();
+    for (int k = 0; k < m; k++) bi_iteration<float>(w, pc, val32_.p, coarse);
     enq += m;
-    hs = read_state<float>(st);
+    hs = bi_state<float>(w);
     if (hs.done || enq >= maxit) break;
     if (hs.res < 0.5 * best) {
       best = hs.res;

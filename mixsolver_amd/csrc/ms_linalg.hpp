@@ -86,7 +86,7 @@ struct LevelFactor {
   DBuf<T> vf, vb, df, db;   // forward / backward entries and diagonals, step order
   void pack(const SellPattern &P, const T *F, bool ic0);
   DBuf<T> xf, xb;           // vectors in level order (SellPattern::sweep_ordered)
-  void apply(const SellPattern &P, const T *F, bool ic0, const T *in, T *out, const int *done);
+  void apply(const SellPattern &P, bool ic0, const T *in, T *out, const int *done);
 };
 void factor_levels(const SellPattern &P, double *F, bool ic0, int *flag);
 
@@ -130,8 +130,10 @@ class Krylov {
  private:
   int setup_pc64(PcKind pc, const double *val);
   void setup_pc32(PcKind pc, const double *val);
+  // staged: the launch that formed `in` has done the first stage (Jacobi's
+  // quotient, DILU's first colour)
   template <class T> void apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const T *in, T *out,
-                                   const int *done);
+                                   const int *done, bool staged = false);
   template <class T> KS read_state(KS *d);
   // two-launch PCG (no coarse space): its vectors and partial arrays
   template <class T> struct Cg2 {
@@ -157,7 +159,17 @@ class Krylov {
   template <class T, bool MIXED> void cx_restart(const Cx<T> &c, const T *val, const double *r64, bool direction);
   template <class T, bool MIXED, class X> void cx_update(const Cx<T> &c, const T *val, X *x, bool ride);
   SolveResult bicg32(PcKind pc, int maxit, int window, bool coarse);
-  template <class T> void coarse_apply(const T *in, T *out, const int *done, KS *st);
+  template <class T> void coarse_apply(T *out, KS *st);
+  // BiCGSTAB: vectors, solution, preconditioner, partials and state
+  template <class T> struct Bi {
+    T *r, *r0, *p, *v, *s, *t, *ph, *sh, *x;
+    const T *dg, *fac;
+    T *part;
+    KS *st;
+  };
+  template <class T> void bi_start(const Bi<T> &w);
+  template <class T> void bi_iteration(const Bi<T> &w, PcKind pc, const T *val, bool coarse);
+  template <class T> KS bi_state(const Bi<T> &w);
   void ensure32();
   void coarse_setup(const double *val);   // E = Z^T A Z and its inverse
 

@@ -272,13 +272,13 @@ void SellPattern::build_levels_from(Col col_of) {
     const int nl = (int)ptr.size() - 1;
     for (int l = 0; l < nl;) {
       if (ptr[l + 1] - ptr[l] > kNarrowRows) {
-        seg.push_back({l, l + 1, false, 0, 0, 0, 0});
+        seg.push_back({l, l + 1, false});
         l++;
         continue;
       }
       int e = l;
       while (e < nl && ptr[e + 1] - ptr[e] <= kNarrowRows) e++;
-      seg.push_back({l, e, true, 0, 0, 0, kSegThreads});
+      seg.push_back({l, e, true});
       l = e;
     }
   };
