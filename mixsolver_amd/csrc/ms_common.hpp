@@ -37,6 +37,12 @@ int runtime_device();            // device selected by ensure_runtime (-1 before
 // launches and synchronises there.  Default priority; nullptr restores the
 // library stream.
 void set_thread_stream(hipStream_t s);
+// Streams of worker threads, kept for the next ones (a stream takes
+// milliseconds to create and to destroy): at most kIdleStreams idle ones, each
+// given back when its thread is done with it and has waited for its work.
+constexpr int kIdleStreams = 16;
+hipStream_t borrow_stream();          // nullptr on failure
+void give_back_stream(hipStream_t s);
 // device bytes allocated minus freed by DBuf on the calling thread (the
 // sweep server measures a case's footprint with it)
 long long thread_device_bytes();
@@ -65,12 +71,38 @@ bool col16_far_enabled();
 // state (MIXSOLVER_PIPELINE=0 turns it off)
 bool pipeline_enabled();
 
+// One device allocation that a thread's DBufs are carved from while it is the
+// thread's slab (set_thread_slab), for owners that allocate and free many
+// buffers together: a sweep case has about a hundred, and each hipFree waits
+// for the whole device.  A buffer that does not fit gets its own allocation.
+// The slab must outlive the buffers.
+class Slab {
+ public:
+  explicit Slab(size_t bytes);
+  ~Slab();
+  Slab(const Slab &) = delete;
+  Slab &operator=(const Slab &) = delete;
+  void *take(size_t bytes) {
+    const size_t a = (bytes + 255) & ~size_t(255);
+    if (a > size_ - used_) return nullptr;
+    void *r = p_ + used_;
+    used_ += a;
+    return r;
+  }
+
+ private:
+  char *p_ = nullptr;
+  size_t size_ = 0, used_ = 0;
+};
+Slab *thread_slab();
+void set_thread_slab(Slab *s);
+
 // --------------------------------------------------------- device buffers
 template <class T>
 struct DBuf {
   T *p = nullptr;
   size_t n = 0;
-  bool own = true;   // false: a read-only view of another system's buffer (forked systems)
+  bool own = true;   // false: a read-only view of another system's buffer (forked systems), or part of a slab
   DBuf() = default;
   explicit DBuf(size_t count) { alloc(count); }
   DBuf(const DBuf &) = delete;
@@ -88,6 +120,13 @@ struct DBuf {
   void alloc(size_t count) {
     release();
     n = count;
+    if (count && thread_slab()) {
+      p = static_cast<T *>(thread_slab()->take(count * sizeof(T)));
+      if (p) {
+        own = false;
+        return;
+      }
+    }
     if (count) {
       std::lock_guard<std::recursive_mutex> g(device_alloc_mutex());
       hipError_t e = hipMalloc(&p, count * sizeof(T));

@@ -1425,17 +1425,61 @@ Krylov::Krylov(const SellPattern *pat_) : pat(pat_), n(pat_->n) {
   prz_.alloc(2 * ((size_t)nblk_ + 64) + kMaxAgg);
   st_.alloc(1);
   flag_.alloc(1);
-  std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
-  MS_HIP(hipHostMalloc(&hpin_, 4096, hipHostMallocDefault));
-  for (auto &e : state_ev_) MS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  host_ = borrow_host_state();
+  hpin_ = host_.pin;
+  for (int i = 0; i < 2; i++) state_ev_[i] = host_.ev[i];
 }
 
 Krylov::~Krylov() {
+  if (chunk_exec_) {
+    std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
+    (void)hipGraphExecDestroy(chunk_exec_);
+  }
+  give_back_host_state(host_);
+}
+
+// Pinned page and events of a solver, kept for the next one: allocating and
+// freeing the page alone takes 75 us, and every solver call on a caller's
+// matrix has a solver of its own.  At most kIdleHostStates are kept.
+namespace {
+constexpr size_t kIdleHostStates = 32;
+std::mutex g_host_mu;
+std::vector<Krylov::HostState> g_host_idle;
+}  // namespace
+Krylov::HostState Krylov::borrow_host_state() {
+  int dev = 0;
+  MS_HIP(hipGetDevice(&dev));
+  {
+    std::lock_guard<std::mutex> g(g_host_mu);
+    for (size_t i = 0; i < g_host_idle.size(); i++)
+      if (g_host_idle[i].dev == dev) {
+        const HostState h = g_host_idle[i];
+        g_host_idle.erase(g_host_idle.begin() + i);
+        return h;
+      }
+  }
+  HostState h;
+  h.dev = dev;
   std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
-  if (chunk_exec_) (void)hipGraphExecDestroy(chunk_exec_);
-  for (auto &e : state_ev_)
+  MS_HIP(hipHostMalloc(&h.pin, 4096, hipHostMallocDefault));
+  for (auto &e : h.ev) MS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  return h;
+}
+void Krylov::give_back_host_state(const HostState &h) {
+  if (!h.pin) return;
+  // nothing of this solver may still write the page
+  const bool ok = hipStreamSynchronize(stream()) == hipSuccess;
+  if (ok) {
+    std::lock_guard<std::mutex> g(g_host_mu);
+    if (g_host_idle.size() < kIdleHostStates) {
+      g_host_idle.push_back(h);
+      return;
+    }
+  }
+  std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
+  for (const auto &e : h.ev)
     if (e) (void)hipEventDestroy(e);
-  if (hpin_) (void)hipHostFree(hpin_);
+  (void)hipHostFree(h.pin);
 }
 
 void Krylov::ensure32() {

@@ -126,8 +126,16 @@ class Krylov {
 
   const SellPattern *pat;
   int n;
+  struct HostState {   // pinned page for the solver state, and its events
+    int dev = 0;
+    void *pin = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+  };
 
  private:
+  static HostState borrow_host_state();
+  static void give_back_host_state(const HostState &h);
+  HostState host_;
   int setup_pc64(PcKind pc, const double *val);
   void setup_pc32(PcKind pc, const double *val);
   // staged: the launch that formed `in` has done the first stage (Jacobi's

@@ -154,12 +154,13 @@ class Sweep {
 
   void worker() {
     if (hipSetDevice(dev_ < 0 ? 0 : dev_) != hipSuccess) return;
-    hipStream_t st = nullptr;
-    if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return;
+    hipStream_t st = borrow_stream();
+    if (!st) return;
     set_thread_stream(st);
     for (;;) {
       SweepCase *c = nullptr;
       long long held = 0;   // bytes this case has reserved
+      long long need = 0;   // bytes of the buffers a case allocates, once known
       bool probe = false;
       {
         std::unique_lock<std::mutex> lk(mu_);
@@ -169,6 +170,7 @@ class Sweep {
         queue_.pop_front();
         active_++;
         peak_ = std::max(peak_, active_);
+        need = need_;
         if (footprint_ > 0) {
           held = reserve_of(footprint_);
           reserved_ += held;
@@ -183,8 +185,22 @@ class Sweep {
       long long fp = 0;
       int state = 2, steps = 0;
       try {
+        // the buffers of a case whose footprint is known come from one
+        // allocation: a hundred of them took 4 ms to allocate and, since each
+        // free waits for the device and so for the other cases, ten times that
+        // to free
+        std::unique_ptr<Slab> slab;
+        struct SlabGuard {
+          ~SlabGuard() { set_thread_slab(nullptr); }
+        } guard;
+        if (need > 0) {
+          slab = std::make_unique<Slab>((size_t)need + kSlabRounding);
+          set_thread_slab(slab.get());
+        }
         std::unique_ptr<System> f;
-        {
+        if (slab) {
+          f.reset(fork_system(base_, c->groups));
+        } else {
           std::lock_guard<std::recursive_mutex> g(device_alloc_mutex());
           f.reset(fork_system(base_, c->groups));
         }
@@ -198,7 +214,8 @@ class Sweep {
             fp = thread_device_bytes() - b0;
             if (probe) {
               std::lock_guard<std::mutex> lk(mu_);
-              footprint_ = std::max(footprint_, fp);
+              need_ = fp;
+              footprint_ = std::max(footprint_, fp + kSlabRounding);
               held = reserve_of(footprint_);
               reserved_ += held;
               probing_ = false;
@@ -219,8 +236,12 @@ class Sweep {
         c->stats[7] = f->st_mom_its;
         fp = std::max(fp, thread_device_bytes() - b0);
         if (c->keep) keep_fields(*f, *c);
-        std::lock_guard<std::recursive_mutex> g(device_alloc_mutex());
-        f.reset();
+        if (slab) {
+          f.reset();
+        } else {
+          std::lock_guard<std::recursive_mutex> g(device_alloc_mutex());
+          f.reset();
+        }
       } catch (const Error &e) {
         state = 3;
         c->err = e.code;
@@ -249,7 +270,7 @@ class Sweep {
       done_cv_.notify_all();
     }
     set_thread_stream(nullptr);
-    (void)hipStreamDestroy(st);
+    give_back_stream(st);
   }
 
   // final fields in the natural cell order
@@ -274,7 +295,8 @@ class Sweep {
   std::deque<SweepCase *> queue_;
   std::map<long long, std::unique_ptr<SweepCase>> cases_;
   long long next_id_ = 1, submitted_ = 0, done_ = 0, failed_ = 0, steps_ = 0;
-  long long footprint_ = 0, reserved_ = 0;
+  static constexpr long long kSlabRounding = 1 << 17;   // 256-byte alignment of a few hundred buffers
+  long long footprint_ = 0, reserved_ = 0, need_ = 0;
   long long active_ = 0, peak_ = 0;
   bool probing_ = false, stop_ = false;
 };

@@ -27,8 +27,8 @@ def _couplings(name):
         return chain(2, 1)
     if name == "more":          # nine lower entries in most rows
         return chain(700, 1, 2, 3, 5, 8, 13, 21, 34, 55)
-    if name == "far":           # one-row levels, neighbours 20000 positions back
-        return chain(30000, 1, 20000)
+    if name == "far":           # one-row levels, neighbours 17000 positions back
+        return chain(20000, 1, 17000)
     if name == "edge":          # the ring's last and first position, and one beyond
         return chain(17000, 1, 16383, 16384, 16385)
     if name == "wide":          # 60 levels of 600 rows, neighbours 24000 back: level order
