@@ -230,6 +230,7 @@ void build_schur(System &s, const std::vector<int> &agg_dev, int nagg) {
   }
   S->kry = std::make_unique<Krylov>(&S->pat);
   S->val.alloc(S->pat.nstore);
+  S->val.zero();   // padding slots take part in products
   S->rhs.alloc(n1);
   S->d.alloc(n1);
   S->r64.alloc(n);

@@ -1501,6 +1501,7 @@ System *fork_system(System &b, const std::vector<ms_bcgroup_t> &groups) {
     R->P = b.schur->P;
     R->kry = std::make_unique<Krylov>(R->P);
     R->val.alloc(R->P->nstore);
+    R->val.zero();
     R->rhs.alloc(R->n1);
     R->d.alloc(R->n1);
     R->r64.alloc(s.nc);
