@@ -272,6 +272,7 @@ struct SellPattern {
   };
   std::vector<LevSeg> seg_f, seg_b;
   SweepPlan sweep_f, sweep_b;
+  bool triangle_free = false;   // no two neighbours share a neighbour (set with the levels)
   bool sweep_ordered = false;   // one run each way, vectors in level order (d_lev_fb: forward position of a backward one)
   DBuf<int> d_lev_fb;
   // colour classes: rows of colour c are [col_ptr[c], col_ptr[c+1])

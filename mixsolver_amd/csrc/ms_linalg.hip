@@ -1635,7 +1635,7 @@ int Krylov::setup_pc64(PcKind pc, const double *val) {
   MS_HIP(hipMemcpyAsync(fac_.p, val, pat->nstore * sizeof(double), hipMemcpyDeviceToDevice, stream()));
   MS_HIP(hipMemsetAsync(flag_.p, 0, sizeof(int), stream()));
   const bool ic0 = pc == PC_NATURAL_IC0;
-  factor_levels(*pat, fac_.p, ic0, flag_.p);
+  factor_levels(*pat, fac_.p, ic0, flag_.p, diag_);
   lev_.pack(*pat, fac_.p, ic0);
   int h = 0;
   MS_HIP(hipMemcpyAsync(hpin_, flag_.p, sizeof(int), hipMemcpyDeviceToHost, stream()));

@@ -88,7 +88,10 @@ struct LevelFactor {
   DBuf<T> xf, xb;           // vectors in level order (SellPattern::sweep_ordered)
   void apply(const SellPattern &P, bool ic0, const T *in, T *out, const int *done);
 };
-void factor_levels(const SellPattern &P, double *F, bool ic0, int *flag);
+struct DiagFactor {   // work arrays of factor_levels: entries and diagonal in step order, factor's diagonal
+  DBuf<double> lo, up, dg, d;
+};
+void factor_levels(const SellPattern &P, double *F, bool ic0, int *flag, DiagFactor &D);
 
 class Krylov {
  public:
@@ -188,6 +191,7 @@ class Krylov {
   DBuf<int> flag_;
   LevelFactor<double> lev_;
   LevelFactor<float> lev32_;
+  DiagFactor diag_;
   CoarseMat cm_;             // E, E^-1 and nu of the coarse space for the current matrix
   DBuf<double> co_part_;     // chunk sums of a BiCGSTAB coarse correction
   const MatFree *mf_ = nullptr;
