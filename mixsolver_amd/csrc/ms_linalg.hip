@@ -838,6 +838,139 @@ __global__ __launch_bounds__(kBlock) void k_cx_p(Chunks C, const T *r, const T *
   }
 }
 
+// -------------------------------------------------------- PCG of one workgroup
+// A system whose matrix fits one workgroup's registers: FP64, Jacobi, at most
+// kSmallRows rows and kSmallWidth entries per row.  The direction is in LDS,
+// everything else in registers, two rows per thread at most, and an iteration
+// is three barriers instead of two launches, whose latency is all that the
+// two-launch form spends on such a system: 7.4 us an iteration at 1,728 rows,
+// here 2.5.  A launch runs at most kSmallIters iterations, so that it ends
+// whatever maxit is; p and r.z are kept for the next.
+constexpr int kSmallRows = 2048, kSmallWidth = 8, kSmallThreads = 1024, kSmallIters = 4096;
+
+template <int NV>
+__device__ __forceinline__ void small_sums(double (&v)[NV], double *lds) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int j = 0; j < NV; j++) v[j] = wave_sum(v[j]);
+  if (lane == 0)
+#pragma unroll
+    for (int j = 0; j < NV; j++) lds[w * NV + j] = v[j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    double s = lds[j];
+    for (int q = 1; q < nw; q++) s = s + lds[q * NV + j];
+    v[j] = s;
+  }
+}
+
+template <int R>   // rows per thread
+__global__ __launch_bounds__(kSmallThreads) void k_cg_small(int n, Mat A, const double *val, const double *dg,
+                                                            double *x, double *r, double *p, KS *st, int iters) {
+  if (st->done) return;
+  __shared__ double ps[kSmallRows], l1[kSmallThreads / 64], l2[2 * (kSmallThreads / 64)];
+  const int t = threadIdx.x, nt = blockDim.x;
+  const double bnrm = st->bnrm, tol = st->tol;
+  int it = st->it, c[R][kSmallWidth];
+  const bool first = it == 0;
+  double rz = st->rz2[0];
+  double a[R][kSmallWidth], xi[R], ri[R], di[R], pi[R];
+#pragma unroll
+  for (int u = 0; u < R; u++) {
+    const int i = t + u * nt;
+    const bool in = i < n;
+    const long long o0 = in ? A.off[i >> 6] : 0;
+    const int w = in ? (int)((A.off[(i >> 6) + 1] - o0) >> 6) : 0;
+#pragma unroll
+    for (int k = 0; k < kSmallWidth; k++) {
+      const long long q = o0 + (i & 63) + (long long)k * kSlice;
+      c[u][k] = k < w ? A.col[q] : (in ? i : 0);
+      a[u][k] = k < w ? val[q] : 0.0;
+    }
+    xi[u] = in ? x[i] : 0.0;
+    ri[u] = in ? r[i] : 0.0;
+    di[u] = in ? dg[i] : 1.0;
+    pi[u] = in && !first ? p[i] : 0.0;
+  }
+  if (first) {
+    double v[1] = {0.0};
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      pi[u] = ri[u] / di[u];
+      v[0] = v[0] + ri[u] * pi[u];
+    }
+    small_sums<1>(v, l1);
+    rz = v[0];
+  }
+  int ierr = 0, done = 0;
+  double res = st->res;
+  for (int e = 0; e < iters; e++) {
+#pragma unroll
+    for (int u = 0; u < R; u++)
+      if (t + u * nt < n) ps[t + u * nt] = pi[u];
+    __syncthreads();
+    double qi[R], v1[1] = {0.0};
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < kSmallWidth; k++) s = s + a[u][k] * ps[c[u][k]];
+      qi[u] = s;
+      v1[0] = v1[0] + pi[u] * s;
+    }
+    small_sums<1>(v1, l1);   // its barrier also ends the reads of ps
+    it++;
+    if (fabs(v1[0]) < kTiny) {
+      ierr = 2;
+      done = 1;
+      break;
+    }
+    const double alpha = rz / v1[0];
+    double v2[2] = {0.0, 0.0}, zi[R];
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      xi[u] = xi[u] + alpha * pi[u];
+      ri[u] = ri[u] - alpha * qi[u];
+      zi[u] = ri[u] / di[u];
+      v2[0] = v2[0] + ri[u] * ri[u];
+      v2[1] = v2[1] + ri[u] * zi[u];
+    }
+    small_sums<2>(v2, l2);
+    res = sqrt(v2[0]) / bnrm;
+    if (res <= tol) {
+      done = 1;
+      break;
+    }
+    if (fabs(rz) < kTiny) {
+      ierr = 2;
+      done = 1;
+      break;
+    }
+    const double beta = v2[1] / rz;
+    rz = v2[1];
+#pragma unroll
+    for (int u = 0; u < R; u++) pi[u] = zi[u] + beta * pi[u];
+  }
+#pragma unroll
+  for (int u = 0; u < R; u++) {
+    const int i = t + u * nt;
+    if (i < n) {
+      x[i] = xi[u];
+      r[i] = ri[u];
+      p[i] = pi[u];
+    }
+  }
+  __syncthreads();   // every thread has read the state
+  if (t == 0) {
+    st->it = it;
+    st->rz2[0] = rz;
+    st->res = res;
+    st->ierr = ierr;
+    st->done = done;
+  }
+}
+
 __global__ void k_clear_pup(KS *st) {
   if (threadIdx.x == 0) st->pup = 0;
 }
@@ -1977,6 +2110,14 @@ void Krylov::cg2_iteration(const Cg2<T> &c, const T *val, const T *fac, X *x, hi
   cg2_precond<T>(c, val, fac);
 }
 
+// the whole matrix fits the registers of one workgroup (k_cg_small)
+bool Krylov::small_system() const {
+  if (n > kSmallRows) return false;
+  for (int s = 0; s < pat->nslices; s++)
+    if (pat->off[s + 1] - pat->off[s] > (long long)kSmallWidth * kSlice) return false;
+  return true;
+}
+
 SolveResult Krylov::pcg(const double *val, const double *b, double *x, double tol, int maxit, PcKind pc,
                         bool coarse, bool reuse) {
   SolveResult R;
@@ -2020,6 +2161,26 @@ SolveResult Krylov::pcg(const double *val, const double *b, double *x, double to
   if (hs.done) return R;
   const int jac = pc == PC_JACOBI;
   const int *done = &st->done;
+  if (!coarse && jac && small_system()) {
+    const int rows = n <= kSmallThreads ? 1 : 2, nt = (n + 64 * rows - 1) / (64 * rows) * 64;
+    for (int left = maxit; left > 0 && !hs.done; left -= kSmallIters) {
+      const int m = std::min(left, kSmallIters);
+      if (rows == 1)
+        hipLaunchKernelGGL(k_cg_small<1>, dim3(1), dim3(nt), 0, S, n, A, val, dg_.p, x, r_.p, p_.p, st, m);
+      else
+        hipLaunchKernelGGL(k_cg_small<2>, dim3(1), dim3(nt), 0, S, n, A, val, dg_.p, x, r_.p, p_.p, st, m);
+      MS_CHECK_LAUNCH();
+      hs = read_state<double>(st);
+    }
+    R.it = hs.it;
+    R.res = hs.res;
+    R.ierr = hs.ierr;
+    if (!hs.done) {        // DO-loop exhaustion: it = maxit + 1, ierr = 1
+      R.it = maxit + 1;
+      R.ierr = 1;
+    }
+    return R;
+  }
   if (!coarse) {
     const Cg2<double> cg = cg2<double>(pc);
     cg2_start<double>(cg, val, fac_.p);

@@ -146,6 +146,7 @@ class Krylov {
   template <class T> void apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const T *in, T *out,
                                    const int *done, bool staged = false);
   template <class T> KS read_state(KS *d);
+  bool small_system() const;
   // two-launch PCG (no coarse space): its vectors and partial arrays
   template <class T> struct Cg2 {
     PcKind pc = PC_JACOBI;

@@ -33,7 +33,12 @@ def _system(n, lags, seed=3):
     return rp, (cols[o] + 1).astype(np.int32), vals[o], rng.normal(size=n)
 
 
-@pytest.mark.parametrize("n,lags", [(1, ()), (2, (1,)), (255, (1, 7)), (256, (1, 7)), (257, (1, 7, 100)),
+# up to 2048 rows of at most 8 entries the FP64 solve is one workgroup's: one
+# and two rows per thread, a last wavefront with few rows, and the first sizes
+# on either side that take the two launches
+@pytest.mark.parametrize("n,lags", [(64, (1, 5)), (1023, (1, 30, 31)), (1024, (1, 30, 31)), (1025, (1, 30, 31)),
+                                    (2047, (1, 40)), (2048, (1, 40, 900)), (2049, (1, 40)), (2000, (1, 2, 3, 4)),
+                                    (1, ()), (2, (1,)), (255, (1, 7)), (256, (1, 7)), (257, (1, 7, 100)),
                                     (5000, (1, 2, 3, 5, 8, 13, 21)), (2048 * 256 + 3, (1, 300))])
 def test_two_launch_pcg_against_oracle(n, lags):
     from oracle import pyoracle
