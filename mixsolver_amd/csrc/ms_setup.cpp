@@ -1092,27 +1092,38 @@ System *create_system(int nnodes, const double *x, int nfaces, const long long *
   s.face_upload(s.d_c1, s.c1);
   s.face_upload(s.d_fgrp, s.fgrp);
   if (s.nper > 0) s.face_upload(s.d_pidx, s.pidx);
-  s.d_cf_ptr.upload(s.cf_ptr);
   {
-    std::vector<int> ent(s.cf_ent.size());
-    for (size_t k = 0; k < ent.size(); k++) ent[k] = 2 * s.fo2d[s.cf_ent[k] >> 1] + (s.cf_ent[k] & 1);
+    std::vector<int> len(nc);
+    s.cf_off.assign((nc + 63) / 64 + 1, 0);
+    for (int r = 0; r < nc; r++) len[r] = s.cf_ptr[r + 1] - s.cf_ptr[r];
+    for (size_t q = 0; q + 1 < s.cf_off.size(); q++) {
+      const int r1 = std::min(nc, 64 * (int)(q + 1));
+      s.cf_off[q + 1] = s.cf_off[q] + 64LL * *std::max_element(len.begin() + 64 * q, len.begin() + r1);
+    }
+    std::vector<int> ent(s.cf_off.back(), 0), oth(s.cf_off.back(), -1);
+    std::vector<long long> slot(s.cf_off.back(), -1);
+    int r = 0;
+    s.each_entry([&](int k, long long q) {
+      const int f = s.cf_ent[k] >> 1, side = s.cf_ent[k] & 1;
+      while (k >= s.cf_ptr[r + 1]) r++;
+      ent[q] = 2 * s.fo2d[f] + side;
+      if (s.c1[f] < 0) return;
+      oth[q] = side == 0 ? s.c1[f] : s.c0[f];
+      const long long *b = s.cf_slot.data() + s.cf_ptr[r], *e = s.cf_slot.data() + k;
+      slot[q] = 2 * s.cf_slot[k] + (std::find(b, e, s.cf_slot[k]) == e ? 1 : 0);
+    });
+    s.d_cf_off.upload(s.cf_off);
+    s.d_cf_len.upload(len);
     s.d_cf_ent.upload(ent);
+    s.d_e_oth.upload(oth);
+    s.d_cf_slot.upload(slot);
   }
   if (s.renumbered) s.d_o2n.upload(s.o2n);
-  s.d_cf_slot.upload(s.cf_slot);
   s.d_diag_slot.upload(s.diag_slot);
   s.face_upload(s.d_xf, s.xf, 3);
   s.face_upload(s.d_sf, s.sf, 3);
   s.face_upload(s.d_area, s.area);
   s.face_upload(s.d_lf, s.lf);
-  {
-    std::vector<int> oth(s.cf_ent.size());
-    for (size_t k = 0; k < oth.size(); k++) {
-      const int f = s.cf_ent[k] >> 1;
-      oth[k] = s.c1[f] < 0 ? -1 : ((s.cf_ent[k] & 1) == 0 ? s.c1[f] : s.c0[f]);
-    }
-    s.d_e_oth.upload(oth);
-  }
   s.entry_upload(s.d_e_lf, s.lf);
   s.entry_upload(s.d_e_sf, s.sf, 3);
   s.d_vol.upload(vol);
@@ -1440,7 +1451,8 @@ System *fork_system(System &b, const std::vector<ms_bcgroup_t> &groups) {
   s.d_c0.alias(b.d_c0);
   s.d_c1.alias(b.d_c1);
   s.d_fgrp.alias(b.d_fgrp);
-  s.d_cf_ptr.alias(b.d_cf_ptr);
+  s.d_cf_off.alias(b.d_cf_off);
+  s.d_cf_len.alias(b.d_cf_len);
   s.d_cf_ent.alias(b.d_cf_ent);
   s.d_cf_slot.alias(b.d_cf_slot);
   s.d_diag_slot.alias(b.d_diag_slot);
@@ -1540,7 +1552,8 @@ DMesh System::dmesh() const {
   m.lf = d_lf.p;
   m.vol = d_vol.p;
   m.xc = d_xc.p;
-  m.cf_ptr = d_cf_ptr.p;
+  m.cf_off = d_cf_off.p;
+  m.cf_len = d_cf_len.p;
   m.cf_ent = d_cf_ent.p;
   m.pair_n0 = P->color_ptr.size() == 3 ? P->color_ptr[1] : 0;
   m.e_oth = d_e_oth.p;
@@ -1632,7 +1645,7 @@ size_t System::device_bytes() const {
     b += v->bytes();
   b += d_fflag.bytes() + d_tmode_s.bytes() + d_cztype.bytes() + d_iface_vel.bytes() + d_iface_p.bytes() +
        d_iface_slip_C.bytes() + d_iface_peer_vel.bytes() + d_tval_s.bytes();
-  b += d_c0.bytes() + d_c1.bytes() + d_fgrp.bytes() + d_pidx.bytes() + d_cf_ptr.bytes() + d_cf_ent.bytes() + d_cf_slot.bytes() +
+  b += d_c0.bytes() + d_c1.bytes() + d_fgrp.bytes() + d_pidx.bytes() + d_cf_off.bytes() + d_cf_len.bytes() + d_cf_ent.bytes() + d_cf_slot.bytes() +
        d_diag_slot.bytes();
   b += d_o2n.bytes() + d_fo2d.bytes() + d_face_get.bytes() + d_ref2dev.bytes();
   b += d_e_oth.bytes() + d_e_lf.bytes() + d_e_sf.bytes() + d_e_Dm.bytes() + d_e_muf.bytes() + d_e_tcor.bytes();

@@ -23,13 +23,15 @@ struct DMesh {
   int pair_n0;                             // > 0: two-colour numbering, rows of colour 0 (cell_row)
   const int *c0, *c1, *fgrp;               // c1 < 0 on boundary faces
   const double *xf, *sf, *area, *lf, *vol, *xc;
-  const int *cf_ptr, *cf_ent;              // cell -> faces ascending, ent = 2*face + side
+  const long long *cf_off;                 // cell -> faces ascending, in slices of 64 cells (cf_begin)
+  const int *cf_len, *cf_ent;              // ent = 2*face + side
   // the same per cell-face entry k (cf order), so a cell's face loads are
   // adjacent in memory: the other cell (-1 on boundary faces), lf, sf (3),
   // Dm, muf, tcor (3) of the entry's face
   const int *e_oth;
   const double *e_lf, *e_sf, *e_Dm, *e_muf, *e_tcor;
-  const long long *cf_slot, *diag_slot;    // matrix slot of (cell, other) / (cell, cell)
+  const long long *cf_slot;                // 2 * matrix slot of (cell, other) + first face of the pair, or -1
+  const long long *diag_slot;              // matrix slot of (cell, cell)
   const double *dn, *dvs, *Dm, *muf, *tcor, *dw, *Dmb;   // momentum / PPE face constants
   const double *Dt, *kf, *Dtb;                           // energy face constants
   const signed char *tmode;                // boundary thermal mode 0 neumann0 1 dirichlet 2 flux
@@ -151,20 +153,29 @@ struct System {
   double flux_ref = 1.0;
   double bnd_area = 0.0;   // boundary area (flux_ref)
   // device mesh data
-  DBuf<int> d_c0, d_c1, d_fgrp, d_cf_ptr, d_cf_ent;
-  DBuf<long long> d_cf_slot, d_diag_slot;
+  DBuf<int> d_c0, d_c1, d_fgrp, d_cf_len, d_cf_ent;
+  DBuf<long long> d_cf_off, d_cf_slot, d_diag_slot;
   // numbering maps of the API boundary (ms_io.hip): cells (renumbered systems),
   // faces and matrix slots (uploaded on first use)
   DBuf<int> d_o2n, d_fo2d, d_face_get;
   DBuf<long long> d_ref2dev;
   DBuf<int> d_e_oth;
   DBuf<double> d_e_lf, d_e_sf, d_e_Dm, d_e_muf, d_e_tcor;
+  // The device's cell-face entries: slices of 64 cells, as long as their
+  // longest cell; entry kk of cell r at cf_off[r / 64] + 64 kk + r % 64.
+  std::vector<long long> cf_off;
+  template <class F>
+  void each_entry(F fn) const {   // fn(entry of cf_ent, its device position)
+    for (int r = 0; r < nc; r++)
+      for (int k = cf_ptr[r]; k < cf_ptr[r + 1]; k++) fn(k, cf_off[r >> 6] + 64LL * (k - cf_ptr[r]) + (r & 63));
+  }
   // host face array (face order, width values per face) -> per cell-face entry
   template <class T>
   void entry_upload(DBuf<T> &d, const std::vector<T> &h, int width = 1) const {
-    std::vector<T> t((size_t)width * cf_ent.size());
-    for (size_t k = 0; k < cf_ent.size(); k++)
-      for (int w = 0; w < width; w++) t[(size_t)width * k + w] = h[(size_t)width * (cf_ent[k] >> 1) + w];
+    std::vector<T> t((size_t)width * cf_off.back());
+    each_entry([&](int k, long long q) {
+      for (int w = 0; w < width; w++) t[(size_t)width * q + w] = h[(size_t)width * (cf_ent[k] >> 1) + w];
+    });
     d.upload(t);
   }
   DBuf<double> d_xf, d_sf, d_area, d_lf, d_vol, d_xc;

@@ -1,0 +1,60 @@
+"""Device layouts of the cell-face entries and of the reduced product's columns."""
+import numpy as np
+import pytest
+
+from mixsolver_amd import meshgen
+from mixsolver_amd.solver import Case
+
+pytestmark = pytest.mark.gpu
+
+CTL = """rho = 1.0
+mu = 0.05
+transient = true
+dt = 0.02
+n_time_max = 3
+n_correct = 2
+time_scheme = 2
+lin_tol = 1e-12
+lin_max = 5000
+conv_blend = 0.5
+nonorth_corr = 1.0
+ppe_precond = jacobi
+gpu_mom_precond = jacobi
+body_force = 1.0 0.0 0.0
+bc = 5 wall
+periodic = 7 6
+periodic = 9 8
+"""
+
+
+def box(nx, ny, nz, copies):
+    """copies periods of an nx-cell period in x"""
+    zid = dict(xmin=6, xmax=7, ymin=5, ymax=5, zmin=8, zmax=9)
+    return meshgen.hex_box(np.linspace(0.0, 1.0 * copies, copies * nx + 1), meshgen.tanh_stretch(ny, 1.1),
+                           np.linspace(0.0, 1.5, nz + 1), zone_ids=zid, jitter=0.1, seed=7, periodic=("x", "z"),
+                           tile_x=nx)
+
+
+@pytest.mark.parametrize("ny,nz", [(6, 2), (6, 3), (8, 4), (9, 8), (13, 5)])
+def test_cells_joined_by_two_faces(ny, nz):
+    """Two cells to a period: each pair shares an interior and a joined face,
+    so one matrix entry takes both.  Two periods have four cells in x and
+    entries of one face each, and the same flow; the systems are solved to
+    1e-12 and six of them follow one another, hence 1e-9.  nz = 2 joins pairs in
+    z as well; the cell counts end within, at and after a slice of 64."""
+    nx = 2
+    rng = np.random.default_rng(11)
+    u1 = rng.uniform(-0.5, 0.5, size=(nz, ny, nx, 3))
+    u1[..., 0] += 1.0
+    res = []
+    for copies in (1, 2):
+        m = box(nx, ny, nz, copies)
+        cs = Case.from_control(m, CTL)
+        cs.set_field("u", np.concatenate([u1] * copies, axis=2).reshape(-1, 3))
+        assert cs.piso_run(3) == 0
+        res.append((cs.get("u").reshape(nz, ny, -1, 3), cs.get("p").reshape(nz, ny, -1)))
+    (ua, pa), (ub, pb) = res
+    assert np.abs(ua - u1).max() > 1e-3
+    for half in (slice(0, nx), slice(nx, 2 * nx)):
+        assert np.abs(ub[:, :, half] - ua).max() < 1e-9 * np.abs(ua).max()
+        assert np.abs(pb[:, :, half] - pa).max() < 1e-9 * np.abs(pa).max()
