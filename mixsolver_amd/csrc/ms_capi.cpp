@@ -609,12 +609,12 @@ int ms_time_kernel(ms_system *h, int which, int reps, double *avg_ms, double *al
     // algorithmic bytes of one SpMV: nnz (value + column index) + one int per row + x and y
     if (alg_bytes) *alg_bytes = (double)P.nnz * (sz + idx) + 4.0 * (P.n + 1) + 2.0 * P.n * sz;
     if (alg_bytes && red && fp32 && K.matfree_on()) {
-      // the matrix-free product: A's nonzeros (FP32 weight + column index)
+      // the matrix-free product: A's nonzeros (FP32 weight + 16-bit column)
       // and one int per row of A, x read by each stage, the colour-0
       // intermediate (h, x_ref) written and read, q written
       const SellPattern &F = *s.P;
       const double n0 = s.schur->n0, n1 = s.schur->n1;
-      *alg_bytes = (double)F.nnz * 4.0 + (F.has16 ? 2.0 * F.nnz + 4.0 * F.nfar : 4.0 * F.nnz) + 4.0 * (F.n + 1) +
+      *alg_bytes = (double)F.nnz * 4.0 + 2.0 * F.nnz + 4.0 * (F.n + 1) +
                    2.0 * n1 * 4.0 +
                    2.0 * n0 * 8.0 + n1 * 4.0;
     }

@@ -44,6 +44,47 @@ __device__ __forceinline__ int col_at(const Mat &A, long long q, int r, int s) {
   }
 }
 
+// Place of slot k of a row (lane of its slice) in the operands of the
+// matrix-free product, within a slice of wd slots: the slots go in groups of
+// four, then two, then one, the members of a group side by side, so a row takes
+// 7 slots in three loads instead of seven (a wavefront's load of any width
+// takes 16 cycles of the address unit).
+__device__ __forceinline__ int mf_pos(int wd, int k, int lane) {
+  const int q4 = wd & ~3, rest = wd - q4;
+  if (k < q4) return 64 * (k & ~3) + 4 * lane + (k & 3);
+  if (rest < 2) return 64 * q4 + lane;
+  return k < q4 + 2 ? 64 * q4 + 2 * lane + (k & 1) : 64 * (q4 + 2) + lane;
+}
+// the slots [0, W) of a row: p its slice's start
+template <int W>
+__device__ __forceinline__ void mf_load(const float *p, int lane, float (&a)[W]) {
+  constexpr int Q = W & ~3, R = W - Q;
+#pragma unroll
+  for (int k = 0; k < Q; k += 4) {
+    const float4 v = *reinterpret_cast<const float4 *>(p + 64 * k + 4 * lane);
+    a[k] = v.x, a[k + 1] = v.y, a[k + 2] = v.z, a[k + 3] = v.w;
+  }
+  if constexpr (R >= 2) {
+    const float2 v = *reinterpret_cast<const float2 *>(p + 64 * Q + 2 * lane);
+    a[Q] = v.x, a[Q + 1] = v.y;
+  }
+  if constexpr (R & 1) a[W - 1] = p[64 * (W - 1) + lane];
+}
+template <int W>
+__device__ __forceinline__ void mf_load(const unsigned short *p, int lane, unsigned (&a)[W]) {
+  constexpr int Q = W & ~3, R = W - Q;
+#pragma unroll
+  for (int k = 0; k < Q; k += 4) {
+    const uint2 v = *reinterpret_cast<const uint2 *>(p + 64 * k + 4 * lane);
+    a[k] = v.x & 0xFFFFu, a[k + 1] = v.x >> 16, a[k + 2] = v.y & 0xFFFFu, a[k + 3] = v.y >> 16;
+  }
+  if constexpr (R >= 2) {
+    const unsigned v = *reinterpret_cast<const unsigned *>(p + 64 * Q + 2 * lane);
+    a[Q] = v & 0xFFFFu, a[Q + 1] = v >> 16;
+  }
+  if constexpr (R & 1) a[W - 1] = p[64 * (W - 1) + lane];
+}
+
 // Row set of a cell-wise kernel: plain blocks of kBlock rows, or (coarse
 // space active) one chunk of rows of a single aggregate per workgroup.
 struct Rows {

@@ -5,17 +5,20 @@
 // (mod_uns_linsolver_mpi.f90: bicgstab_ilu0_mpi :155-229, cg_jacobi_mpi
 // :235-300, cg_ic0_mpi :306-363; factorizations mod_uns_linsolver.f90:79-142
 // and :328-399).  Scalars (alpha, beta, rho, omega, residuals, iteration
-// count, breakdown flags) live in device memory; they are updated by the
-// one-workgroup finisher of each two-stage reduction, so an iteration needs
-// no host round trip.  The host enqueues iterations in chunks and reads the
+// count, breakdown flags) live in device memory; every workgroup of the
+// launch that needs a reduced value sums the partials of the launch before in
+// a fixed order, and one of them keeps the state, so an iteration needs no
+// host round trip.  The host enqueues iterations in chunks and reads the
 // state once per chunk; every iteration kernel returns at once when the
 // state says done.
 //
-// Kernel fusion per PCG iteration (FP64 path):
-//   Jacobi: [q = A p, p.q] [x,r update, r.r, r.(r/d)] [p = r/d + beta p]
-//   DILU  : [q = A p, p.q] [x,r update, r.r, z = r/d on colour 0]
-//           [forward sweeps colours 1..c-1, backward sweeps c-2..0, r.z]
-//           [p = z + beta p]
+// Launches per PCG iteration:
+//   no coarse space, Jacobi: [p = z + beta p, q = A p, p.q] [x,r update, r.r, r.z]
+//   (one launch a solve on small FP64 systems, k_cg_small), and otherwise with
+//   the sweeps and r.z between the two;
+//   coarse space: [q = A p, p.q] (two launches matrix-free) [x,r update, r.r,
+//   r.(r/d), Z^T r] [sweeps of DILU, with nu = E^-1 Z^T r riding the first;
+//   Jacobi: nu in a launch of its own] [p = z + nu + beta p].
 // Vectors are templated on the value type: double for the FP64 path, float
 // for the inner iterations of mixed precision (FP32 products and FP32
 // accumulation of dot-product partials; scalar recurrences in double).
@@ -98,29 +101,45 @@ __device__ __forceinline__ float pu_val(int j, const float *p, const PUp &u, flo
   return p[j];
 }
 
+// 16-bit columns of the product (k_mf_cols).  Its two stages at 2M cells took 10.4
+// and 11.9 us with 32-bit columns and a load per slot, 10.2 and 10.8 so: 52
+// bytes a row instead of 64, but the chain offset - column - gather in the two
+// rounds of workgroups now takes most of it.
+struct MfCols {
+  const unsigned short *c16;
+  const int *win;
+};
+// column of slot code o: w holds window v of the row's slice in lane v + at;
+// every lane of the wavefront takes part
+__device__ __forceinline__ int mf_col(unsigned o, int w, int at, int r) {
+  const int b = __shfl(w, (int)(o >> 12) + at, 64);
+  return o == 0xFFFFu ? r : b + (int)(o & 4095u);
+}
+
 // x_ref (slot 1's column, the row's first colour-1 neighbour) is taken from
-// the columns already loaded, so its gather is issued with the others
-template <int C16, int W, bool PU>
-__device__ __forceinline__ float mf1_row(int k, int s, long long base, int n0, const Mat &A, const float *w,
+// the columns already loaded, so its gather is issued with the others.
+// The diagonal comes first in a colour-0 row: its column is the row's own.
+template <int W, bool PU>
+__device__ __forceinline__ float mf1_row(int k, const unsigned short *c16, int win, const float *w, int n0,
                                          const float *x, float &xr, const PUp &u, float beta, bool up) {
-  int c[W];
+  unsigned o[W];
   float a[W], xv[W];
-  c[0] = k;   // the diagonal comes first in a colour-0 row: its column is not read
+  mf_load<W>(c16, k & 63, o);
+  mf_load<W>(w, k & 63, a);
+  int c[W];
 #pragma unroll
-  for (int j = 1; j < W; j++) c[j] = col_at<C16>(A, base + (long long)j * kSlice, k, s);
+  for (int j = 0; j < W; j++) c[j] = j == 0 ? k : mf_col(o[j], win, 0, k);
 #pragma unroll
-  for (int j = 0; j < W; j++) a[j] = w[base + (long long)j * kSlice];
-#pragma unroll
-  for (int j = 0; j < W; j++) xv[j] = c[j] < n0 ? 0.f : pu_val<PU>(c[j] - n0, x, u, beta, up);
+  for (int j = 0; j < W; j++) xv[j] = j == 0 || c[j] < n0 ? 0.f : pu_val<PU>(c[j] - n0, x, u, beta, up);
   xr = c[1] >= n0 ? xv[1] : 0.f;
   float acc = 0.f;
 #pragma unroll
-  for (int j = 0; j < W; j++) acc = acc + a[j] * (c[j] < n0 ? xr : xr - xv[j]);
+  for (int j = 0; j < W; j++) acc = acc + a[j] * (j == 0 || c[j] < n0 ? xr : xr - xv[j]);
   return acc;
 }
 
-template <int C16, bool PU>
-__global__ void k_mf_stage1(int n0, Mat A, const float *w, const float *x, float2 *hx, KS *st, PUp u) {
+template <bool PU>
+__global__ void k_mf_stage1(int n0, Mat A, MfCols m, const float *w, const float *x, float2 *hx, KS *st, PUp u) {
   if (st->done) return;
   float beta = 0.f;
   bool up = false;
@@ -128,40 +147,44 @@ __global__ void k_mf_stage1(int n0, Mat A, const float *w, const float *x, float
     up = st->pup != 0;
     beta = (float)st->beta;
   }
-  const int k = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-  if (k >= n0) return;
-  const int s = k >> 6;
+  // rows beyond the last repeat it without storing: all lanes pass on windows
+  const int k1 = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x, k = min(k1, n0 - 1);
+  const int s = __builtin_amdgcn_readfirstlane(k >> 6);   // the slice is the wavefront's: scalar loads
   const long long o0 = A.off[s];
   const int wd = (int)((A.off[s + 1] - o0) >> 6);
   const long long base = o0 + (k & 63);
+  const int win = m.win[16 * s + (threadIdx.x & 15)];
+  const bool near16 = m.win[16 * s + 15] != 0;
+  const unsigned short *c16 = m.c16 + o0;
+  const float *ws = w + o0;
   // slot 0 is the diagonal (colour-1 columns are above every colour-0 row)
   float xr = 0.f, acc;
-  if (wd == 7) acc = mf1_row<C16, 7, PU>(k, s, base, n0, A, w, x, xr, u, beta, up);
-  else if (wd == 6) acc = mf1_row<C16, 6, PU>(k, s, base, n0, A, w, x, xr, u, beta, up);
-  else if (wd == 5) acc = mf1_row<C16, 5, PU>(k, s, base, n0, A, w, x, xr, u, beta, up);
+  if (wd == 7 && near16) acc = mf1_row<7, PU>(k, c16, win, ws, n0, x, xr, u, beta, up);
+  else if (wd == 6 && near16) acc = mf1_row<6, PU>(k, c16, win, ws, n0, x, xr, u, beta, up);
+  else if (wd == 5 && near16) acc = mf1_row<5, PU>(k, c16, win, ws, n0, x, xr, u, beta, up);
   else {
-    const int c1 = wd > 1 ? col_at<C16>(A, base + kSlice, k, s) : k;
+    const int c1 = wd > 1 ? A.col[base + kSlice] : k;
     xr = c1 >= n0 ? pu_val<PU>(c1 - n0, x, u, beta, up) : 0.f;
     acc = 0.f;
     for (int j = 0; j < wd; j++) {
-      const long long q = base + (long long)j * kSlice;
-      const int c = col_at<C16>(A, q, k, s);
-      acc = acc + w[q] * (c < n0 ? xr : xr - pu_val<PU>(c - n0, x, u, beta, up));
+      const int c = A.col[base + (long long)j * kSlice];
+      acc = acc + ws[mf_pos(wd, j, k & 63)] * (c < n0 ? xr : xr - pu_val<PU>(c - n0, x, u, beta, up));
     }
   }
-  hx[k] = make_float2(acc, xr);
+  if (k1 < n0) hx[k] = make_float2(acc, xr);
 }
 
-template <int C16, int W>
-__device__ __forceinline__ float mf2_row(int r, int s, long long base, int n0, const Mat &A, const float *w,
+// the last slot is the diagonal of a colour-1 row, or padding
+template <int W>
+__device__ __forceinline__ float mf2_row(int r, const unsigned short *c16, int win, int at, const float *w, int n0,
                                          const float2 *hx, float xi) {
-  int c[W];
+  unsigned o[W];
   float a[W];
-  c[W - 1] = r;   // the last slot is the diagonal of a colour-1 row, or padding
+  mf_load<W>(c16, r & 63, o);
+  mf_load<W>(w, r & 63, a);
+  int c[W];
 #pragma unroll
-  for (int j = 0; j + 1 < W; j++) c[j] = col_at<C16>(A, base + (long long)j * kSlice, r, s);
-#pragma unroll
-  for (int j = 0; j < W; j++) a[j] = w[base + (long long)j * kSlice];
+  for (int j = 0; j < W; j++) c[j] = j + 1 == W ? r : mf_col(o[j], win, at, r);
   float2 h[W];
 #pragma unroll
   for (int j = 0; j < W; j++) h[j] = c[j] < n0 ? hx[c[j]] : make_float2(0.f, 0.f);
@@ -171,9 +194,9 @@ __device__ __forceinline__ float mf2_row(int r, int s, long long base, int n0, c
   return acc;
 }
 
-template <int C16, bool PU>
-__global__ void k_mf_stage2(int n0, int n1, Mat A, const float *w, float *x, const float2 *hx, float *q, KS *st,
-                            float *part, PUp u) {
+template <bool PU>
+__global__ void k_mf_stage2(int n0, int n1, Mat A, MfCols m, const float *w, float *x, const float2 *hx, float *q,
+                            KS *st, float *part, PUp u) {
   if (st->done) return;
   float beta = 0.f;
   bool up = false;
@@ -181,32 +204,43 @@ __global__ void k_mf_stage2(int n0, int n1, Mat A, const float *w, float *x, con
     up = st->pup != 0;
     beta = (float)st->beta;
   }
-  const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  const int i1 = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x, i = min(i1, n1 - 1);
   float v[1] = {0.f};
-  if (i < n1) {
-    const int r = n0 + i, s = r >> 6;
-    const long long o0 = A.off[s];
-    const int wd = (int)((A.off[s + 1] - o0) >> 6);
-    const long long base = o0 + (r & 63);
-    const float xi = pu_val<PU>(i, x, u, beta, up);
-    if (up) x[i] = xi;
-    float acc;
-    if (wd == 7) acc = mf2_row<C16, 7>(r, s, base, n0, A, w, hx, xi);
-    else if (wd == 6) acc = mf2_row<C16, 6>(r, s, base, n0, A, w, hx, xi);
-    else if (wd == 5) acc = mf2_row<C16, 5>(r, s, base, n0, A, w, hx, xi);
-    else {
-      acc = 0.f;
-      for (int j = 0; j < wd; j++) {
-        const long long qq = base + (long long)j * kSlice;
-        const int c = col_at<C16>(A, qq, r, s);
-        if (c < n0) {
-          const float2 h = hx[c];
-          acc = acc + w[qq] * ((xi - h.y) + h.x);
-        } else {
-          acc = acc + w[qq] * xi;
-        }
+  // the rows of a wavefront lie in one slice or two (n0 is not a multiple of
+  // 64): both slices' data come by scalar loads, a row selects its own; the
+  // windows of the second are in lanes 16..31
+  const int r = n0 + i, s0 = __builtin_amdgcn_readfirstlane(r >> 6);
+  const bool first = (r >> 6) == s0;
+  const int s1 = __all(first) ? s0 : s0 + 1;
+  const long long oa = A.off[s0], ob = A.off[s1];
+  const int wa = (int)((A.off[s0 + 1] - oa) >> 6), wb = (int)((A.off[s1 + 1] - ob) >> 6);
+  const int win = m.win[16 * ((threadIdx.x & 16) ? s1 : s0) + (threadIdx.x & 15)], at = first ? 0 : 16;
+  const bool near16 = m.win[16 * s0 + 15] != 0 && m.win[16 * s1 + 15] != 0;
+  const int wd = wa == wb ? wa : 0;
+  const float xi = pu_val<PU>(i, x, u, beta, up);
+  float acc;
+  const long long o0 = first ? oa : ob;
+  const unsigned short *c16 = m.c16 + o0;
+  const float *ws = w + o0;
+  if (wd == 7 && near16) acc = mf2_row<7>(r, c16, win, at, ws, n0, hx, xi);
+  else if (wd == 6 && near16) acc = mf2_row<6>(r, c16, win, at, ws, n0, hx, xi);
+  else if (wd == 5 && near16) acc = mf2_row<5>(r, c16, win, at, ws, n0, hx, xi);
+  else {
+    acc = 0.f;
+    const int wl = first ? wa : wb;
+    for (int j = 0; j < wl; j++) {
+      const int c = A.col[o0 + (long long)j * kSlice + (r & 63)];
+      const float a = ws[mf_pos(wl, j, r & 63)];
+      if (c < n0) {
+        const float2 h = hx[c];
+        acc = acc + a * ((xi - h.y) + h.x);
+      } else {
+        acc = acc + a * xi;
       }
     }
+  }
+  if (i1 < n1) {
+    if (up) x[i] = xi;
     q[i] = acc;
     v[0] = xi * acc;
   }
@@ -1648,24 +1682,19 @@ void Krylov::spmv32(const double *val64, const float *v32, float *p, float *q, K
   if (matfree_on()) {
     const MatFree &M = *mf_;
     const Mat AM = matof(M.A);
+    const MfCols mc{M.c16, M.win};
     const dim3 G0(nblocks(M.n0));
     const PUp u = pu ? *pu : PUp{};
     // stage 1 then stage 2; the start event on the first launch, the stop
     // event on the second
     auto launch = [&](auto k1, auto k2) {
-      if (e0) hipExtLaunchKernelGGL(k1, G0, B, 0, S, e0, nullptr, 0, M.n0, AM, M.w, p, M.hx, st, u);
-      else hipLaunchKernelGGL(k1, G0, B, 0, S, M.n0, AM, M.w, p, M.hx, st, u);
-      if (e1) hipExtLaunchKernelGGL(k2, G, B, 0, S, nullptr, e1, 0, M.n0, M.n1, AM, M.w, p, M.hx, q, st, part, u);
-      else hipLaunchKernelGGL(k2, G, B, 0, S, M.n0, M.n1, AM, M.w, p, M.hx, q, st, part, u);
+      if (e0) hipExtLaunchKernelGGL(k1, G0, B, 0, S, e0, nullptr, 0, M.n0, AM, mc, M.w, p, M.hx, st, u);
+      else hipLaunchKernelGGL(k1, G0, B, 0, S, M.n0, AM, mc, M.w, p, M.hx, st, u);
+      if (e1) hipExtLaunchKernelGGL(k2, G, B, 0, S, nullptr, e1, 0, M.n0, M.n1, AM, mc, M.w, p, M.hx, q, st, part, u);
+      else hipLaunchKernelGGL(k2, G, B, 0, S, M.n0, M.n1, AM, mc, M.w, p, M.hx, q, st, part, u);
     };
-    const bool c16 = M.A->has16;
-    if (pu) {
-      if (c16) launch(k_mf_stage1<1, true>, k_mf_stage2<1, true>);
-      else launch(k_mf_stage1<0, true>, k_mf_stage2<0, true>);
-    } else {
-      if (c16) launch(k_mf_stage1<1, false>, k_mf_stage2<1, false>);
-      else launch(k_mf_stage1<0, false>, k_mf_stage2<0, false>);
-    }
+    if (pu) launch(k_mf_stage1<true>, k_mf_stage2<true>);
+    else launch(k_mf_stage1<false>, k_mf_stage2<false>);
     return;
   }
   const Mat A = matof(pat);

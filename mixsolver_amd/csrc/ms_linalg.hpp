@@ -48,7 +48,7 @@ double time_stream(long long bytes, int kind, int reps);
 // two-colour system (rows [0,n0) colour 0, [n0,n0+n1) colour 1 of the full
 // matrix A), for the FP32 inner iterations of the reduced solve: two
 // launches over A's rows instead of one over the formed S.  w holds, in A's
-// SELL layout, -a_kj / a_kk off the diagonal and (row sum) / a_kk on it for
+// slices and in the order of mf_pos, -a_kj / a_kk off the diagonal and (row sum) / a_kk on it for
 // the colour-0 rows, -a_ij and the row sum for the colour-1 rows; hx holds
 // (h_k, x_ref_k) per colour-0 row between the two launches.
 struct MatFree {
@@ -57,6 +57,8 @@ struct MatFree {
   float *w = nullptr;
   float2 *hx = nullptr;
   const int *agg1 = nullptr;   // aggregate of every colour-1 row (coarse space), for the fused p update
+  const unsigned short *c16 = nullptr;   // A's columns in 16 bits, in w's order (k_mf_cols)
+  const int *win = nullptr;              // their windows, 16 per slice
 };
 // the pending p update p = r/d + nu[agg] + beta p, applied inside the next
 // matrix-free product instead of its own launch (MIXSOLVER_P_FUSED=1;

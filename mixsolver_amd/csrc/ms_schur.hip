@@ -167,8 +167,50 @@ __global__ void k_mf_values(Mat A, const double *val, int n0, int n, float *w) {
     if (k == dk) v = c0 ? (d != 0.0 ? (float)(sum / d) : 0.f) : (float)sum;
     else if (A.col[q] == r) v = 0.f;   // padding
     else v = c0 ? (d != 0.0 ? (float)(-val[q] / d) : 0.f) : (float)(-val[q]);
-    w[q] = v;
+    w[o0 + mf_pos(wd, k, r & 63)] = v;
   }
+}
+
+// Columns of the matrix-free product in 16 bits, one wavefront per slice: up
+// to 15 windows of 4,096 columns, their starts in win[16 s ..], and per slot
+// the window (4 bits) and the place in it (12); 0xFFFF is the row itself
+// (diagonal, padding).  Rows are grouped by aggregate, so a slice's neighbours
+// lie in its own aggregate and a few others, far apart: one 16-bit range per
+// slice or per slot does not reach them.  Windows are laid from the lowest
+// column not yet covered; a slice that needs more keeps the 32-bit columns
+// (win[16 s + 15] = 0, else 1).
+__global__ void k_mf_cols(int nslices, int n, Mat A, unsigned short *c16, int *win) {
+  const int s = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (s >= nslices) return;
+  const int r = s * 64 + lane;
+  const long long o0 = A.off[s];
+  const int wd = (int)((A.off[s + 1] - o0) >> 6);
+  constexpr int kNone = 0x7FFFFFFF;
+  int from = 0, used = 0;   // columns below `from` are covered
+  for (int v = 0; v <= 15; v++) {
+    int lo = kNone;
+    for (int k = 0; k < wd; k++) {
+      const int c = r < n ? A.col[o0 + (long long)k * kSlice + lane] : r;
+      if (c != r && c >= from) lo = min(lo, c);
+    }
+    for (int o = 32; o > 0; o >>= 1) lo = min(lo, __shfl_xor(lo, o, 64));
+    if (lo == kNone) break;
+    used = v + 1;
+    if (v == 15) break;
+    if (lane == 0) win[16 * s + v] = lo;
+    from = lo + 4096;
+    for (int k = 0; k < wd; k++) {
+      const int c = r < n ? A.col[o0 + (long long)k * kSlice + lane] : r;
+      if (c != r && c >= lo && c < from)
+        c16[o0 + mf_pos(wd, k, lane)] = (unsigned short)(v << 12 | (c - lo));
+    }
+  }
+  for (int k = 0; k < wd; k++) {
+    const int c = r < n ? A.col[o0 + (long long)k * kSlice + lane] : r;
+    if (c == r) c16[o0 + mf_pos(wd, k, lane)] = 0xFFFF;
+  }
+  if (lane >= used && lane < 15) win[16 * s + lane] = 0;
+  if (lane == 0) win[16 * s + 15] = used <= 15;
 }
 
 // sum of the workgroup partials on the host, in index order
@@ -235,14 +277,26 @@ void build_schur(System &s, const std::vector<int> &agg_dev, int nagg) {
   S->d.alloc(n1);
   S->r64.alloc(n);
   S->part.alloc(nblocks(n) + 64);
-  attach_matfree(*S, s.P);
+  attach_matfree(*S, s.P, nullptr);
   s.schur = std::move(S);
 }
 
-void attach_matfree(SchurSystem &S, const SellPattern *A) {
+void attach_matfree(SchurSystem &S, const SellPattern *A, const SchurSystem *base) {
   S.mf_w.alloc(A->nstore);
   S.mf_hx.alloc(std::max(S.n0, 1));
-  S.mf = MatFree{S.n0, S.n1, A, S.mf_w.p, S.mf_hx.p, nullptr};
+  S.mf = MatFree{S.n0, S.n1, A, S.mf_w.p, S.mf_hx.p, nullptr, nullptr, nullptr};
+  if (base) {
+    S.mf_c16.alias(base->mf_c16);
+    S.mf_win.alias(base->mf_win);
+  } else {
+    S.mf_c16.alloc(A->nstore);
+    S.mf_win.alloc(16 * (size_t)A->nslices);
+    hipLaunchKernelGGL(k_mf_cols, dim3(nblocks(A->nslices, kBlock / 64)), dim3(kBlock), 0, stream(), A->nslices, A->n,
+                       matof(A), S.mf_c16.p, S.mf_win.p);
+    MS_CHECK_LAUNCH();
+  }
+  S.mf.c16 = S.mf_c16.p;
+  S.mf.win = S.mf_win.p;
   const Coarse &C = S.P->coarse;
   if (C.k > 0) {   // aggregate of every colour-1 row, from the aggregate chunks
     std::vector<int> agg(S.n1, 0);

@@ -1518,7 +1518,7 @@ System *fork_system(System &b, const std::vector<ms_bcgroup_t> &groups) {
     R->d.alloc(R->n1);
     R->r64.alloc(s.nc);
     R->part.alloc(nblocks(s.nc) + 64);
-    attach_matfree(*R, s.P);
+    attach_matfree(*R, s.P, b.schur.get());
     s.schur = std::move(R);
   }
   MS_HIP(hipStreamSynchronize(st));

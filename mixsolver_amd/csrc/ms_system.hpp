@@ -82,6 +82,8 @@ struct SchurSystem {
   // colour-0 intermediate (MatFree)
   DBuf<float> mf_w;
   DBuf<float2> mf_hx;
+  DBuf<unsigned short> mf_c16;
+  DBuf<int> mf_win;   // 16-bit columns and their windows (k_mf_cols)
   DBuf<int> mf_agg;   // aggregate of every colour-1 row (the fused p update)
   MatFree mf;
   std::vector<double> hpart;
@@ -298,8 +300,9 @@ double norm2_ref(const double *v, int n);
 std::vector<int> rcb_aggregates(int n, const std::vector<double> &xc, int k);
 void build_schur(System &s, const std::vector<int> &agg_dev, int nagg);
 // the reduced system's matrix-free S over the full pattern A (buffers and
-// the Krylov hook)
-void attach_matfree(SchurSystem &S, const SellPattern *A);
+// the Krylov hook); base: the reduced system of a forked system's base, whose
+// columns it shares
+void attach_matfree(SchurSystem &S, const SellPattern *A, const SchurSystem *base);
 SolveResult schur_solve(System &s, const double *val, const double *b, double *x, double tol, int maxit, bool mixed,
                         double inner_tol, bool reuse);
 void cell_ordering(int nc, const std::vector<int> &ptr, const std::vector<int> &adj, const std::vector<double> &xc,

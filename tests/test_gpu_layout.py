@@ -58,3 +58,53 @@ def test_cells_joined_by_two_faces(ny, nz):
     for half in (slice(0, nx), slice(nx, 2 * nx)):
         assert np.abs(ub[:, :, half] - ua).max() < 1e-9 * np.abs(ua).max()
         assert np.abs(pb[:, :, half] - pa).max() < 1e-9 * np.abs(pa).max()
+
+
+def channel(nx, ny, nz, **over):
+    ctl = f"""rho = 1.0
+mu = {1.0 / 180.0!r}
+transient = true
+dt = {2 * np.pi / nx / 30!r}
+n_time_max = 1
+n_correct = 2
+time_scheme = 2
+lin_tol = 1e-10
+lin_max = 20000
+ppe_precond = jacobi
+body_force = 1.0 0.0 0.0
+bc = 5 wall
+periodic = 7 6
+periodic = 9 8
+"""
+    m = meshgen.channel(nx, ny, nz, periodic=True)
+    cs = Case.from_control(m, ctl, gpu_ppe_precond=0, gpu_mom_precond=2, gpu_coarse=32, gpu_ppe_solver=2, **over)
+    u = np.random.default_rng(3).uniform(-0.5, 0.5, size=(m.ncells, 3))
+    u[:, 0] += 15.0
+    cs.set_field("u", u)
+    return cs
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(6, 5, 4), (10, 9, 6), (520, 260, 4)])
+def test_reduced_product_columns(nx, ny, nz):
+    """Mixed and FP64 reduced solves of the same p' systems.  The FP32 iterations
+    use the matrix-free product and its 16-bit columns, the FP64 ones the formed
+    matrix.  Few-cell planes put rows of both colours and several planes into a
+    slice; planes of 67,600 rows of a colour, joined to each other's far side,
+    put columns more than 65,535 apart into a slot.  Both solves end at a
+    residual of 1e-10 of the full system; the difference of the fields is that
+    times the condition number, at most 1e4 here, hence 1e-6.  A wrong column
+    would leave the FP32 iterations without convergence: the FP64 iterations
+    stay below a tenth of all."""
+    res = []
+    for prec in (0, 1):
+        cs = channel(nx, ny, nz, gpu_precision=prec)
+        assert cs.piso_run(1) == 0
+        assert np.all(cs.history()[:, 7] <= 1e-10)
+        st = cs.solver_stats()
+        if prec:
+            assert st["ppe_iters_fp64"] <= 0.1 * (st["ppe_iters_fp32"] + st["ppe_iters_fp64"])
+        p = cs.get("p")
+        res.append((cs.get("u"), p - p.mean()))
+    (ua, pa), (ub, pb) = res
+    assert np.abs(ua - ub).max() <= 1e-6 * np.abs(ua).max()
+    assert np.abs(pa - pb).max() <= 1e-6 * np.abs(pa).max()
