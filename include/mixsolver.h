@@ -203,7 +203,11 @@ int ms_periodic_match(int nnodes, const double *x, int nfaces, const long long *
  * (mod_uns_fields.f90:50-71, filled by setup_porous_fields :418-504)
  * "porosity" "perm_dir"(3,nc) "inertial" "disp_l" "disp_t" "bj_alpha" "k_s"
  * "rho_s" "cp_s" "h_sf" "a_sf" "q_src";
- * geometry (read-only): "xf" "sf" "area" "vol" "xc" "lf". */
+ * geometry (read-only): "xf" "sf" "area" "vol" "xc" "lf".
+ * ms_get_field may be called from any number of threads, also while another
+ * thread runs a driver on the same system: it then returns the field as it is
+ * between two of the driver's kernels and leaves the run unchanged.  Other
+ * calls on one system must not overlap. */
 int ms_set_field(ms_system *s, const char *name, const double *host, long long n);
 int ms_get_field(ms_system *s, const char *name, double *host, long long n);
 int ms_set_ts_order(ms_system *s, int ts_order);

@@ -51,6 +51,10 @@ void count_device_bytes(long long delta);
 // that no thread allocates or frees (which may synchronise the device) while
 // another thread captures a graph.
 std::recursive_mutex &device_alloc_mutex();
+// Taken around work that a thread may put on the library stream while another
+// thread drives it, so that none of it lands in the other's capture; no lock on
+// a thread with a stream of its own.
+std::unique_lock<std::recursive_mutex> library_stream_lock();
 // replay the mixed-precision PCG chunk (16 iterations) from a captured HIP
 // graph instead of launching its kernels one by one (default on; the
 // environment variable MIXSOLVER_GRAPHS=0 or ms_set_graphs(0) turns it off)

@@ -7,9 +7,12 @@
 // temporary copy: a 2M-cell velocity field took 15 ms to set and 20 ms to
 // get, now 1.7 and 4.8 ms, of which the copy over PCIe is most.
 //
-// The staging buffer is the face coefficient array af, which every driver and
-// per-call routine forms before it reads it, so it is free between calls and
-// no device memory is held for this.
+// Every transfer has a staging buffer of its own, from a small pool, so a
+// thread that reads fields while another runs the solver, or reads other
+// fields, takes nothing of theirs.  The face and matrix maps are held by the
+// system from their first use (4 bytes per face and direction, 8 per nonzero).
+#include <mutex>
+
 #include "ms_system.hpp"
 
 namespace ms {
@@ -43,28 +46,89 @@ __global__ void k_get_slots(long long m, const long long *slot, const double *sr
   if (t < m) dst[t] = src[slot[t]];
 }
 
+// A device buffer of kStageValues, from the idle ones or new.  It goes back
+// with keep(), once its work has been waited for; a transfer that fails frees
+// it instead, which waits for the device.  At most kIdleStages are kept (64
+// MB).  Never part of a thread's slab, which ends with its owner.
+constexpr long long kStageValues = 1 << 21;
+constexpr size_t kIdleStages = 4;
+std::mutex g_stage_mu;
+std::vector<std::pair<int, double *>> g_idle_stages;   // (device, buffer)
+class Stage {
+ public:
+  Stage() {
+    MS_HIP(hipGetDevice(&dev_));
+    {
+      std::lock_guard<std::mutex> g(g_stage_mu);
+      for (size_t i = 0; i < g_idle_stages.size(); i++)
+        if (g_idle_stages[i].first == dev_) {
+          p = g_idle_stages[i].second;
+          g_idle_stages.erase(g_idle_stages.begin() + i);
+          return;
+        }
+    }
+    std::lock_guard<std::recursive_mutex> g(device_alloc_mutex());
+    if (hipMalloc(&p, kStageValues * sizeof(double)) != hipSuccess) fail(MS_ENOMEM, "hipMalloc failed");
+  }
+  Stage(const Stage &) = delete;
+  Stage &operator=(const Stage &) = delete;
+  void keep() {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    if (g_idle_stages.size() >= kIdleStages) return;
+    g_idle_stages.push_back({dev_, p});
+    p = nullptr;
+  }
+  ~Stage() {
+    if (!p) return;
+    std::lock_guard<std::recursive_mutex> g(device_alloc_mutex());
+    (void)hipFree(p);
+  }
+  double *p = nullptr;
+
+ private:
+  int dev_ = 0;
+};
+
 // the caller's n values in pieces of the staging buffer's size
 template <class Get>
-void pieces_out(System &s, long long n, double *h, Get get) {
-  const long long step = (long long)s.af.n;
-  for (long long e0 = 0; e0 < n; e0 += step) {
-    const long long m = std::min(step, n - e0);
-    get(e0, m);
+void pieces_out(long long n, double *h, Get get) {
+  const auto lk = library_stream_lock();
+  Stage st;
+  for (long long e0 = 0; e0 < n; e0 += kStageValues) {
+    const long long m = std::min(kStageValues, n - e0);
+    get(e0, m, st.p);
     MS_CHECK_LAUNCH();
-    MS_HIP(hipMemcpyAsync(h + e0, s.af.p, m * sizeof(double), hipMemcpyDeviceToHost, stream()));
+    MS_HIP(hipMemcpyAsync(h + e0, st.p, m * sizeof(double), hipMemcpyDeviceToHost, stream()));
     MS_HIP(hipStreamSynchronize(stream()));
   }
+  st.keep();
 }
 template <class Set>
-void pieces_in(System &s, long long n, const double *h, Set set) {
-  const long long step = (long long)s.af.n;
-  for (long long e0 = 0; e0 < n; e0 += step) {
-    const long long m = std::min(step, n - e0);
-    MS_HIP(hipMemcpyAsync(s.af.p, h + e0, m * sizeof(double), hipMemcpyHostToDevice, stream()));
-    set(e0, m);
+void pieces_in(long long n, const double *h, Set set) {
+  const auto lk = library_stream_lock();
+  Stage st;
+  for (long long e0 = 0; e0 < n; e0 += kStageValues) {
+    const long long m = std::min(kStageValues, n - e0);
+    MS_HIP(hipMemcpyAsync(st.p, h + e0, m * sizeof(double), hipMemcpyHostToDevice, stream()));
+    set(e0, m, st.p);
     MS_CHECK_LAUNCH();
     MS_HIP(hipStreamSynchronize(stream()));
   }
+  st.keep();
+}
+// the device copy of a map, made on its first use; calls on one system may come from several threads
+template <class T, class Host>
+const T *map_on_device(System &s, DBuf<T> &d, Host host) {
+  std::lock_guard<std::mutex> g(s.map_mu);
+  if (!d.n) {
+    const std::vector<T> &h = host();
+    const auto lk = library_stream_lock();
+    DBuf<T> t;
+    t.upload(h);
+    MS_HIP(hipStreamSynchronize(stream()));
+    d = std::move(t);
+  }
+  return d.p;
 }
 dim3 grid(long long m) { return dim3((unsigned)((m + kBlock - 1) / kBlock)); }
 
@@ -78,12 +142,13 @@ void cells_out(System &s, const DBuf<double> &buf, int w, double *h) {
   if (buf.n < (size_t)n) fail(MS_EINVAL, "internal: cell array not allocated");
   const double *dev = buf.p;
   if (!s.renumbered) {
+    const auto lk = library_stream_lock();
     MS_HIP(hipMemcpyAsync(h, dev, n * sizeof(double), hipMemcpyDeviceToHost, stream()));
     MS_HIP(hipStreamSynchronize(stream()));
     return;
   }
-  pieces_out(s, n, h, [&](long long e0, long long m) {
-    hipLaunchKernelGGL(k_get_cells, grid(m), dim3(kBlock), 0, stream(), m, e0, w, t.d_o2n.p, dev, s.af.p);
+  pieces_out(n, h, [&](long long e0, long long m, double *stage) {
+    hipLaunchKernelGGL(k_get_cells, grid(m), dim3(kBlock), 0, stream(), m, e0, w, t.d_o2n.p, dev, stage);
   });
 }
 void cells_in(System &s, const double *h, int w, DBuf<double> &buf) {
@@ -92,12 +157,13 @@ void cells_in(System &s, const double *h, int w, DBuf<double> &buf) {
   if (buf.n < (size_t)n) buf.alloc(n);   // zone properties get their arrays when they are set
   double *dev = buf.p;
   if (!s.renumbered) {
+    const auto lk = library_stream_lock();
     MS_HIP(hipMemcpyAsync(dev, h, n * sizeof(double), hipMemcpyHostToDevice, stream()));
     MS_HIP(hipStreamSynchronize(stream()));
     return;
   }
-  pieces_in(s, n, h, [&](long long e0, long long m) {
-    hipLaunchKernelGGL(k_set_cells, grid(m), dim3(kBlock), 0, stream(), m, e0, w, t.d_o2n.p, s.af.p, dev);
+  pieces_in(n, h, [&](long long e0, long long m, const double *stage) {
+    hipLaunchKernelGGL(k_set_cells, grid(m), dim3(kBlock), 0, stream(), m, e0, w, t.d_o2n.p, stage, dev);
   });
 }
 
@@ -107,30 +173,29 @@ void cells_in(System &s, const double *h, int w, DBuf<double> &buf) {
 void faces_out(System &s, const DBuf<double> &buf, double *h) {
   if (buf.n < (size_t)s.nf) fail(MS_EINVAL, "internal: face array not allocated");
   const double *dev = buf.p;
-  if (!s.d_face_get.n) {
+  const int *map = map_on_device(s, s.d_face_get, [&] {
     std::vector<int> idx(s.nf);
     for (int g = 0; g < s.nf; g++) idx[g] = s.shadow[g] >= 0 ? ~s.fo2d[s.shadow[g]] : s.fo2d[g];
-    s.d_face_get.upload(idx);
-    MS_HIP(hipStreamSynchronize(stream()));
-  }
-  pieces_out(s, s.nf, h, [&](long long e0, long long m) {
-    hipLaunchKernelGGL(k_get_faces, grid(m), dim3(kBlock), 0, stream(), m, s.d_face_get.p + e0, dev, s.af.p);
+    return idx;
+  });
+  pieces_out(s.nf, h, [&](long long e0, long long m, double *stage) {
+    hipLaunchKernelGGL(k_get_faces, grid(m), dim3(kBlock), 0, stream(), m, map + e0, dev, stage);
   });
 }
 void faces_in(System &s, const double *h, DBuf<double> &buf) {
   if (buf.n < (size_t)s.nf) buf.alloc(s.nf);
   double *dev = buf.p;
-  if (!s.d_fo2d.n) s.d_fo2d.upload(s.fo2d);
-  pieces_in(s, s.nf, h, [&](long long e0, long long m) {
-    hipLaunchKernelGGL(k_set_faces, grid(m), dim3(kBlock), 0, stream(), m, s.d_fo2d.p + e0, s.af.p, dev);
+  const int *map = map_on_device(s, s.d_fo2d, [&]() -> const std::vector<int> & { return s.fo2d; });
+  pieces_in(s.nf, h, [&](long long e0, long long m, const double *stage) {
+    hipLaunchKernelGGL(k_set_faces, grid(m), dim3(kBlock), 0, stream(), m, map + e0, stage, dev);
   });
 }
 
 // the matrix in the caller's CSR order
 void matrix_values_out(System &s, double *h) {
-  if (!s.d_ref2dev.n) s.d_ref2dev.upload(s.ref2dev);
-  pieces_out(s, (long long)s.ref2dev.size(), h, [&](long long e0, long long m) {
-    hipLaunchKernelGGL(k_get_slots, grid(m), dim3(kBlock), 0, stream(), m, s.d_ref2dev.p + e0, s.val.p, s.af.p);
+  const long long *map = map_on_device(s, s.d_ref2dev, [&]() -> const std::vector<long long> & { return s.ref2dev; });
+  pieces_out((long long)s.ref2dev.size(), h, [&](long long e0, long long m, double *stage) {
+    hipLaunchKernelGGL(k_get_slots, grid(m), dim3(kBlock), 0, stream(), m, map + e0, s.val.p, stage);
   });
 }
 

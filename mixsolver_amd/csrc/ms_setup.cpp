@@ -119,6 +119,10 @@ std::recursive_mutex &device_alloc_mutex() {
   static std::recursive_mutex m;
   return m;
 }
+std::unique_lock<std::recursive_mutex> library_stream_lock() {
+  if (t_stream) return {};
+  return std::unique_lock<std::recursive_mutex>(device_alloc_mutex());
+}
 int runtime_device() { return g_device; }
 long long thread_device_bytes() { return t_dev_bytes; }
 void count_device_bytes(long long delta) { t_dev_bytes += delta; }

@@ -158,7 +158,8 @@ struct System {
   DBuf<int> d_c0, d_c1, d_fgrp, d_cf_len, d_cf_ent;
   DBuf<long long> d_cf_off, d_cf_slot, d_diag_slot;
   // numbering maps of the API boundary (ms_io.hip): cells (renumbered systems),
-  // faces and matrix slots (uploaded on first use)
+  // faces and matrix slots (uploaded on first use, under map_mu)
+  std::mutex map_mu;
   DBuf<int> d_o2n, d_fo2d, d_face_get;
   DBuf<long long> d_ref2dev;
   DBuf<int> d_e_oth;
@@ -266,7 +267,8 @@ void periodic_match(int nnodes, const double *x, int nfaces, const long long *fp
                     const int *c0, const int *c1, const int *zone, int ncells, const ms_ctrl_t *ctrl, int *partner);
 
 // Arrays across the API boundary, natural order on the host and device order
-// on the device (ms_io.hip); they use af as staging and return synchronised.
+// on the device (ms_io.hip); they return synchronised and share nothing with
+// the solver, so one thread may read while another runs a driver.
 void cells_out(System &s, const DBuf<double> &buf, int w, double *h);
 void cells_in(System &s, const double *h, int w, DBuf<double> &buf);
 void faces_out(System &s, const DBuf<double> &buf, double *h);
