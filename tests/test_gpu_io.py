@@ -58,3 +58,43 @@ def test_matrix_of_a_renumbered_system():
         cs.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 12), (32, 16, 16), (34, 18, 16), (64, 32, 16)])
+def test_fields_on_both_sides_of_the_host_route(shape):
+    """Arrays of up to 32,768 values are reordered on the host, larger ones on
+    the device: 3,072 to 32,768 cells of one, three and nine values (32,768
+    among the sizes) and 9,000 to 100,000 faces."""
+    m = meshgen.channel(*shape, periodic=True)
+    rng = np.random.default_rng(3)
+    dev = Case.from_control(m, CTL + "periodic = 7 6\nperiodic = 9 8\n", gpu_ppe_precond=2, gpu_mom_precond=2)
+    assert dev.info["renumbered"]
+    vals = {k: rng.normal(size=m.ncells * n) for k, n in dict(u=3, p=1, gu=9, T=1, disp_l=1, perm_dir=3).items()}
+    for k, v in vals.items():
+        dev.set_field(k, v)
+    for k, v in vals.items():
+        assert np.array_equal(np.ravel(dev.get(k)), v), k
+    flux = rng.normal(size=m.nfaces)
+    dev.set_field("flux", flux)
+    got, inner = dev.get("flux"), m.c1 > 0
+    assert np.array_equal(got[inner], flux[inner])
+    for a, b in ((7, 6), (9, 8)):
+        assert np.array_equal(np.sort(got[m.zone == a]), np.sort(-got[m.zone == b]))
+    dev.close()
+
+
+def test_matrix_values_reordered_on_the_device():
+    """A matrix of 59,000 entries, beyond what the host reorders."""
+    m = meshgen.channel(24, 20, 18)
+    ctl = CTL + "bc = 6 velocity-inlet 1.0 0.0 0.0\nbc = 7 pressure-outlet 0.0\nbc = 4 symmetry\n"
+    u = np.random.default_rng(4).normal(size=(m.ncells, 3))
+    out = []
+    for over in ({}, dict(gpu_ppe_precond=2, gpu_mom_precond=2)):
+        cs = Case.from_control(m, ctl, **over)
+        cs.set_field("u", u)
+        cs.compute_gradients()
+        cs.flux_rhiechow()
+        out.append(cs.momentum_assembly(1) + cs.ppe_assembly() + (cs.get("flux"),))
+        cs.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
