@@ -37,12 +37,6 @@ int runtime_device();            // device selected by ensure_runtime (-1 before
 // launches and synchronises there.  Default priority; nullptr restores the
 // library stream.
 void set_thread_stream(hipStream_t s);
-// Streams of worker threads, kept for the next ones (a stream takes
-// milliseconds to create and to destroy): at most kIdleStreams idle ones, each
-// given back when its thread is done with it and has waited for its work.
-constexpr int kIdleStreams = 16;
-hipStream_t borrow_stream();          // nullptr on failure
-void give_back_stream(hipStream_t s);
 // device bytes allocated minus freed by DBuf on the calling thread (the
 // sweep server measures a case's footprint with it)
 long long thread_device_bytes();

@@ -64,36 +64,6 @@ hipStream_t stream() {
 }
 void set_thread_stream(hipStream_t s) { t_stream = s; }
 
-static std::mutex g_idle_mu;
-static std::vector<std::pair<int, hipStream_t>> g_idle_streams;   // (device, stream)
-hipStream_t borrow_stream() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  {
-    std::lock_guard<std::mutex> g(g_idle_mu);
-    for (size_t i = 0; i < g_idle_streams.size(); i++)
-      if (g_idle_streams[i].first == dev) {
-        hipStream_t s = g_idle_streams[i].second;
-        g_idle_streams.erase(g_idle_streams.begin() + i);
-        return s;
-      }
-  }
-  hipStream_t s = nullptr;
-  return hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess ? s : nullptr;
-}
-void give_back_stream(hipStream_t s) {
-  int dev = 0;
-  const bool ok = hipStreamSynchronize(s) == hipSuccess && hipGetDevice(&dev) == hipSuccess;
-  if (ok) {
-    std::lock_guard<std::mutex> g(g_idle_mu);
-    if ((int)g_idle_streams.size() < kIdleStreams) {
-      g_idle_streams.push_back({dev, s});
-      return;
-    }
-  }
-  (void)hipStreamDestroy(s);
-}
-
 static thread_local Slab *t_slab = nullptr;
 Slab *thread_slab() { return t_slab; }
 void set_thread_slab(Slab *s) { t_slab = s; }
