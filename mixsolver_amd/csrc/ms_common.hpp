@@ -8,6 +8,8 @@
 #include <string>
 #include <vector>
 
+#include "ms_sweep_plan.hpp"
+
 #include "../../include/mixsolver.h"
 
 namespace ms {
@@ -166,9 +168,6 @@ struct DBuf {
 };
 
 constexpr int kBlock = 256;   // 4 wave64 per workgroup
-constexpr int kSlice = 64;    // SELL slice height = one wavefront
-constexpr int kSegThreads = 1024;   // workgroup of a run of narrow levels
-constexpr int kNarrowRows = 2048;   // widest level such a run takes
 
 inline int nblocks(long long n, int b = kBlock) { return (int)((n + b - 1) / b); }
 
@@ -216,14 +215,6 @@ struct CoarseMat {
 };
 
 // ------------------------------------------------------ level schedules
-// One step of the workgroup that walks a run of narrow levels (ms_levels.hip):
-// rows [t0, t0 + n) of the level order, entry k of its lane t at
-// base + k * roundup(n, 64) + t, w entries at most; near: all
-// neighbours of its rows are in the workgroup's ring (1), or not (0)
-struct SweepStep {
-  int t0, n, w, near;
-  long long base;
-};
 struct SweepPlan {
   int nsteps = 0;
   int width = 0;       // entries per row of every step (more: rows beyond the width fetched ahead exist)
@@ -259,17 +250,11 @@ struct SellPattern {
   std::vector<int> lev_ptr_f, lev_ptr_b;   // rows grouped per level
   DBuf<int> d_lev_rows_f, d_lev_rows_b, d_lev_ptr_f, d_lev_ptr_b;
   // launch plan of a sweep: runs of consecutive narrow levels (at most
-  // kNarrowRows rows each) go to one workgroup that steps through them
-  // (steps [s0, s1), positions from t0 on, `block` threads); every wider
-  // level is a launch of its own
-  struct LevSeg {
-    int l0, l1;
-    bool narrow;
-    int s0 = 0, s1 = 0, t0 = 0, block = kSegThreads;
-    SweepStep step{};   // a wide level's
-  };
+  // kNarrowRows rows each) go to one workgroup that steps through them; every
+  // wider level is a launch of its own
   std::vector<LevSeg> seg_f, seg_b;
   SweepPlan sweep_f, sweep_b;
+  bool sweep_packed = false;    // the sweeps read packed copies of the factor (sweep_packs)
   bool triangle_free = false;   // no two neighbours share a neighbour (set with the levels)
   bool sweep_ordered = false;   // one run each way, vectors in level order (d_lev_fb: forward position of a backward one)
   DBuf<int> d_lev_fb;

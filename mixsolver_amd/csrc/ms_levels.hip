@@ -121,6 +121,80 @@ __global__ __launch_bounds__(kSegThreads) void k_factor_seg(const int *lev_ptr, 
   }
 }
 
+// --------------------------------------------------------- unpacked sweeps
+// Patterns that are not packed (sweep_packs): the same two launch forms, from
+// the factor in the matrix's own layout.
+
+// forward substitution of row i (unit lower for ILU(0), L of IC(0))
+template <class T>
+__device__ void lower_row(int i, const LMat &A, const T *F, const T *r, T *z, int ic0) {
+  const long long bi = A.off[i >> 6] + (i & 63);
+  const int dpi = A.diagk[i];
+  T s = r[i];
+  for (int k = 0; k < dpi; k++) {
+    const long long q = bi + (long long)k * kSlice;
+    s = s - F[q] * z[A.col[q]];
+  }
+  z[i] = ic0 ? s / F[bi + (long long)dpi * kSlice] : s;
+}
+
+// backward substitution of row i (U of ILU(0), L^T of IC(0) via tpos)
+template <class T>
+__device__ void upper_row(int i, const LMat &A, const long long *tpos, const T *F, T *z, int ic0) {
+  const long long bi = A.off[i >> 6] + (i & 63);
+  const int dpi = A.diagk[i], len = A.rowlen[i];
+  T s = z[i];
+  if (ic0) {
+    for (int k = len - 1; k > dpi; k--) {
+      const long long q = bi + (long long)k * kSlice;
+      s = s - F[tpos[q]] * z[A.col[q]];
+    }
+  } else {
+    for (int k = dpi + 1; k < len; k++) {
+      const long long q = bi + (long long)k * kSlice;
+      s = s - F[q] * z[A.col[q]];
+    }
+  }
+  z[i] = s / F[bi + (long long)dpi * kSlice];
+}
+
+template <class T>
+__global__ void k_lower_level(const int *rows, int nr, LMat A, const T *F, const T *r, T *z, int ic0,
+                              const int *done) {
+  if (*done) return;
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < nr) lower_row(rows[t], A, F, r, z, ic0);
+}
+template <class T>
+__global__ void k_upper_level(const int *rows, int nr, LMat A, const long long *tpos, const T *F, T *z, int ic0,
+                              const int *done) {
+  if (*done) return;
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < nr) upper_row(rows[t], A, tpos, F, z, ic0);
+}
+template <class T>
+__global__ __launch_bounds__(kSegThreads) void k_lower_seg(const int *lev_ptr, int l0, int l1, const int *rows,
+                                                           LMat A, const T *F, const T *r, T *z, int ic0,
+                                                           const int *done) {
+  if (*done) return;
+  for (int l = l0; l < l1; l++) {
+    const int a = lev_ptr[l], b = lev_ptr[l + 1];
+    for (int t = a + (int)threadIdx.x; t < b; t += kSegThreads) lower_row(rows[t], A, F, r, z, ic0);
+    __syncthreads();
+  }
+}
+template <class T>
+__global__ __launch_bounds__(kSegThreads) void k_upper_seg(const int *lev_ptr, int l0, int l1, const int *rows,
+                                                           LMat A, const long long *tpos, const T *F, T *z, int ic0,
+                                                           const int *done) {
+  if (*done) return;
+  for (int l = l0; l < l1; l++) {
+    const int a = lev_ptr[l], b = lev_ptr[l + 1];
+    for (int t = a + (int)threadIdx.x; t < b; t += kSegThreads) upper_row(rows[t], A, tpos, F, z, ic0);
+    __syncthreads();
+  }
+}
+
 // ------------------------------------------------------------ packed sweeps
 // One workgroup steps through a run of narrow levels.  A step is a level, or
 // a part of at most kSegThreads rows of a wider one; a row's place in the
@@ -144,11 +218,8 @@ __global__ __launch_bounds__(kSegThreads) void k_factor_seg(const int *lev_ptr, 
 // 0.25 us a level where the level is its latency, about 45 GB/s where it is
 // wide, which is what one compute unit draws.
 constexpr int kRing = 16384;   // positions kept in LDS (128 KB in FP64)
-constexpr int kPre = 4;        // most entries per row that are fetched ahead (hexahedra 3, prisms 2-3)
 constexpr int kOrderedBlock = 512;   // widest level (in whole wavefronts) from which vectors go in level order
 constexpr int kAheadRows = 3, kAheadOrdered = 4;   // steps fetched ahead (vectors in row order / level order)
-
-constexpr int kTailSteps = 6;  // empty steps after the last, so that fetching ahead needs no bound
 
 // LDS only: a release of the ring's writes, no wait for loads or stores in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -184,7 +255,7 @@ __global__ __launch_bounds__(kSegThreads) void k_sweep_seg(const SweepStep *__re
   // not queue behind the fetches
   typedef const __attribute__((address_space(4))) SweepStep *StepPtr;
   const StepPtr sp = (StepPtr)(unsigned long long)steps;
-  auto desc = [&](int s) { return SweepStep{sp[s].t0, sp[s].n, sp[s].w, sp[s].near, sp[s].base}; };
+  auto desc = [&](int s) { return SweepStep{sp[s].t0, sp[s].n, sp[s].w, sp[s].near, sp[s].base, sp[s].stride}; };
   // the loads of lanes beyond a step's rows go to its last row: no branch
   // around them, so nothing waits for them before their step
   auto lane = [&](const SweepStep &d) { return (unsigned)min(t, max(d.n, 1) - 1); };
@@ -193,7 +264,7 @@ __global__ __launch_bounds__(kSegThreads) void k_sweep_seg(const SweepStep *__re
   // four SIMDs)
   auto fetch = [&](Ahead<T, W> &a, const SweepStep &d, int row) {
     const unsigned l = lane(d);
-    const int stride = (d.n + 63) & ~63;
+    const int stride = d.stride;
     const int *pc = pcol + d.base;
     const T *pv = pval + d.base;
     const T *pw = FAC == 1 ? pval2 + d.base : nullptr;
@@ -248,7 +319,7 @@ __global__ __launch_bounds__(kSegThreads) void k_sweep_seg(const SweepStep *__re
     if (!near && lo > seg0) __syncthreads();
     auto solve = [&](auto get) {
       T sum = p.rhs;
-      const int stride = (e.n + 63) & ~63;
+      const int stride = e.stride;
       if (MORE && DESC)
         for (int k = e.w - 1; k >= W; k--) {
           const long long q = e.base + (long long)k * stride + t;
@@ -316,7 +387,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep_wide(SweepStep d, const int *_
                                                        const int *done) {
   const int dn = *done, t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= d.n) return;
-  const int stride = (d.n + 63) & ~63;
+  const int stride = d.stride;
   const int row = rows[d.t0 + t];
   int c[W];
   T v[W], z[W];
@@ -353,7 +424,7 @@ __global__ __launch_bounds__(kBlock) void k_diag_wide(SweepStep d, const int *ro
                                                       double *out, int *flag) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= d.n) return;
-  const int stride = (d.n + 63) & ~63;
+  const int stride = d.stride;
   double sum = pdiag[d.t0 + t];
   for (int k = 0; k < d.w; k++) {
     const long long q = d.base + (long long)k * stride + t;
@@ -411,7 +482,7 @@ __global__ void k_find_triangle(int n, LMat A, int *found) {
 __global__ void k_pack_cols_wide(SweepStep d, const int *rows, LMat A, int upper, int *pcol) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= d.n) return;
-  const int stride = (d.n + 63) & ~63;
+  const int stride = d.stride;
   const int r = rows[d.t0 + t], dk = A.diagk[r];
   const long long br = A.off[r >> 6] + (r & 63);
   const int k0 = upper ? dk + 1 : 0, m = upper ? A.rowlen[r] - dk - 1 : dk;
@@ -425,7 +496,7 @@ __global__ void k_pack_cols_wide(SweepStep d, const int *rows, LMat A, int upper
 __global__ void k_pack_cols(SweepStep *steps, int seg0, const int *rows, const int *pos, LMat A, int upper,
                             int *pcol) {
   const SweepStep d = steps[blockIdx.x];
-  const int stride = (d.n + 63) & ~63;
+  const int stride = d.stride;
   __shared__ int far;
   if (threadIdx.x == 0) far = 0;
   __syncthreads();
@@ -454,7 +525,7 @@ template <class T>
 __global__ void k_pack_vals(const SweepStep *steps, const int *rows, LMat A, int upper, const long long *tpos,
                             const T *F, T *pval, T *pdiag) {
   const SweepStep d = steps[blockIdx.x];
-  const int stride = (d.n + 63) & ~63;
+  const int stride = d.stride;
   for (int t = blockIdx.y * kBlock + threadIdx.x; t < d.n; t += kBlock * gridDim.y) {
     const int r = rows[d.t0 + t], dk = A.diagk[r];
     const long long br = A.off[r >> 6] + (r & 63);
@@ -485,52 +556,26 @@ __global__ void k_scatter(int n, const int *idx, const T *in, T *out, const int 
 
 // The steps of every run of narrow levels, and their packed columns.
 void plan_sweeps(SellPattern &P, const std::vector<int> &rows_f, const std::vector<int> &rows_b) {
-  std::vector<int> pos_f(P.n);
-  for (int t = 0; t < P.n; t++) pos_f[rows_f[t]] = t;
-  auto plan = [&](bool upper, const std::vector<int> &lev, const std::vector<int> &rows,
-                  std::vector<SellPattern::LevSeg> &segs, SweepPlan &S, const DBuf<int> &d_rows) {
-    std::vector<SweepStep> st;
-    long long base = 0;
-    int widest_row = 1;
-    for (int r = 0; r < P.n; r++)
-      widest_row = std::max(widest_row, upper ? P.rowlen[r] - P.diagk[r] - 1 : P.diagk[r]);
-    S.width = std::min(widest_row, kPre);
-    S.more = widest_row > kPre;
-    auto add = [&](int t, int n) {
-      SweepStep d{t, n, S.width, 0, base};
-      for (int i = 0; S.more && i < n; i++) {
-        const int r = rows[t + i];
-        d.w = std::max(d.w, upper ? P.rowlen[r] - P.diagk[r] - 1 : P.diagk[r]);
-      }
-      base += (long long)d.w * ((n + 63) & ~63);
-      st.push_back(d);
-    };
-    for (auto &g : segs) {
-      g.s0 = (int)st.size();
-      g.t0 = lev[g.l0];
-      if (!g.narrow) {
-        add(g.t0, lev[g.l1] - g.t0);
-        g.s1 = (int)st.size();
-        g.step = st.back();
-        continue;
-      }
-      int widest = 1;
-      for (int l = g.l0; l < g.l1; l++) widest = std::max(widest, lev[l + 1] - lev[l]);
-      g.block = std::min(kSegThreads, (widest + kSlice - 1) / kSlice * kSlice);
-      for (int l = g.l0; l < g.l1; l++)
-        for (int t = lev[l]; t < lev[l + 1]; t += g.block) add(t, std::min(g.block, lev[l + 1] - t));
-      g.s1 = (int)st.size();
-      for (int i = 0; i < kTailSteps; i++) st.push_back(SweepStep{0, 0, 0, 0, 0});
-    }
-    S.nent = base;
-    S.nsteps = (int)st.size();
+  const SweepSteps F = sweep_steps(P.lev_ptr_f, P.seg_f, [&](int t) { return P.diagk[rows_f[t]]; });
+  const SweepSteps B = sweep_steps(P.lev_ptr_b, P.seg_b, [&](int t) {
+    return P.rowlen[rows_b[t]] - P.diagk[rows_b[t]] - 1;
+  });
+  P.sweep_packed = sweep_packs(F.nent + B.nent, P.nstore);
+  P.triangle_free = P.sweep_ordered = false;
+  if (!P.sweep_packed) return;
+  auto plan = [&](bool upper, const SweepSteps &H, const std::vector<int> &rows, const std::vector<LevSeg> &segs,
+                  SweepPlan &S, const DBuf<int> &d_rows) {
+    S.width = H.width;
+    S.more = H.more;
+    S.nent = H.nent;
+    S.nsteps = (int)H.st.size();
     if (!S.nsteps) return;
     std::vector<int> pos(P.n);
     for (int t = 0; t < P.n; t++) pos[rows[t]] = t;
     DBuf<int> d_pos;
     d_pos.upload(pos);
-    S.steps.upload(st);
-    S.col.alloc(std::max<long long>(base, 1));
+    S.steps.upload(H.st);
+    S.col.alloc(std::max<long long>(S.nent, 1));
     for (const auto &g : segs)
       if (g.narrow)
         hipLaunchKernelGGL(k_pack_cols, dim3(g.s1 - g.s0), dim3(kBlock), 0, stream(), S.steps.p + g.s0, g.t0,
@@ -541,8 +586,8 @@ void plan_sweeps(SellPattern &P, const std::vector<int> &rows_f, const std::vect
     MS_CHECK_LAUNCH();
     MS_HIP(hipStreamSynchronize(stream()));   // the host arrays above and d_pos go out of scope
   };
-  plan(false, P.lev_ptr_f, rows_f, P.seg_f, P.sweep_f, P.d_lev_rows_f);
-  plan(true, P.lev_ptr_b, rows_b, P.seg_b, P.sweep_b, P.d_lev_rows_b);
+  plan(false, F, rows_f, P.seg_f, P.sweep_f, P.d_lev_rows_f);
+  plan(true, B, rows_b, P.seg_b, P.sweep_b, P.d_lev_rows_b);
   // Vectors in level order: the rows of a level are far apart in row order
   // (a diagonal plane of a grid), so reading and writing them there costs
   // the one workgroup a cache line per row, 150 us per sweep against 84
@@ -560,7 +605,8 @@ void plan_sweeps(SellPattern &P, const std::vector<int> &rows_f, const std::vect
   P.sweep_ordered = P.seg_f.size() == 1 && P.seg_b.size() == 1 && P.seg_f[0].narrow && P.seg_b[0].narrow &&
                     P.seg_f[0].block >= kOrderedBlock;
   if (P.sweep_ordered) {
-    std::vector<int> fb(P.n);
+    std::vector<int> pos_f(P.n), fb(P.n);
+    for (int t = 0; t < P.n; t++) pos_f[rows_f[t]] = t;
     for (int t = 0; t < P.n; t++) fb[t] = pos_f[rows_b[t]];
     P.d_lev_fb.upload(fb);
     MS_HIP(hipStreamSynchronize(stream()));
@@ -570,6 +616,7 @@ void plan_sweeps(SellPattern &P, const std::vector<int> &rows_f, const std::vect
 // the factor F (SELL layout) in the order of the packed sweeps
 template <class T>
 void LevelFactor<T>::pack(const SellPattern &P, const T *F, bool ic0) {
+  if (!P.sweep_packed) return;
   auto one = [&](const SweepPlan &S, const DBuf<int> &rows, DBuf<T> &v, DBuf<T> &d, bool upper) {
     if (!S.nsteps) return;
     if (v.n < (size_t)S.nent) v.alloc(S.nent);
@@ -587,7 +634,7 @@ void LevelFactor<T>::pack(const SellPattern &P, const T *F, bool ic0) {
 }
 
 template <class T, bool DIV, bool DESC>
-static void sweep_run(const SweepPlan &S, const SellPattern::LevSeg &g, const int *rows, const T *v, const T *d,
+static void sweep_run(const SweepPlan &S, const LevSeg &g, const int *rows, const T *v, const T *d,
                       const T *in, T *out, const int *done) {
   auto go = [&](auto k) {
     hipLaunchKernelGGL(k, dim3(1), dim3(g.block), 0, stream(), S.steps.p + g.s0, g.s1 - g.s0, g.t0, rows, S.col.p, v,
@@ -606,7 +653,7 @@ static void sweep_run(const SweepPlan &S, const SellPattern::LevSeg &g, const in
 }
 
 template <class T, bool DIV, bool DESC>
-static void sweep_wide(const SweepPlan &S, const SellPattern::LevSeg &g, const int *rows, const T *v, const T *d,
+static void sweep_wide(const SweepPlan &S, const LevSeg &g, const int *rows, const T *v, const T *d,
                        const T *in, T *out, const int *done) {
   auto go = [&](auto k) {
     hipLaunchKernelGGL(k, dim3(nblocks(g.step.n)), dim3(kBlock), 0, stream(), g.step, rows, S.col.p, v, d, in, out,
@@ -621,14 +668,37 @@ static void sweep_wide(const SweepPlan &S, const SellPattern::LevSeg &g, const i
 
 // out = (L U)^-1 in or (L L^T)^-1 in
 template <class T>
-void LevelFactor<T>::apply(const SellPattern &P, bool ic0, const T *in, T *out, const int *done) {
+void LevelFactor<T>::apply(const SellPattern &P, bool ic0, const T *F, const T *in, T *out, const int *done) {
   hipStream_t S = stream();
   const dim3 G(nblocks(P.n)), B(kBlock);
-  auto fwd = [&](const SellPattern::LevSeg &g, const int *rows, const T *x, T *y) {
+  if (!P.sweep_packed) {
+    const LMat A = lmat(P);
+    for (const auto &g : P.seg_f) {
+      const int a = P.lev_ptr_f[g.l0], m = P.lev_ptr_f[g.l1] - a;
+      if (g.narrow)
+        hipLaunchKernelGGL(k_lower_seg<T>, dim3(1), dim3(kSegThreads), 0, S, P.d_lev_ptr_f.p, g.l0, g.l1,
+                           P.d_lev_rows_f.p, A, F, in, out, (int)ic0, done);
+      else
+        hipLaunchKernelGGL(k_lower_level<T>, dim3(nblocks(m)), B, 0, S, P.d_lev_rows_f.p + a, m, A, F, in, out,
+                           (int)ic0, done);
+    }
+    for (const auto &g : P.seg_b) {
+      const int a = P.lev_ptr_b[g.l0], m = P.lev_ptr_b[g.l1] - a;
+      if (g.narrow)
+        hipLaunchKernelGGL(k_upper_seg<T>, dim3(1), dim3(kSegThreads), 0, S, P.d_lev_ptr_b.p, g.l0, g.l1,
+                           P.d_lev_rows_b.p, A, P.d_tpos.p, F, out, (int)ic0, done);
+      else
+        hipLaunchKernelGGL(k_upper_level<T>, dim3(nblocks(m)), B, 0, S, P.d_lev_rows_b.p + a, m, A, P.d_tpos.p, F,
+                           out, (int)ic0, done);
+    }
+    MS_CHECK_LAUNCH();
+    return;
+  }
+  auto fwd = [&](const LevSeg &g, const int *rows, const T *x, T *y) {
     if (ic0) sweep_run<T, true, false>(P.sweep_f, g, rows, vf.p, df.p, x, y, done);
     else sweep_run<T, false, false>(P.sweep_f, g, rows, vf.p, df.p, x, y, done);
   };
-  auto bwd = [&](const SellPattern::LevSeg &g, const int *rows, const T *x, T *y) {
+  auto bwd = [&](const LevSeg &g, const int *rows, const T *x, T *y) {
     if (ic0) sweep_run<T, true, true>(P.sweep_b, g, rows, vb.p, db.p, x, y, done);
     else sweep_run<T, true, false>(P.sweep_b, g, rows, vb.p, db.p, x, y, done);
   };

@@ -1862,8 +1862,8 @@ void Krylov::apply_pc(PcKind pc, const T *val, const T *fac, const T *dg, const 
           hipLaunchKernelGGL((k_dilu_bwd<T, 0>), dim3(nblocks(cp[c + 1] - cp[c])), dim3(kBlock), 0, stream(), cp[c],
                              cp[c + 1], A, val, dg, in, out, done, (T *)nullptr);
   } else {
-    if constexpr (sizeof(T) == 8) lev_.apply(*pat, pc == PC_NATURAL_IC0, in, out, done);
-    else lev32_.apply(*pat, pc == PC_NATURAL_IC0, in, out, done);
+    if constexpr (sizeof(T) == 8) lev_.apply(*pat, pc == PC_NATURAL_IC0, fac, in, out, done);
+    else lev32_.apply(*pat, pc == PC_NATURAL_IC0, fac, in, out, done);
   }
   MS_CHECK_LAUNCH();
 }

@@ -88,7 +88,8 @@ struct LevelFactor {
   DBuf<T> vf, vb, df, db;   // forward / backward entries and diagonals, step order
   void pack(const SellPattern &P, const T *F, bool ic0);
   DBuf<T> xf, xb;           // vectors in level order (SellPattern::sweep_ordered)
-  void apply(const SellPattern &P, bool ic0, const T *in, T *out, const int *done);
+  // F: the factor in the matrix's layout, read where it is not packed
+  void apply(const SellPattern &P, bool ic0, const T *F, const T *in, T *out, const int *done);
 };
 struct DiagFactor {   // work arrays of factor_levels: entries and diagonal in step order, factor's diagonal
   DBuf<double> lo, up, dg, d;
