@@ -342,6 +342,24 @@ __device__ __forceinline__ void cg_sums(int n1, const T *p1, int n2, const T *p2
   block_reduce<OpSum, 2, T, kBlock>(a, lds);
 }
 
+// Partials too many for every workgroup of the next launch to add up, to
+// kFoldParts (two arrays with grid.y = 2): a launch of 4.6 us against reads
+// that every workgroup repeats at some 15 TB/s out of the L2s, so worth it
+// above kFoldBytes.  DILU sweeps over 2M rows leave 7,813 for the 2,048
+// workgroups of k_cg_ps: 47.8 us after folding, 54.9 without, and an iteration
+// takes 114 us of kernels (118 in the seven launches of a finisher each).
+constexpr int kFoldParts = 64;
+constexpr long long kFoldBytes = 64LL << 20;
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_fold_parts(int n, const T *a, const T *b, T *out, const KS *st) {
+  if (st->done) return;
+  const T *src = blockIdx.y ? b : a;
+  const int i0 = (int)((long long)blockIdx.x * n / kFoldParts), i1 = (int)((long long)(blockIdx.x + 1) * n / kFoldParts);
+  T v[1] = {T(0)};
+  for (int i = i0 + threadIdx.x; i < i1; i += kBlock) v[0] = v[0] + src[i];
+  block_partials<OpSum, 1>(v, out, blockIdx.y * kFoldParts + blockIdx.x);
+}
+
 struct CgParts {   // r.r and r.z partials of the last update / preconditioner
   int nrr, nrz;
 };
@@ -2061,13 +2079,28 @@ static Chunks chunks_of(const SellPattern *pat) {
   return Chunks{C.d_chunk_ptr.p, C.d_chunk_agg.p, C.d_chunk_pos.p, C.nchunks};
 }
 
+// the partials a (and b) for a launch of `readers` workgroups that all add them
+// up: as they are, or folded
+template <class T>
+Krylov::Parts<T> Krylov::parts_for(int readers, int m, const T *a, const T *b, const KS *st) {
+  if ((long long)m * readers * (long long)sizeof(T) * (b ? 2 : 1) <= kFoldBytes) return {m, a, b};
+  // the end of the partials' buffer: the solvers use six of its eight parts at most
+  T *out;
+  if constexpr (sizeof(T) == 8) out = part_.p + part_.n - 2 * kFoldParts;
+  else out = part32_.p + part32_.n - 2 * kFoldParts;
+  hipLaunchKernelGGL(k_fold_parts<T>, dim3(kFoldParts, b ? 2 : 1), dim3(kBlock), 0, stream(), m, a, b, out, st);
+  return {kFoldParts, out, out + kFoldParts};
+}
+
 // the preconditioner of the current r, and p
 template <class T, bool MIXED>
 void Krylov::cx_p(const Cx<T> &c, int what) {
   Chunks C = chunks_of(pat);
   if (what == kCxTest) C.n = 0;
-  hipLaunchKernelGGL((k_cx_p<T, MIXED>), dim3(what == kCxTest ? 1 : c.G), dim3(kBlock), 0, stream(), C, c.r, c.z, c.dg,
-                     c.mode, c.p, cm_.nu.p, st_.p, CgParts{c.G, c.nrz}, c.rr, c.rz, c.ncn, cnu_split_.p, what);
+  const int G = what == kCxTest ? 1 : c.G;
+  const Parts<T> rz = parts_for<T>(G, c.nrz, c.rz, nullptr, st_.p);
+  hipLaunchKernelGGL((k_cx_p<T, MIXED>), dim3(G), dim3(kBlock), 0, stream(), C, c.r, c.z, c.dg, c.mode, c.p, cm_.nu.p,
+                     st_.p, CgParts{c.G, rz.n}, c.rr, rz.a, c.ncn, cnu_split_.p, what);
 }
 
 template <class T, bool MIXED>
@@ -2096,7 +2129,8 @@ void Krylov::cx_restart(const Cx<T> &c, const T *val, const double *r64, bool di
 // the part of an iteration after the product
 template <class T, bool MIXED, class X>
 void Krylov::cx_update(const Cx<T> &c, const T *val, X *x, bool ride) {
-  hipLaunchKernelGGL((k_cx_update<T, X>), dim3(c.G), dim3(kBlock), 0, stream(), chunks_of(pat), nblk_, c.pq, c.p, c.q,
+  const Parts<T> pq = parts_for<T>(c.G, nblk_, c.pq, nullptr, st_.p);
+  hipLaunchKernelGGL((k_cx_update<T, X>), dim3(c.G), dim3(kBlock), 0, stream(), chunks_of(pat), pq.n, pq.a, c.p, c.q,
                      x, c.r, c.z, c.dg, c.mode, pat->color_ptr[1], st_.p, c.rr, c.rz, c.csum);
   cx_direction<T, MIXED>(c, val, ride ? kCxTest : kCxAll);
 }
@@ -2126,11 +2160,11 @@ void Krylov::cg2_iteration(const Cg2<T> &c, const T *val, const T *fac, X *x, hi
   const Mat A = matof(pat);
   const dim3 G(c.G), B(kBlock);
   hipStream_t S = stream();
+  const Parts<T> rz = parts_for<T>(c.G, c.nrz, c.rz, nullptr, st_.p);
+  const CgParts np{c.G, rz.n};
   auto ps = [&](auto k) {
-    if (e0) hipExtLaunchKernelGGL(k, G, B, 0, S, e0, e1, 0, n, A, val, c.z, c.p0, c.p1, c.q, st_.p, CgParts{c.G, c.nrz},
-                                  c.rr, c.rz, c.pq);
-    else hipLaunchKernelGGL(k, G, B, 0, S, n, A, val, c.z, c.p0, c.p1, c.q, st_.p, CgParts{c.G, c.nrz}, c.rr, c.rz,
-                            c.pq);
+    if (e0) hipExtLaunchKernelGGL(k, G, B, 0, S, e0, e1, 0, n, A, val, c.z, c.p0, c.p1, c.q, st_.p, np, c.rr, rz.a, c.pq);
+    else hipLaunchKernelGGL(k, G, B, 0, S, n, A, val, c.z, c.p0, c.p1, c.q, st_.p, np, c.rr, rz.a, c.pq);
   };
   if (sizeof(T) == 4 && pat->has16) ps(k_cg_ps<T, MIXED, 1>);
   else ps(k_cg_ps<T, MIXED, 0>);
@@ -2335,14 +2369,16 @@ void Krylov::bi_iteration(const Bi<T> &w, PcKind pc, const T *val, bool coarse) 
   const bool c16 = c16_of<T>(pat);
   if (c16) hipLaunchKernelGGL((k_bi_spmv_dot<T, 1>), GS, B, 0, S, n, A, val, w.ph, w.r0, w.v, w.st, pt[2]);
   else hipLaunchKernelGGL((k_bi_spmv_dot<T, 0>), GS, B, 0, S, n, A, val, w.ph, w.r0, w.v, w.st, pt[2]);
-  hipLaunchKernelGGL(k_bi_s<T>, G, B, 0, S, C, n, w.r, w.v, w.s, w.sh, w.dg, mode, c0end, w.st, nblk_, pt[2], pt[3],
+  const Parts<T> vr = parts_for<T>(G0, nblk_, pt[2], nullptr, w.st);
+  hipLaunchKernelGGL(k_bi_s<T>, G, B, 0, S, C, n, w.r, w.v, w.s, w.sh, w.dg, mode, c0end, w.st, vr.n, vr.a, pt[3],
                      csum);
   finish<OpSum, 1>(G0, pt[3], FinBiS{w.st});
   apply_pc<T>(pc, val, w.fac, w.dg, w.s, w.sh, done, true);
   if (coarse) coarse_apply<T>(w.sh, w.st);
   if (c16) hipLaunchKernelGGL((k_bi_spmv_omega<T, 1>), GS, B, 0, S, n, A, val, w.sh, w.s, w.t, w.st, pt[4], pt[5]);
   else hipLaunchKernelGGL((k_bi_spmv_omega<T, 0>), GS, B, 0, S, n, A, val, w.sh, w.s, w.t, w.st, pt[4], pt[5]);
-  hipLaunchKernelGGL(k_bi_xr<T>, G, B, 0, S, C, n, w.ph, w.sh, w.s, w.t, w.r0, w.x, w.r, w.st, nblk_, pt[4], pt[5],
+  const Parts<T> tt = parts_for<T>(G0, nblk_, pt[4], pt[5], w.st);
+  hipLaunchKernelGGL(k_bi_xr<T>, G, B, 0, S, C, n, w.ph, w.sh, w.s, w.t, w.r0, w.x, w.r, w.st, tt.n, tt.a, tt.b,
                      pt[0], pt[1]);
 }
 

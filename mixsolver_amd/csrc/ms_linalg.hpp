@@ -175,6 +175,11 @@ class Krylov {
   template <class T, bool MIXED, class X> void cx_update(const Cx<T> &c, const T *val, X *x, bool ride);
   SolveResult bicg32(PcKind pc, int maxit, int window, bool coarse);
   template <class T> void coarse_apply(T *out, KS *st);
+  template <class T> struct Parts {   // one or two arrays of n partials
+    int n;
+    const T *a, *b;
+  };
+  template <class T> Parts<T> parts_for(int readers, int m, const T *a, const T *b, const KS *st);
   // BiCGSTAB: vectors, solution, preconditioner, partials and state
   template <class T> struct Bi {
     T *r, *r0, *p, *v, *s, *t, *ph, *sh, *x;

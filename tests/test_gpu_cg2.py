@@ -58,3 +58,28 @@ def test_two_launch_pcg_against_oracle(n, lags):
         r = b - np.bincount(row, val * x[ci - 1], n)
         assert ierr == 0 and res <= 1e-10
         assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(b), (prec, np.linalg.norm(r) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("kind", ["cg_ic0", "bicgstab_ilu0"])
+def test_folded_partials_against_oracle(kind):
+    """Systems whose partials are folded before the launches that add them up:
+    2.2M rows leave 8,594 a launch, above the line of PCG in FP64 and of
+    BiCGSTAB in FP64 and FP32.  Six levels of 400,000 rows, so the sweeps are
+    short."""
+    from oracle import pyoracle
+    n = 2_200_000
+    rp, ci, val, b = _system(n, (400_000, 400_001))
+    bar = 1e-10 if kind == "cg_ic0" else 1e-9
+    for k in (1, 3):
+        x, it, res, ierr = getattr(linsolver, kind)(rp, ci, val, b, np.zeros(n), 1e-30, k)
+        xr, itr, resr, ierrr = pyoracle.solve(kind, rp, ci, val, b, np.zeros(n), 1e-30, k)
+        assert (it, ierr) == (itr, ierrr), k
+        assert np.linalg.norm(x - xr) <= bar * np.linalg.norm(xr), k
+        assert abs(res - resr) <= bar * resr, (k, res, resr)
+    if kind == "cg_ic0":
+        return
+    x, _, res, ierr = linsolver.solve(rp, ci, val, b, np.zeros(n), 1e-10, 500, precision="mixed", inner_tol=0.1,
+                                      solver="bicgstab", precond="natural")
+    row = np.repeat(np.arange(n), np.diff(rp))
+    r = b - np.bincount(row, val * x[ci - 1], n)
+    assert ierr == 0 and np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(b)
