@@ -378,8 +378,9 @@ __global__ __launch_bounds__(kSegThreads) void k_sweep_seg(const SweepStep *__re
 // A wide level: a thread per row, its entries packed as above with the
 // neighbours' rows in pcol.  The row id, columns and values are independent
 // loads (through the SELL offsets they were a chain of three), and only the
-// neighbours' values follow them: a level of 48,000 rows of a prism mesh
-// takes 3.0 us instead of 3.7.
+// neighbours' values follow them.  Averages over the levels of multicolour
+// ILU(0) sweeps on prisms, four of 48,000 rows: 2.7 us, through the offsets
+// 3.7; of 480,000 rows, which memory bounds: 7.8 and 8.9.
 template <class T, int W, bool MORE, bool DIV, bool DESC>
 __global__ __launch_bounds__(kBlock) void k_sweep_wide(SweepStep d, const int *__restrict__ rows,
                                                        const int *__restrict__ pcol, const T *__restrict__ pval,
@@ -659,10 +660,12 @@ static void sweep_wide(const SweepPlan &S, const LevSeg &g, const int *rows, con
     hipLaunchKernelGGL(k, dim3(nblocks(g.step.n)), dim3(kBlock), 0, stream(), g.step, rows, S.col.p, v, d, in, out,
                        done);
   };
-  if (S.more) go(k_sweep_wide<T, kPre, true, DIV, DESC>);
-  else if (S.width == 4) go(k_sweep_wide<T, 4, false, DIV, DESC>);
-  else if (S.width == 3) go(k_sweep_wide<T, 3, false, DIV, DESC>);
-  else if (S.width == 2) go(k_sweep_wide<T, 2, false, DIV, DESC>);
+  // by the level's own width: with colour classes it goes from none below the
+  // first class to all of a row's neighbours below the last
+  if (g.step.w > kPre) go(k_sweep_wide<T, kPre, true, DIV, DESC>);
+  else if (g.step.w == 4) go(k_sweep_wide<T, 4, false, DIV, DESC>);
+  else if (g.step.w == 3) go(k_sweep_wide<T, 3, false, DIV, DESC>);
+  else if (g.step.w == 2) go(k_sweep_wide<T, 2, false, DIV, DESC>);
   else go(k_sweep_wide<T, 1, false, DIV, DESC>);
 }
 

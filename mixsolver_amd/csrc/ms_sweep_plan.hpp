@@ -40,7 +40,7 @@ struct LevSeg {
 
 struct SweepSteps {
   std::vector<SweepStep> st;
-  int width = 0;       // entries per row of every step (more: rows beyond the width fetched ahead exist)
+  int width = 0;       // entries per row of every step of a run (more: rows beyond the width fetched ahead exist)
   bool more = false;
   long long nent = 0;
 };
@@ -54,10 +54,10 @@ SweepSteps sweep_steps(const std::vector<int> &lev, std::vector<LevSeg> &segs, W
   for (int t = 0; t < lev.back(); t++) widest_row = std::max(widest_row, width_of(t));
   S.width = std::min(widest_row, kPre);
   S.more = widest_row > kPre;
-  auto add = [&](int t, int n) {
+  auto add = [&](int t, int n, int least) {
     if (n >= kSlice) S.nent = (S.nent + kSlice - 1) / kSlice * kSlice;   // whole wavefronts load aligned
-    SweepStep d{t, n, S.width, 0, S.nent, sweep_stride(n)};
-    for (int i = 0; S.more && i < n; i++) d.w = std::max(d.w, width_of(t + i));
+    SweepStep d{t, n, least, 0, S.nent, sweep_stride(n)};
+    for (int i = 0; (S.more || least < S.width) && i < n; i++) d.w = std::max(d.w, width_of(t + i));
     S.nent += (long long)d.w * d.stride;
     S.st.push_back(d);
   };
@@ -65,7 +65,7 @@ SweepSteps sweep_steps(const std::vector<int> &lev, std::vector<LevSeg> &segs, W
     g.s0 = (int)S.st.size();
     g.t0 = lev[g.l0];
     if (!g.narrow) {
-      add(g.t0, lev[g.l1] - g.t0);
+      add(g.t0, lev[g.l1] - g.t0, 1);   // a launch of its own, as wide as its own rows
       g.s1 = (int)S.st.size();
       g.step = S.st.back();
       continue;
@@ -74,7 +74,7 @@ SweepSteps sweep_steps(const std::vector<int> &lev, std::vector<LevSeg> &segs, W
     for (int l = g.l0; l < g.l1; l++) widest = std::max(widest, lev[l + 1] - lev[l]);
     g.block = std::min(kSegThreads, (widest + kSlice - 1) / kSlice * kSlice);
     for (int l = g.l0; l < g.l1; l++)
-      for (int t = lev[l]; t < lev[l + 1]; t += g.block) add(t, std::min(g.block, lev[l + 1] - t));
+      for (int t = lev[l]; t < lev[l + 1]; t += g.block) add(t, std::min(g.block, lev[l + 1] - t), S.width);
     g.s1 = (int)S.st.size();
     for (int i = 0; i < kTailSteps; i++) S.st.push_back(SweepStep{});
   }
