@@ -555,9 +555,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_xr(int n, const T *p0, const T *p
   }
 }
 
-// the residual test after the last update of a chunk, for the host to read
-// (the next k_cg_ps comes to the same answer)
-template <class T, bool MIXED>
+// the tests after the last update of a chunk, for the host to read (the next
+// k_cg_ps comes to the same answer; BiCGSTAB tests its rho at the next
+// iteration's start)
+template <class T, bool MIXED, bool PCG = true>
 __global__ __launch_bounds__(kBlock) void k_cg_peek(KS *st, int nrr, const T *rrp) {
   if (st->done || st->it == 0) return;
   T sums[2];
@@ -572,6 +573,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_peek(KS *st, int nrr, const T *rr
     st->rr = (double)sums[0];
     st->res = rn / st->bnrm;
     if (st->res <= st->tol) st->done = 1;
+  }
+  if (PCG && !st->done && fabs(st->rz2[st->par]) < kTiny) {
+    st->ierr = 2;
+    st->done = 1;
   }
 }
 
@@ -2389,7 +2394,7 @@ KS Krylov::bi_state(const Bi<T> &w) {
   T *pt[6];
   bi_parts(pat, w.part, pt);
   const int G0 = std::min((nblk_ + kBlock / kSlice - 1) / (kBlock / kSlice), kCxGrid);
-  hipLaunchKernelGGL((k_cg_peek<T, false>), dim3(1), dim3(kBlock), 0, stream(), w.st, G0, pt[0]);
+  hipLaunchKernelGGL((k_cg_peek<T, false, false>), dim3(1), dim3(kBlock), 0, stream(), w.st, G0, pt[0]);
   MS_CHECK_LAUNCH();
   const KS hs = read_state<T>(w.st);
   if (hs.done == 2) {

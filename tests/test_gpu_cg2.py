@@ -83,3 +83,22 @@ def test_folded_partials_against_oracle(kind):
     row = np.repeat(np.arange(n), np.diff(rp))
     r = b - np.bincount(row, val * x[ci - 1], n)
     assert ierr == 0 and np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n", [1000, 3000])
+@pytest.mark.parametrize("target", [1.5e-308, 3e-308, 1e-308])
+def test_breakdown_of_the_last_iteration(n, target):
+    """r.z below the smallest normal number while p.Ap is above it (1.5e-308),
+    both above (3e-308) and both below: the breakdown is reported with the
+    iteration it belongs to, also when that is the last one allowed."""
+    from oracle import pyoracle
+    i = np.arange(n)
+    rows, cols = np.concatenate([i, i[1:], i[:-1]]), np.concatenate([i, i[:-1], i[1:]])
+    vals = np.concatenate([np.ones(n), np.full(2 * n - 2, 0.45)])
+    o = np.lexsort((cols, rows))
+    rp = (np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]) + 1).astype(np.int32)
+    ci, val, b = (cols[o] + 1).astype(np.int32), vals[o], np.full(n, np.sqrt(target / n))
+    for k in (1, 2, 3):
+        _, it, _, ierr = linsolver.cg_jacobi(rp, ci, val, b, np.zeros(n), 1e-10, k)
+        _, itr, _, ierrr = pyoracle.solve("cg_jacobi", rp, ci, val, b, np.zeros(n), 1e-10, k, mpi=True)
+        assert (it, ierr) == (itr, ierrr), k
