@@ -1,9 +1,11 @@
 """Device layouts of the cell-face entries and of the reduced product's columns."""
+import dataclasses
+
 import numpy as np
 import pytest
 
 from mixsolver_amd import meshgen
-from mixsolver_amd.solver import Case
+from mixsolver_amd.solver import Case, cell_ordering
 
 pytestmark = pytest.mark.gpu
 
@@ -105,6 +107,95 @@ def test_reduced_product_columns(nx, ny, nz):
             assert st["ppe_iters_fp64"] <= 0.1 * (st["ppe_iters_fp32"] + st["ppe_iters_fp64"])
         p = cs.get("p")
         res.append((cs.get("u"), p - p.mean()))
+    (ua, pa), (ub, pb) = res
+    assert np.abs(ua - ub).max() <= 1e-6 * np.abs(ua).max()
+    assert np.abs(pa - pb).max() <= 1e-6 * np.abs(pa).max()
+
+
+def _duct(nx, ny, nz):
+    return meshgen.hex_box(np.linspace(0.0, 4.0, nx + 1), np.linspace(-1.0, 1.0, ny + 1), np.linspace(0.0, 1.0, nz + 1),
+                           zone_ids=dict(xmin=6, xmax=7, ymin=5, ymax=5, zmin=4, zmax=4))
+
+
+def _shuffled(m, cells, seed):
+    """the box with its cells numbered at random, one colour of its
+    checkerboard before the other, so that the greedy colouring finds both"""
+    nx, ny, _ = cells
+    i = np.arange(m.ncells)
+    colour = (i % nx + i // nx % ny + i // (nx * ny)) % 2
+    order = np.lexsort((np.random.default_rng(seed).random(m.ncells), colour))
+    new = np.empty(m.ncells, np.int32)
+    new[order] = i + 1
+    c1 = np.where(m.c1 > 0, new[np.maximum(m.c1, 1) - 1], 0).astype(np.int32)
+    return dataclasses.replace(m, c0=new[m.c0 - 1], c1=c1)
+
+
+def _windows(cs, k):
+    """windows of 4,096 columns that each slice of the full matrix needs (the
+    diagonal apart), from the library's own ordering"""
+    t = cs.topology()
+    rp, ci = t["row_ptr"], t["col_idx"]
+    n = len(rp) - 1
+    n2o, color, nc = cell_ordering(rp, ci, cs.get("xc"), rcm=False, colored=True, coarse=k)
+    assert nc == 2
+    o2n = np.empty(n, np.int64)
+    o2n[n2o] = np.arange(n)
+    row = o2n[np.repeat(np.arange(n), np.diff(rp))]
+    col = o2n[ci - 1]
+    off = row != col
+    s, c = row[off] // 64, col[off]
+    o = np.lexsort((c, s))
+    s, c = s[o], c[o]
+    need = np.zeros((n + 63) // 64, int)
+    for q, cols in zip(np.unique(s), np.split(c, np.nonzero(np.diff(s))[0] + 1)):
+        end = -1
+        for x in cols:
+            if x >= end:
+                need[q] += 1
+                end = x + 4096
+    return need
+
+
+@pytest.mark.parametrize("cells,shuffle", [((120, 50, 50), True), ((90, 40, 40), True), ((400, 1, 1), False),
+                                           ((301, 2, 1), False), ((150, 3, 2), False)])
+def test_reduced_product_forms(cells, shuffle):
+    """Slices that need more than the 15 windows a slice has (cells numbered at
+    random), and few-neighbour meshes whose slices are 3 to 5 slots wide.
+    Mixed against FP64 as above."""
+    m = _duct(*cells)
+    if shuffle:
+        m = _shuffled(m, cells, 5)
+    ctl = f"""rho = 1.0
+mu = 0.05
+transient = true
+dt = {2.0 / cells[0]!r}
+n_time_max = 1
+n_correct = 2
+lin_tol = 1e-10
+lin_max = 20000
+ppe_precond = jacobi
+bc = 6 velocity-inlet 1.0 0.0 0.0
+bc = 7 pressure-outlet 0.0
+bc = 5 wall
+bc = 4 symmetry
+"""
+    res = []
+    for prec in (0, 1):
+        cs = Case.from_control(m, ctl, gpu_ppe_precond=0, gpu_mom_precond=2, gpu_coarse=2, gpu_ppe_solver=2,
+                               gpu_precision=prec, gpu_inner_tol=0.1)
+        if shuffle and not prec:
+            need = _windows(cs, 2)
+            assert (need > 15).any(), need.max()
+        u = np.random.default_rng(3).uniform(-0.05, 0.05, size=(m.ncells, 3))
+        u[:, 0] += 1.0
+        cs.set_field("u", u)
+        assert cs.piso_run(1) == 0
+        assert np.all(cs.history()[:, 7] <= 1e-10)
+        st = cs.solver_stats()
+        if prec:
+            assert st["ppe_iters_fp64"] <= 0.1 * (st["ppe_iters_fp32"] + st["ppe_iters_fp64"])
+        res.append((cs.get("u"), cs.get("p")))
+        cs.close()
     (ua, pa), (ub, pb) = res
     assert np.abs(ua - ub).max() <= 1e-6 * np.abs(ua).max()
     assert np.abs(pa - pb).max() <= 1e-6 * np.abs(pa).max()

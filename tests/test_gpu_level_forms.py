@@ -62,3 +62,29 @@ def test_long_rows_among_short_ones(kind):
     c = np.arange(m + w, n)
     pairs += [(c, c - 1), (c, rng.integers(0, m, t))]
     _against_oracle(kind, n, pairs)
+
+
+def _grid(m):
+    """rows and lower neighbours of an m^3 seven-point grid, and of the (-1, -1,
+    0) diagonal, which closes triangles; every level is a plane of up to 3 m^2 /
+    4 rows, so narrow runs and levels of over 2,048 rows follow one another"""
+    i = np.arange(m ** 3)
+    x, y, z = i % m, i // m % m, i // (m * m)
+    axes = [(i[x > 0], i[x > 0] - 1), (i[y > 0], i[y > 0] - m), (i[z > 0], i[z > 0] - m * m)]
+    d = (x > 0) & (y > 0)
+    return axes, (i[d], i[d] - 1 - m)
+
+
+@pytest.mark.parametrize("kind", ["cg_ic0", "bicgstab_ilu0"])
+def test_general_factor_of_wide_and_narrow_levels(kind):
+    """A pattern with triangles takes the general elimination: a launch per
+    wide level, one workgroup per run of narrow ones, in turn."""
+    axes, diagonal = _grid(64)
+    _against_oracle(kind, 64 ** 3, axes + [diagonal])
+
+
+@pytest.mark.parametrize("where", ["lower", "upper"])
+def test_general_factor_of_an_asymmetric_pattern(where):
+    """Entries without a transpose (ILU(0) only), with their triangles."""
+    axes, (i, j) = _grid(64)
+    _against_oracle("bicgstab_ilu0", 64 ** 3, axes, [(i, j) if where == "lower" else (j, i)])
