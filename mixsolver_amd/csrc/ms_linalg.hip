@@ -1659,7 +1659,9 @@ Krylov::HostState Krylov::borrow_host_state() {
 }
 void Krylov::give_back_host_state(const HostState &h) {
   if (!h.pin) return;
-  // nothing of this solver may still write the page
+  // nothing of this solver may still write the page; waiting on a stream that
+  // another thread (a server's) is capturing would end that capture
+  const auto lk = library_stream_lock();
   const bool ok = hipStreamSynchronize(stream()) == hipSuccess;
   if (ok) {
     std::lock_guard<std::mutex> g(g_host_mu);
@@ -1668,7 +1670,7 @@ void Krylov::give_back_host_state(const HostState &h) {
       return;
     }
   }
-  std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
+  std::lock_guard<std::recursive_mutex> alk(device_alloc_mutex());
   for (const auto &e : h.ev)
     if (e) (void)hipEventDestroy(e);
   (void)hipHostFree(h.pin);

@@ -90,3 +90,35 @@ def test_threads_read_their_own_fields():
         t.join()
     assert not bad, bad
     cs.close()
+
+
+def test_systems_end_beside_a_server():
+    """Systems are destroyed while a server's worker runs and captures its
+    rounds on the library stream: every request is solved, and as alone."""
+    from mixsolver_amd.serve import LaplacianPattern, Server, request_mesh
+    P = LaplacianPattern(request_mesh(5000, "hex", seed=1))
+    rng = np.random.default_rng(8)
+    reqs = [(P.values(rng), P.rhs(rng)) for _ in range(3)]
+    systems = [_case(gpu_ppe_precond=2) for _ in range(12)]
+    srv = Server(precond="dilu", coarse=0, round_iters=4)
+    pid = srv.add_pattern(P.row_ptr, P.col_idx, P.xc)
+    alone = [srv.result(srv.submit(pid, v, b, tol=1e-10, maxit=5000), timeout_ms=-1)["x"] for v, b in reqs]
+    stop, bad, solved = threading.Event(), [], [0]
+
+    def serve():
+        while not stop.is_set():
+            tickets = [srv.submit(pid, v, b, tol=1e-10, maxit=5000) for v, b in reqs]
+            for t, x in zip(tickets, alone):
+                r = srv.result(t, timeout_ms=-1)
+                if r["ierr"] != 0 or not np.array_equal(r["x"], x):
+                    bad.append(r["ierr"])
+                solved[0] += 1
+    th = threading.Thread(target=serve)
+    th.start()
+    for cs in systems:
+        time.sleep(5e-3)
+        cs.close()
+    stop.set()
+    th.join()
+    srv.close()
+    assert not bad and solved[0] >= 3
