@@ -609,12 +609,22 @@ int ms_time_kernel(ms_system *h, int which, int reps, double *avg_ms, double *al
     // algorithmic bytes of one SpMV: nnz (value + column index) + one int per row + x and y
     if (alg_bytes) *alg_bytes = (double)P.nnz * (sz + idx) + 4.0 * (P.n + 1) + 2.0 * P.n * sz;
     if (alg_bytes && red && fp32 && K.matfree_on()) {
-      // the matrix-free product: A's nonzeros (FP32 weight + 16-bit column)
-      // and one int per row of A, x read by each stage, the colour-0
-      // intermediate (h, x_ref) written and read, q written
+      // the matrix-free product: A's nonzeros (FP32 weight + column, 16 bits
+      // in the slices that have windows and an unrolled body, else 32) and one
+      // int per row of A, x read by each stage, the colour-0 intermediate
+      // (h, x_ref) written and read, q written
       const SellPattern &F = *s.P;
       const double n0 = s.schur->n0, n1 = s.schur->n1;
-      *alg_bytes = (double)F.nnz * 4.0 + 2.0 * F.nnz + 4.0 * (F.n + 1) +
+      std::vector<int> win(s.schur->mf_win.n);
+      s.schur->mf_win.download(win.data(), win.size());
+      MS_HIP(hipStreamSynchronize(stream()));
+      double cols = 0.0;
+      for (int q = 0; q < F.nslices; q++) {
+        const long long w = (F.off[q + 1] - F.off[q]) / kSlice;
+        const bool c16 = win[16 * (size_t)q + 15] != 0 && w >= 5 && w <= 7;
+        for (int r = q * kSlice; r < std::min(F.n, (q + 1) * kSlice); r++) cols += (c16 ? 2.0 : 4.0) * F.rowlen[r];
+      }
+      *alg_bytes = (double)F.nnz * 4.0 + cols + 4.0 * (F.n + 1) +
                    2.0 * n1 * 4.0 +
                    2.0 * n0 * 8.0 + n1 * 4.0;
     }

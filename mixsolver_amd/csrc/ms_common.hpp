@@ -151,8 +151,6 @@ struct DBuf {
     n = 0;
     own = true;
   }
-  // bytes this buffer owns (0 for a view)
-  size_t owned_bytes() const { return own ? n * sizeof(T) : 0; }
   void upload(const T *h, size_t count) {
     if (count > n) alloc(count);
     if (count) MS_HIP(hipMemcpyAsync(p, h, count * sizeof(T), hipMemcpyHostToDevice, stream()));
@@ -178,8 +176,8 @@ inline int nblocks(long long n, int b = kBlock) { return (int)((n + b - 1) / b);
 // Z the aggregate indicator matrix and E = Z^T A Z.  The device numbering
 // keeps every aggregate contiguous inside each colour, so the rows are cut
 // into chunks of at most kBlock rows that each lie in one aggregate; the
-// cell-wise PCG kernels run one workgroup per chunk, which turns Z^T r into
-// per-workgroup partial sums and Z nu into a broadcast.
+// cell-wise PCG kernels give a wavefront (k_cx_*) or a workgroup (the others) a
+// chunk, which turns Z^T r into one sum per chunk and Z nu into a broadcast.
 constexpr int kMaxAgg = 1024;
 constexpr int kInvRegMax = 256;   // largest E of the one-workgroup register inverter (request server)
 struct Coarse {

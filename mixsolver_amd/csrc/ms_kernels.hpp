@@ -244,25 +244,11 @@ struct FinPap {
 };
 struct FinUpdate {
   KS *st;
-  int jac;
   __device__ bool skip() const { return st->done != 0; }
   template <class T> __device__ void operator()(const T *a) const {
     st->rr = a[0];
     st->res = sqrt((double)a[0]) / st->bnrm;
-    if (st->res <= st->tol) {
-      st->done = 1;
-      return;
-    }
-    if (jac) {
-      if (fabs(st->rz) < kTiny) {
-        st->ierr = 2;
-        st->done = 1;
-      } else {
-        const double rzn = rz_total(st, (double)a[1]);
-        st->beta = rzn / st->rz;
-        st->rz = rzn;
-      }
-    }
+    if (st->res <= st->tol) st->done = 1;
   }
 };
 struct FinRz {
@@ -407,11 +393,6 @@ __global__ void k_dilu_setup(int r0, int r1, Mat A, const long long *tpos, const
 }
 
 // ------------------------------------------------------------ coarse space
-// Finisher of the update reduction with the coarse solve (one workgroup):
-// the scalar sums as k_finish, then c_a = sum of the last partial over the
-// chunks of aggregate a (fixed order), nu = E^-1 c and c.nu, before the
-// functor runs on thread 0.
-
 // Coarse solve riding along a DILU forward-sweep launch: nwg extra
 // workgroups of kBlock threads, each recomputing c = Z^T r from the chunk
 // sums and four rows of nu = E^-1 c;
@@ -552,6 +533,10 @@ __device__ void coarse_solve(const T *partial, const CoDev &co) {
   if (threadIdx.x == 0) co.st->cnu = prod[0];
 }
 
+// Finisher of the update reduction with the coarse solve (one workgroup):
+// the scalar sums as k_finish, then c_a = sum of the last partial over the
+// chunks of aggregate a (fixed order), nu = E^-1 c and c.nu, before the
+// functor runs on thread 0.
 template <int NV, class T, class Fin>
 __global__ __launch_bounds__(kFinThreads) void k_finish_co(int nparts, const T *partial, Fin fin, CoDev co) {
   if (fin.skip()) return;

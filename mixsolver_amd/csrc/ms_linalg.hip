@@ -303,8 +303,8 @@ __global__ void k_pcg_p(Rows R, const T *r, const T *z, const T *dg, int jac, T 
 // partials.  The grid is capped so that the partials every workgroup reads
 // stay few; a workgroup takes a contiguous range of row blocks.
 // Kernel time per iteration, five launches before, two now: 13.4 -> 7.4 us at
-// 1,728 rows in FP64, 15.5 -> 7.3 at 16,384, 21 -> 13.2 at 216,000; 20.5 ->
-// 16.3 at 432,000 rows in FP32.
+// 1,728 rows in FP64 (a size that k_cg_small takes since), 15.5 -> 7.3 at
+// 16,384, 21 -> 13.2 at 216,000; 20.5 -> 16.3 at 432,000 rows in FP32.
 // The parity of the iteration comes from the device's own count: st->it
 // changes in k_cg_xr only, st->par in k_cg_ps only.
 constexpr int kCgGrid = 2048;
@@ -2315,7 +2315,7 @@ SolveResult Krylov::pcg(const double *val, const double *b, double *x, double to
       finish<OpSum, 1>(nblk_, part, FinPap{st});
       hipLaunchKernelGGL((k_pcg_update<double, double>), GR, B, 0, S, RW, p_.p, q_.p, x, r_.p, z_.p, dg_.p, 0, 0, st,
                          part);
-      finish_co<3>((int)GR.x, part, FinUpdate{st, 0}, co);
+      finish_co<3>((int)GR.x, part, FinUpdate{st}, co);
       apply_pc<double>(pc, val, fac_.p, dg_.p, r_.p, z_.p, done);
       hipLaunchKernelGGL(k_dot<double>, G, B, 0, S, n, r_.p, z_.p, st, part);
       finish<OpSum, 1>(nblk_, part, FinRz{st});
@@ -2549,9 +2549,9 @@ bool schur_matfree_enabled() {
 }
 void set_schur_matfree(bool on) { g_schur_mf.store(on ? 1 : 0); }
 // E^-1 of a coarse space of at most 256 aggregates by one workgroup in FP32
-// (MIXSOLVER_COARSE_INV32=1) instead of k launches in FP64; off by default:
-// the one workgroup takes longer than the k launches over the grid (17.17
-// against 17.64 PISO steps/s at 2M cells, 256 aggregates)
+// (MIXSOLVER_COARSE_INV32=1) instead of k / 32 launches over the chip in FP64
+// (k_gj_block); off by default: the one workgroup takes longer (21.99 against
+// 22.90 PISO steps/s at 2M cells, 256 aggregates)
 static bool coarse_inv32_enabled() {
   static const bool on = [] {
     const char *e = std::getenv("MIXSOLVER_COARSE_INV32");

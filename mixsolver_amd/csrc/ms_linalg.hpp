@@ -5,7 +5,7 @@
 namespace ms {
 
 struct KS {              // device-resident solver scalars (one per solve)
-  double bnrm, rz, pap, alpha, beta, res, rho, rho_old, omega, snrm, tt, rr;
+  double bnrm, rz, pap, alpha, beta, res, rho, omega, snrm, tt, rr;
   double rmax, delta;    // reliable updates: largest sloppy |r| since the last update, trigger ratio
   double sigma, scale;   // FP32 iteration runs on r/sigma; scale = sigma_old/sigma_new at an update
   double cnu;            // coarse part of r.z: (Z^T r) . E^-1 (Z^T r)
