@@ -304,7 +304,10 @@ __global__ void k_pcg_p(Rows R, const T *r, const T *z, const T *dg, int jac, T 
 // stay few; a workgroup takes a contiguous range of row blocks.
 // Kernel time per iteration, five launches before, two now: 13.4 -> 7.4 us at
 // 1,728 rows in FP64 (a size that k_cg_small takes since), 15.5 -> 7.3 at
-// 16,384, 21 -> 13.2 at 216,000; 20.5 -> 16.3 at 432,000 rows in FP32.
+// 16,384, 21 -> 13.2 at 216,000; 20.5 -> 16.3 at 432,000 rows in FP32.  Every
+// size takes this form: whole PISO steps with FP64 DILU-PCG p' solves, before
+// and now, 92 -> 84 ms at 480,000 cells, 199 -> 179 at 1M, 353 -> 338 at 2M
+// and 2541 -> 2449 at 8.2M (k_fold_parts from 1M on).
 // The parity of the iteration comes from the device's own count: st->it
 // changes in k_cg_xr only, st->par in k_cg_ps only.
 constexpr int kCgGrid = 2048;
