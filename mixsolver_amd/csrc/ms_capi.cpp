@@ -159,7 +159,10 @@ int ms_system_destroy(ms_system *s) {
   return guarded([&] {
     if (!s) return;
     if (s->s && s->s->nforks.load() > 0) fail(MS_EINVAL, "the system still has sweep cases (destroy the sweep first)");
-    MS_HIP(hipStreamSynchronize(stream()));
+    {
+      const auto lk = library_stream_lock();   // a server may be capturing on it
+      MS_HIP(hipStreamSynchronize(stream()));
+    }
     delete s;
   });
 }
@@ -258,7 +261,6 @@ int ms_set_field(ms_system *h, const char *name, const double *host, long long n
             break;
           }
     }
-    MS_HIP(hipStreamSynchronize(stream()));
   });
 }
 

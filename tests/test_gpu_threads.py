@@ -106,13 +106,16 @@ def test_systems_end_beside_a_server():
     stop, bad, solved = threading.Event(), [], [0]
 
     def serve():
-        while not stop.is_set():
-            tickets = [srv.submit(pid, v, b, tol=1e-10, maxit=5000) for v, b in reqs]
-            for t, x in zip(tickets, alone):
-                r = srv.result(t, timeout_ms=-1)
-                if r["ierr"] != 0 or not np.array_equal(r["x"], x):
-                    bad.append(r["ierr"])
-                solved[0] += 1
+        try:
+            while not stop.is_set():
+                tickets = [srv.submit(pid, v, b, tol=1e-10, maxit=5000) for v, b in reqs]
+                for t, x in zip(tickets, alone):
+                    r = srv.result(t, timeout_ms=-1)
+                    if r["ierr"] != 0 or not np.array_equal(r["x"], x):
+                        bad.append(r["ierr"])
+                    solved[0] += 1
+        except BaseException as e:   # noqa: B902 -- reported by the main thread
+            bad.append(e)
     th = threading.Thread(target=serve)
     th.start()
     for cs in systems:
@@ -121,4 +124,4 @@ def test_systems_end_beside_a_server():
     stop.set()
     th.join()
     srv.close()
-    assert not bad and solved[0] >= 3
+    assert not bad and solved[0] >= 3, bad
