@@ -65,8 +65,8 @@ std::mutex g_stage_mu;
 std::vector<std::pair<int, double *>> g_idle_stages;   // (device, buffer)
 class Stage {
  public:
-  Stage() {
-    MS_HIP(hipGetDevice(&dev_));
+  Stage() : dev_(runtime_device()) {
+    MS_HIP(hipSetDevice(dev_));   // a reader's thread may not have chosen the library's device
     {
       std::lock_guard<std::mutex> g(g_stage_mu);
       for (size_t i = 0; i < g_idle_stages.size(); i++)
@@ -98,7 +98,7 @@ class Stage {
   double *p = nullptr;
 
  private:
-  int dev_ = 0;
+  int dev_;
 };
 
 // the caller's n values in pieces of the staging buffer's size; false: no
@@ -140,6 +140,7 @@ const T *map_on_device(System &s, DBuf<T> &d, Host host) {
   if (!d.n) {
     const std::vector<T> &h = host();
     const auto lk = library_stream_lock();
+    MS_HIP(hipSetDevice(runtime_device()));
     DBuf<T> t;
     try {
       t.alloc(h.size());
